@@ -474,7 +474,7 @@ std::string validate(const hx_host_mesh* d, const Sizes& z)
 // The face-flux folding tables (Dev_mesh::partner, mortar_con) of a validated mesh. Every element face in a connection
 // that touches no hanging-face mortar gets its neighbour slot, the packed direction with its side, the connection class
 // and a boundary bit, and (deformed connections) the connection's normal slot; every other face (mortar neighbours,
-// coarse hanging faces) is marked precomputed. Connections touching a mortar are listed per class.
+// coarse hanging faces) is marked precomputed. Every entry ends with the face's own slot. Connections touching a mortar are listed per class.
 // ref_con[4 * i + f]: the connection (class << 30 | index) of mortar f of refined face i, -1 where the face has none.
 // Returns whether the mortars of every refined face are exactly the fine faces its stretch leaves (Restrict_refined's)
 // and each is in a connection, which k_mortar_restrict requires.
@@ -487,6 +487,7 @@ bool build_partners(const hx_host_mesh* d, const Sizes& z, std::vector<int> (&pa
     partner[c].assign(size_t(d->n_elem[c]) * nf * 4, 0);
     for (long long k = 0; k < (long long)d->n_elem[c] * nf; ++k) {
       partner[c][4 * k] = -1;
+      partner[c][4 * k + 3] = d->face_slot[c][k];
       owner[d->face_slot[c][k]] = c | int(k << 1);
     }
   }

@@ -52,10 +52,10 @@ struct Dev_mesh
   hx_bc* bcs;
   double* bc_cache;  // [n_bc_con][nv][nfq] boundary-face state cache
   // Face-flux folding (the update path): each element computes its faces' numerical fluxes itself from its own and its
-  // neighbour's extrapolated states. partner[cls][e * 2nd + face] = {neighbour slot, info, connection normal slot, 0}
-  // with info = packed direction | side << 6 | connection class << 7 | boundary << 8, or neighbour slot -1 where the
-  // flux is computed before the Local (faces of hanging-face mortars, coarse hanging faces). The connections that
-  // touch a mortar are listed per class in mortar_con. The state blocks of the faces are double-buffered: block 0 of a
+  // neighbour's extrapolated states. partner[cls][e * 2nd + face] = {neighbour slot, info, connection normal slot,
+  // own slot} with info = packed direction | side << 6 | connection class << 7 | boundary << 8, or neighbour slot -1
+  // where the flux is computed before the Local (faces of hanging-face mortars, coarse hanging faces). The connections
+  // that touch a mortar are listed per class in mortar_con. The state blocks of the faces are double-buffered: block 0 of a
   // slot is read from faces (alt_rd 0) or faces_alt [n_slot][nv][nfq] (alt_rd 1) and written to the one alt_wr names;
   // the LDG blocks stay in faces. alt_rd = alt_wr = 0 everywhere else.
   int* partner[2];

@@ -164,12 +164,14 @@ void k_fused_local_euler(const Fused_member* __restrict__ mem, const Fused_plan*
   extern __shared__ double fused_lds_all[];
   float* mtab = reinterpret_cast<float*>(fused_lds_all);
   double* fused_lds = fused_lds_all + fused_table_doubles<P, RSS...>();
-  for_tiles<PERSIST>(plan->n_tiles, order, chunk, [&](int tile) {
+  // (the bodies are inlined by force: as functions of their own they would reach the LDS through flat addresses and keep
+  // their arguments in scratch memory)
+  for_tiles<PERSIST>(plan->n_tiles, order, chunk, [&](int tile) __attribute__((always_inline)) {
     const int s = fused_segment(plan, tile);
     const Fused_member& mb = mem[plan->member[s]];
     const int blk = tile - plan->first[s];
     const bool def = plan->cls[s] == HX_DEFORMED;
-    dispatch_rs<RSS...>(plan->rs[s], [&](auto rs_c) {
+    dispatch_rs<RSS...>(plan->rs[s], [&](auto rs_c) __attribute__((always_inline)) {
       constexpr int RS = decltype(rs_c)::value;
       using T = typename P::T;
       const Eops<RS, double>& o = eops_of<RS>(ops);

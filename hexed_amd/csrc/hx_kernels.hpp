@@ -566,86 +566,119 @@ __global__ __launch_bounds__(256) void k_neighbor_mortar(Dev_mesh m)
   if (i < m.n_mortar_con[cls]) neighbor_con<ND, RS, DEF, VISC>(m, m.mortar_con[cls][i], f);
 }
 
-// Face-flux folding: the numerical flux of face point p of face `face` of element e (class cls), times this side's
-// sign, computed from the two extrapolated states exactly as Neighbor computes it for the connection (Spatial.hpp:
-// 613-704, the operands in the connection's side order), and with VISC the LDG average of the two states. A face whose
-// flux a launch before the Local computed (hanging faces) reads flux and average from its own slot. On a boundary
-// connection the element also writes the ghost side's flux into the ghost slot's block 0 in the primary buffer, where
-// Neighbor leaves it.
-template <int ND, int RS, bool VISC>
-__device__ inline void face_flux(const Dev_mesh& m, int cls, int e, int face, int p, double (&fl)[ND + 2],
-                                 double (&avg)[ND + 2])
+// Face-flux folding, in three steps so that a kernel can have every load of one step in flight before it waits for the
+// first: the face's entry of the partner table, the operands it points at, and the flux.
+struct Face_ref
+{
+  int ps, info, cn, own;  // Dev_mesh::partner: neighbour slot, info, connection normal slot, own slot
+};
+__device__ __forceinline__ Face_ref face_ref(const Dev_mesh& m, int cls, size_t k)
+{
+  const int4 p = reinterpret_cast<const int4*>(m.partner[cls])[k];
+  return {p.x, p.y, p.z, p.w};
+}
+
+// The operands of the numerical flux at face point p: both extrapolated states in the connection's side order and the
+// connection normal. Branch-free (a branch makes the compiler wait for the loads before it): a face whose flux is
+// precomputed reads its own slot twice, and a Cartesian connection's normal is loaded from the own state's address and
+// not used -- except on Cartesian elements (DEF false), where deformed connections are the rare boundary faces.
+template <int ND, int RS>
+struct Face_in
+{
+  double u0[ND + 2], u1[ND + 2], n[ND];
+};
+template <int ND, int RS, bool DEF>
+__device__ __forceinline__ void face_in(const Dev_mesh& m, const Face_ref& r, int p, Face_in<ND, RS>& in)
 {
   constexpr int NFQ = Shape<ND, RS>::NFQ, NV = ND + 2;
-  const size_t k = size_t(e) * 2 * ND + face;
-  const int* pi = m.partner[cls] + 4 * k;
-  const int own_slot = m.face_slot[cls][k];
-  const double* own = state_ptr(m, own_slot, m.alt_rd);
-  const int ps = pi[0];
-  if (ps < 0) {
-    for (int v = 0; v < NV; ++v) fl[v] = own[v * NFQ + p];
-    if constexpr (VISC) {
-      const double* l = slot_ptr(m, own_slot) + NV * NFQ;
-      for (int v = 0; v < NV; ++v) avg[v] = l[v * NFQ + p];
-    }
-    return;
-  }
-  const int info = pi[1];
+  const bool pre = r.ps < 0;
+  const int info = pre ? 0 : r.info;
   const Dir dir(info & 63);
-  const bool side1 = (info >> 6) & 1, def = (info >> 7) & 1, bc = (info >> 8) & 1;
-  const double* par = state_ptr(m, ps, m.alt_rd);
-  int f0 = p, f1 = p;
-  double sg0 = 1., sg1 = 1.;
-  double n[ND];
-  if (def) {
-    if (side1) f0 = face0_index<ND, RS>(dir, p);
-    else f1 = face1_index<ND, RS>(dir, p);
-    sg0 = 1 - 2 * int(dir.flip_normal(0));
-    sg1 = 1 - 2 * int(dir.flip_normal(1));
-    const double* nn = m.normals + size_t(pi[2]) * ND * NFQ;
-    for (int j = 0; j < ND; ++j) n[j] = sg0 * nn[j * NFQ + f0];
-  } else {
-    for (int j = 0; j < ND; ++j) n[j] = (j == dir.i_dim0);
-  }
+  const bool side1 = (info >> 6) & 1, def = (info >> 7) & 1;
+  const double* own = state_ptr(m, r.own, m.alt_rd);
+  const double* par = state_ptr(m, pre ? r.own : r.ps, m.alt_rd);
+  int fp = side1 ? face0_index<ND, RS>(dir, p) : face1_index<ND, RS>(dir, p);
+  fp = def ? fp : p;
+  const int f0 = side1 ? fp : p, f1 = side1 ? p : fp;
   const double* a0 = side1 ? par : own;
   const double* a1 = side1 ? own : par;
-  double u0[NV], u1[NV];
   for (int v = 0; v < NV; ++v) {
-    u0[v] = a0[v * NFQ + f0];
-    u1[v] = a1[v * NFQ + f1];
+    in.u0[v] = a0[v * NFQ + f0];
+    in.u1[v] = a1[v * NFQ + f1];
   }
+  if constexpr (DEF) {
+    const double* nn = def ? m.normals + size_t(r.cn) * ND * NFQ : own;
+    for (int j = 0; j < ND; ++j) in.n[j] = nn[j * NFQ + f0];
+  } else {
+    for (int j = 0; j < ND; ++j) in.n[j] = 0.;
+    if (def) {
+      const double* nn = m.normals + size_t(r.cn) * ND * NFQ;
+      for (int j = 0; j < ND; ++j) in.n[j] = nn[j * NFQ + f0];
+    }
+  }
+}
+
+// The numerical flux times this side's sign, exactly as Neighbor computes it for the connection (Spatial.hpp:613-704),
+// and with VISC the LDG average of the two states. A face whose flux a launch before the Local computed (hanging faces)
+// takes flux and average from its own slot. On a boundary connection the element also writes the ghost side's flux into
+// the ghost slot's block 0 in the primary buffer, where Neighbor leaves it (`write`: not for a thread past the last
+// element).
+template <int ND, int RS, bool VISC>
+__device__ __forceinline__ void face_flux(const Dev_mesh& m, const Face_ref& r, int p, bool write, const Face_in<ND, RS>& in,
+                                          double (&fl)[ND + 2], double (&avg)[ND + 2])
+{
+  constexpr int NFQ = Shape<ND, RS>::NFQ, NV = ND + 2;
+  const bool pre = r.ps < 0;
+  const int info = pre ? 0 : r.info;
+  const Dir dir(info & 63);
+  const bool side1 = (info >> 6) & 1, def = (info >> 7) & 1, bc = (info >> 8) & 1;
+  const double sg0 = def ? 1 - 2 * int(dir.flip_normal(0)) : 1, sg1 = def ? 1 - 2 * int(dir.flip_normal(1)) : 1;
+  double n[ND];
+  for (int j = 0; j < ND; ++j) n[j] = def ? sg0 * in.n[j] : double(j == dir.i_dim0);
   if constexpr (VISC)
-    for (int v = 0; v < NV; ++v) avg[v] = .5 * (u0[v] + u1[v]);
+    for (int v = 0; v < NV; ++v) avg[v] = .5 * (in.u0[v] + in.u1[v]);
   double F0[NV], F1[NV];
-  flux_conv<ND>(u0, n, F0);
-  flux_conv<ND>(u1, n, F1);
+  flux_conv<ND>(in.u0, n, F0);
+  flux_conv<ND>(in.u1, n, F1);
   double nsq = 0;
   for (int j = 0; j < ND; ++j) nsq += n[j] * n[j];
-  const double c = fmax(char_speed<ND>(u0), char_speed<ND>(u1)) * sqrt(nsq);
-  double* ghost = (bc && !side1) ? slot_ptr(m, ps) : nullptr;
-  for (int v = 0; v < NV; ++v) {
-    const double x = .5 * (F0[v] + F1[v] + c * (u0[v] - u1[v]));
-    fl[v] = (side1 ? sg1 : sg0) * x;
-    if (ghost) ghost[v * NFQ + f1] = sg1 * x;
+  const double c = fmax(char_speed<ND>(in.u0), char_speed<ND>(in.u1)) * sqrt(nsq);
+  for (int v = 0; v < NV; ++v) fl[v] = .5 * (F0[v] + F1[v] + c * (in.u0[v] - in.u1[v]));
+  if (bc && !side1 && write) {
+    double* ghost = slot_ptr(m, r.ps);
+    const int f1 = def ? face1_index<ND, RS>(dir, p) : p;
+    for (int v = 0; v < NV; ++v) ghost[v * NFQ + f1] = sg1 * fl[v];
   }
+  for (int v = 0; v < NV; ++v) fl[v] = pre ? in.u0[v] : (side1 ? sg1 : sg0) * fl[v];
+  if constexpr (VISC)
+    if (pre) {
+      const double* l = slot_ptr(m, r.own) + NV * NFQ;
+      for (int v = 0; v < NV; ++v) avg[v] = l[v * NFQ + p];
+    }
 }
 
 // The faces' numerical fluxes of the workgroup's elements into dst[EPB][2ND][NV][NFQ] (element stride `per`), one thread
 // per face point (face-flux folding, in place of load_faces)
-template <int ND, int RS, int NT>
+template <int ND, int RS, bool DEF, int NT>
 __device__ inline void fold_fluxes(const Dev_mesh& m, int cls, int blk, double* dst, int per)
 {
   using S = Shape<ND, RS>;
   constexpr int NFP = 2 * ND * S::NFQ, NV = S::NV, NFQ = S::NFQ;
   const int n = m.n_elem[cls];
-  for (int k = threadIdx.x; k < S::EPB * NFP; k += NT) {
+#pragma unroll
+  for (int k0 = 0; k0 < S::EPB * NFP; k0 += NT) {
+    // (threads past the last face point repeat the first one instead of branching)
+    const bool own = k0 + int(threadIdx.x) < S::EPB * NFP;
+    const int k = own ? k0 + int(threadIdx.x) : 0;
     const int el = k / NFP, r = k % NFP, face = r / NFQ, p = r % NFQ;
     const int e = blk * S::EPB + el;
     double fl[NV], avg[NV];
-    if (e < n) face_flux<ND, RS, false>(m, cls, e, face, p, fl, avg);
-    else
-      for (int v = 0; v < NV; ++v) fl[v] = 0.;
-    for (int v = 0; v < NV; ++v) dst[el * per + (face * NV + v) * NFQ + p] = fl[v];
+    const Face_ref fr = face_ref(m, cls, size_t(e < n ? e : n - 1) * 2 * ND + face);
+    Face_in<ND, RS> in;
+    face_in<ND, RS, DEF>(m, fr, p, in);
+    face_flux<ND, RS, false>(m, fr, p, own && e < n, in, fl, avg);
+    if (own)
+      for (int v = 0; v < NV; ++v) dst[el * per + (face * NV + v) * NFQ + p] = fl[v];
   }
 }
 
@@ -799,14 +832,15 @@ constexpr int euler_block()
 // Waves per SIMD that the workgroup's LDS allows (160 KB per CU, 4 SIMDs), at most 5: the register target given to
 // the compiler, so that registers do not lower the occupancy below what LDS permits. With face-flux folding, where a
 // thread computes more than one face point's flux, at most 4 (the registers of two face points' states and fluxes
-// would spill at 5).
+// would spill at 5), and so for the FP32-MFMA form at row size 8.
 template <int ND, int RS, bool DEF, class P, bool FOLD = false>
 constexpr int euler_waves()
 {
   using L = Euler_lds<ND, RS, DEF, P>;
   constexpr int lds = Shape<ND, RS>::EPB * (int(sizeof(typename P::T)) * L::PER_T + 8 * L::PER_D);
   constexpr int w = (163840 / lds) * (euler_block<ND, RS>() / 64) / 4;
-  constexpr int cap = FOLD && Shape<ND, RS>::EPB * 2 * ND * Shape<ND, RS>::NFQ > euler_block<ND, RS>() ? 4 : 5;
+  constexpr bool two = FOLD && Shape<ND, RS>::EPB * 2 * ND * Shape<ND, RS>::NFQ > euler_block<ND, RS>();
+  constexpr int cap = two || (P::mfma && RS == 8) ? 4 : 5;
   return w < 1 ? 1 : (w > cap ? cap : w);
 }
 
@@ -876,7 +910,7 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
   // are not held in registers across the row phases
   const double* mt = m.metrics + (DEF ? size_t(e) * (ND * ND + 1) * NQ + q : 0);
   const double p64 = P::mfma ? pressure_of<ND>(u) : 0.;
-  if constexpr (FOLD) fold_fluxes<ND, RS, NT>(m, cls, blk, ld + L::SB, L::PER_D);
+  if constexpr (FOLD) fold_fluxes<ND, RS, DEF, NT>(m, cls, blk, ld + L::SB, L::PER_D);
   else load_faces<ND, RS, NT>(m, cls, blk, 0, ld + L::SB, L::PER_D);
   for (int i = 0; i < ND; ++i) {
     if (i == ND - 1) {
@@ -1008,11 +1042,20 @@ struct Ns_lds
   static constexpr int SL = 0;                                    // [2ND][NV][NFQ] LDG face state
   static constexpr int SFN = SL + 2 * ND * NV * NFQ;              // [2ND][ND][NFQ] face normals
   static constexpr int P1_D = SFN + (DEF ? 2 * ND * ND * NFQ : 0);
-  static constexpr int SB = 0;                                    // [2ND][NV][NFQ] numerical face fluxes
-  static constexpr int PD = SB + 2 * ND * NV * NFQ;               // [ND][NQP] FP32-MFMA, deformed: pressure part p n_iv
-  static constexpr int RP = PD + ND * NQP;                        // [ND][NQP] FP32-MFMA, deformed: its derivative, summed
-  static constexpr int P2_D = PD + (P::mfma && DEF ? 2 * ND * NQP : 0);
-  static constexpr int PER_D = P1_D > P2_D ? P1_D : P2_D;
+  // numerical face fluxes SB [2ND][NV][NFQ]; FP32-MFMA, deformed: pressure part PD = p n_iv and its derivative RP summed
+  // over the directions, [ND][NQP] each. SB takes the gradient phase's place (the fluxes stay in registers until then),
+  // or, in the FP32-MFMA form where its LDS costs no workgroup per compute unit, a place of its own from the start
+  // (SB_EARLY), which frees the registers: 15 -> 0 spilled per lane, 2.62 -> 2.36 ms per launch on the 48^3 deformed mesh.
+  static constexpr int SB_N = 2 * ND * NV * NFQ, PR_N = P::mfma && DEF ? 2 * ND * NQP : 0;
+  static constexpr int LATE_D = P1_D > SB_N + PR_N ? P1_D : SB_N + PR_N;
+  static constexpr int EARLY_D = (P1_D > PR_N ? P1_D : PR_N) + SB_N;
+  static constexpr int EXTRA = P::mfma ? 16 * Eops<RS, double>::MF_STRIDE + 8 * 2 * ND : 0;  // (with the other arrays)
+  static constexpr int lds_with(int per_d) { return S::EPB * (int(sizeof(typename P::T)) * PER_T + 8 * per_d) + EXTRA; }
+  static constexpr bool SB_EARLY = P::mfma && 163840 / lds_with(EARLY_D) == 163840 / lds_with(LATE_D);
+  static constexpr int SB = SB_EARLY ? EARLY_D - SB_N : 0;
+  static constexpr int PD = SB_EARLY ? 0 : SB_N;
+  static constexpr int RP = PD + ND * NQP;
+  static constexpr int PER_D = SB_EARLY ? EARLY_D : LATE_D;
 };
 
 // waves per SIMD that the Navier-Stokes Local's LDS allows, at most 4 (3 for row sizes above 6, which spill at 4):
@@ -1042,106 +1085,120 @@ void k_local_ns(Dev_mesh m, Eops<RS, double> o,
   __shared__ double ld[EPB * L::PER_D];
   // FP32-MFMA form: the matrix-core operands, read from LDS at each contraction (Contraction_lds)
   __shared__ __align__(16) float mtab[P::mfma ? 4 * Eops<RS, double>::MF_STRIDE : 4];
-  // FP64 form, where the LDS keeps the workgroups per compute unit: the elements' face slots, read with the first
-  // loads so that the viscous flux extrapolations below need no global read ahead of their writes (3.13 -> 3.09 ms on
-  // the 48^3 deformed mesh; the FP32-MFMA form, whose registers are full, lost 1% with it)
+  // where the LDS keeps the workgroups per compute unit, the elements' face slots, so that the viscous flux
+  // extrapolations below need no global read ahead of their writes
   constexpr int LDS_B = EPB * (int(sizeof(T)) * L::PER_T + 8 * L::PER_D), SLOTS_B = 4 * EPB * 2 * ND;
-  constexpr bool STAGE = !P::mfma && 163840 / (LDS_B + SLOTS_B) == 163840 / LDS_B;
+  constexpr bool STAGE = 163840 / (LDS_B + SLOTS_B) == 163840 / LDS_B;
   __shared__ int fsl[STAGE ? EPB * 2 * ND : 1];
   const int t = threadIdx.x;
   const int blk = blockIdx.x;
-  if (STAGE && t < EPB * 2 * ND) {
-    const int e2 = blk * EPB + t / (2 * ND);
-    fsl[t] = e2 < m.n_elem[cls] ? m.face_slot[cls][e2 * 2 * ND + t % (2 * ND)] : 0;
-  }
   const bool pt = t < EPB * NQ;
   const int el = pt ? t / NQ : 0, q = pt ? t % NQ : 0, qp = S::pad(q);
   const int n = m.n_elem[cls];
   const int e = blk * EPB + el;
   const bool valid = pt && e < n;
   T* my = lt + el * L::PER_T;
-  if constexpr (P::mfma) lds_mfma_operands<RS, NT>(od, mtab);
   const auto con = [&] {
     if constexpr (P::mfma) return Contraction_lds<RS>(mtab);
     else return Contraction<RS, P, true>(o, od);
   }();
 
-  // the numerical face fluxes are needed only after the gradient; their loads are issued now and held in
-  // registers so that their latency hides behind the gradient phase
-  constexpr int PF = 2 * ND * NV * NFQ, NSB = FOLD ? 1 : (EPB * PF + NT - 1) / NT;
-  double sb[NSB];
-  if constexpr (!FOLD) {
+  // The element's loads, in two steps: what its index alone locates (face table, point data), then what the face table
+  // points at. Threads past the last element or point read the last one's data instead of branching, and use nothing of
+  // it. (With a branch per operand the loads were waited for one after the other, about eleven memory latencies, a third
+  // of the time an element stayed on its compute unit: FP64 3.10 -> 2.49 ms, FP32-MFMA 2.79 -> 2.36 ms per launch on the 48^3
+  // deformed mesh.)
+  constexpr int NFP = 2 * ND * NFQ, FPT = (EPB * NFP + NT - 1) / NT;
+  const auto face_item = [&](int k, int& el2, int& e2, int& face, int& p) {
+    const int kk = t + k * NT < EPB * NFP ? t + k * NT : 0, r = kk % NFP;
+    el2 = kk / NFP;
+    e2 = blk * EPB + el2;
+    face = r / NFQ;
+    p = r % NFQ;
+  };
+  const int ec = e < n ? e : n - 1;
+  Face_ref fr[FPT];
+  int fns[FPT];
 #pragma unroll
-    for (int k = 0; k < NSB; ++k) {
-      const int kk = t + k * NT, el2 = kk / PF, r = kk % PF, f = r / (NV * NFQ), vq = r % (NV * NFQ);
-      const int e2 = blk * EPB + el2;
-      sb[k] = (kk < EPB * PF && e2 < n) ? state_ptr(m, m.face_slot[cls][e2 * 2 * ND + f], m.alt_rd)[vq] : 0.;
-    }
+  for (int k = 0; k < FPT; ++k) {
+    int el2, e2, face, p;
+    face_item(k, el2, e2, face, p);
+    const size_t kf = size_t(e2 < n ? e2 : n - 1) * 2 * ND + face;
+    fr[k] = face_ref(m, cls, kf);
+    if constexpr (DEF) fns[k] = m.face_nslot[kf];
   }
-  // folded: one thread per face point computes its flux (held in registers until the convective pass, whose LDS it
-  // shares with the gradient phase) and its LDG average (into LDS now)
-  constexpr int NFP = 2 * ND * NFQ, FPT = FOLD ? (EPB * NFP + NT - 1) / NT : 1;
-  double sbf[FPT][NV];
-  if constexpr (FOLD) {
-#pragma unroll
-    for (int k = 0; k < FPT; ++k) {
-      const int kk = t + k * NT, el2 = kk / NFP, r = kk % NFP, face = r / NFQ, p = r % NFQ;
-      const int e2 = blk * EPB + el2;
-      double avg[NV];
-      if (kk < EPB * NFP && e2 < n) {
-        face_flux<ND, RS, true>(m, cls, e2, face, p, sbf[k], avg);
-      } else {
-        for (int v = 0; v < NV; ++v) sbf[k][v] = avg[v] = 0.;
-      }
-      if (kk < EPB * NFP)
-        for (int v = 0; v < NV; ++v) ld[el2 * L::PER_D + L::SL + (face * NV + v) * NFQ + p] = avg[v];
-    }
-  }
-
+  if constexpr (P::mfma) lds_mfma_operands<RS, NT>(od, mtab);
+  __builtin_amdgcn_sched_barrier(0);
+  // the numerical face fluxes (folded: computed here from both sides' states, and held in registers until the convective
+  // pass where the gradient phase has their LDS) and the LDG averages
   double u[NV];
-  const double* st = m.state[cls] + size_t(e) * NV * NQ;
-  for (int v = 0; v < NV; ++v) {
-    u[v] = valid ? st[v * NQ + q] : (v >= ND ? 1. : 0.);
-    if (!P::mfma && pt) my[L::U + v * NQP + qp] = T(u[v]);
-  }
-  T bulk = 0, lap = 0;
-  if (valid && m.av[cls]) {
-    bulk = T(m.av[cls][size_t(e) * 2 * NQ + q]);
-    lap = T(m.av[cls][size_t(e) * 2 * NQ + NQ + q]);
-  }
-  double det = 1.;
   double metd[DEF ? ND : 1][DEF ? ND : 1];
-  if constexpr (DEF) {
-    const double* mt = m.metrics + size_t(e) * (ND * ND + 1) * NQ;
-    for (int i = 0; i < ND; ++i)
-      for (int j = 0; j < ND; ++j) {
-        metd[i][j] = valid ? mt[(i * ND + j) * NQ + q] : double(i == j);
-        if (!P::mfma && pt && j == 0) my[L::SN + i * NQP + qp] = T(metd[i][j]);
+  const double* st = m.state[cls] + size_t(ec) * NV * NQ;
+  const double* mt = m.metrics + (DEF ? size_t(ec) * (ND * ND + 1) * NQ : 0);
+  double sbf[FPT][NV];
+#pragma unroll
+  for (int k = 0; k < FPT; ++k) {
+    int el2, e2, face, p;
+    face_item(k, el2, e2, face, p);
+    const bool own = t + k * NT < EPB * NFP;
+    double nf[DEF ? ND : 1], avg[NV];
+    Face_in<ND, RS> in;
+    if constexpr (FOLD) {
+      face_in<ND, RS, DEF>(m, fr[k], p, in);
+    } else {
+      const double* fs = state_ptr(m, fr[k].own, m.alt_rd);
+      const double* fl = slot_ptr(m, fr[k].own) + NV * NFQ;
+      for (int v = 0; v < NV; ++v) {
+        sbf[k][v] = fs[v * NFQ + p];
+        avg[v] = fl[v * NFQ + p];
       }
-    det = valid ? mt[ND * ND * NQ + q] : 1.;
+    }
+    if constexpr (DEF) {
+      // a face in a Cartesian connection uses the identity normal (Spatial.hpp:331-339,364-367)
+      const double* np = fns[k] >= 0 ? m.normals + size_t(fns[k]) * ND * NFQ : state_ptr(m, fr[k].own, m.alt_rd);
+      for (int j = 0; j < ND; ++j) nf[j] = np[j * NFQ + p];
+    }
+    if (k == FPT - 1) {
+      // the point data arrive while the last flux is formed
+      for (int v = 0; v < NV; ++v) u[v] = st[v * NQ + q];
+      if constexpr (DEF)
+        for (int i = 0; i < ND; ++i) metd[i][0] = mt[i * ND * NQ + q];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (FOLD) face_flux<ND, RS, true>(m, fr[k], p, own && e2 < n, in, sbf[k], avg);
+    if (own) {
+      for (int v = 0; v < NV; ++v) ld[el2 * L::PER_D + L::SL + (face * NV + v) * NFQ + p] = avg[v];
+      if constexpr (DEF)
+        for (int j = 0; j < ND; ++j)
+          ld[el2 * L::PER_D + L::SFN + (face * ND + j) * NFQ + p] = fns[k] >= 0 ? nf[j] : double(j == face / 2);
+      if constexpr (L::SB_EARLY)
+        for (int v = 0; v < NV; ++v) ld[el2 * L::PER_D + L::SB + (face * NV + v) * NFQ + p] = sbf[k][v];
+      if (STAGE && p == 0) fsl[el2 * 2 * ND + face] = fr[k].own;
+    }
   }
+  // (needed after the first gradient component)
+  if constexpr (DEF)
+    for (int i = 0; i < ND; ++i)
+      for (int j = 1; j < ND; ++j) metd[i][j] = mt[(i * ND + j) * NQ + q];
+  const double* avp = m.av[cls] ? m.av[cls] + size_t(ec) * 2 * NQ : st;
+  const double bulk_d = avp[q], lap_d = avp[NQ + q];
+  const double nom = m.nom_size[cls][ec];
+  const double det = DEF ? mt[ND * ND * NQ + q] : 1.;
+  const T bulk = m.av[cls] ? T(bulk_d) : T(0), lap = m.av[cls] ? T(lap_d) : T(0);
+  if constexpr (!P::mfma)
+    if (pt) {
+      for (int v = 0; v < NV; ++v) my[L::U + v * NQP + qp] = T(u[v]);
+      if constexpr (DEF)
+        for (int i = 0; i < ND; ++i) my[L::SN + i * NQP + qp] = T(metd[i][0]);
+    }
   auto metric = [&](int i, int j) -> double {
     if constexpr (DEF) return metd[i][j];
     else return double(i == j);
   };
-  if constexpr (!FOLD) load_faces<ND, RS, NT>(m, cls, blk, 1, ld + L::SL, L::PER_D);
-  if constexpr (DEF) {
-    for (int k = t; k < EPB * 2 * ND * ND * NFQ; k += NT) {
-      const int el2 = k / (2 * ND * ND * NFQ), r = k % (2 * ND * ND * NFQ), f = r / (ND * NFQ), jq = r % (ND * NFQ);
-      const int e2 = blk * EPB + el2;
-      double val = 0.;
-      if (e2 < n) {
-        const int ns_ = m.face_nslot[e2 * 2 * ND + f];
-        // a face in a Cartesian connection uses the identity normal (Spatial.hpp:331-339,364-367)
-        val = ns_ >= 0 ? m.normals[size_t(ns_) * ND * NFQ + jq] : double(jq / NFQ == f / 2);
-      }
-      ld[el2 * L::PER_D + L::SFN + r] = val;
-    }
-  }
   __syncthreads();
   // gradient times Jacobian determinant, divided by the nominal size (Spatial.hpp:371-402), one physical
   // component j at a time
-  const double inv_h = valid ? 1. / m.nom_size[cls][e] : 1.;
+  const double inv_h = 1. / nom;
   T grad[NV][ND];
   if constexpr (!P::mfma) {
     for (int j = 0; j < ND; ++j) {
@@ -1229,20 +1286,14 @@ void k_local_ns(Dev_mesh m, Eops<RS, double> o,
     for (int v = 0; v < NV; ++v) ut[v] = T(u[v]);
     flux_visc<ND>(ns, ut, bulk, lap, grad, fvis);
   }
-  if constexpr (FOLD) {
+  if constexpr (!L::SB_EARLY) {
 #pragma unroll
     for (int k = 0; k < FPT; ++k) {
-      const int kk = t + k * NT, el2 = kk / NFP, r = kk % NFP, face = r / NFQ, p = r % NFQ;
-      if (kk < EPB * NFP)
+      int el2, e2, face, p;
+      face_item(k, el2, e2, face, p);
+      if (t + k * NT < EPB * NFP)
         for (int v = 0; v < NV; ++v) ld[el2 * L::PER_D + L::SB + (face * NV + v) * NFQ + p] = sbf[k][v];
     }
-  } else {
-#pragma unroll
-    for (int k = 0; k < NSB; ++k)
-      if (t + k * NT < EPB * PF) {
-        const int kk = t + k * NT;
-        ld[(kk / PF) * L::PER_D + L::SB + kk % PF] = sb[k];
-      }
   }
   // residual along each direction (Spatial.hpp:444-470). The viscous flux goes first (it is also extrapolated to the
   // LDG blocks of the faces), then the convective flux with its numerical face fluxes. The two rates accumulate in
