@@ -448,10 +448,10 @@ __device__ inline void load_faces(const Dev_mesh& m, int cls, int blk, int ldg, 
 }
 
 // Write_face of the FP64 padded [NVAR][NQP] arrays at `buf` (element stride `per`) into block 0 of every face
-// (Spatial.hpp:29-71)
-template <int ND, int RS, int NT, int NVAR = Shape<ND, RS>::NV>
-__device__ inline void write_faces_from(const Dev_mesh& m, int cls, int blk, const Eops<RS, double>& o, const double* buf,
-                                        int per)
+// (Spatial.hpp:29-71); slots(el2) points at the 2 ND face slots of element el2 of the workgroup
+template <int ND, int RS, int NT, int NVAR, class F>
+__device__ inline void write_faces_to(const Dev_mesh& m, int cls, int blk, const Eops<RS, double>& o, const double* buf,
+                                      int per, F&& slots)
 {
   using S = Shape<ND, RS>;
   const int n = m.n_elem[cls];
@@ -461,11 +461,18 @@ __device__ inline void write_faces_from(const Dev_mesh& m, int cls, int blk, con
       if (e >= n) return;
       double x[RS];
       load_row(buf + el * per + v * S::NQP + base, sd, x);
-      const int* fs = m.face_slot[cls] + e * 2 * ND + 2 * i;
+      const int* fs = slots(el) + 2 * i;
       state_ptr(m, fs[0], m.alt_wr)[v * S::NFQ + r] = row_bound(o, 0, x);
       state_ptr(m, fs[1], m.alt_wr)[v * S::NFQ + r] = row_bound(o, 1, x);
     });
   }
+}
+template <int ND, int RS, int NT, int NVAR = Shape<ND, RS>::NV>
+__device__ inline void write_faces_from(const Dev_mesh& m, int cls, int blk, const Eops<RS, double>& o, const double* buf,
+                                        int per)
+{
+  write_faces_to<ND, RS, NT, NVAR>(m, cls, blk, o, buf, per,
+                                   [&](int el) { return m.face_slot[cls] + (blk * Shape<ND, RS>::EPB + el) * 2 * ND; });
 }
 
 // ---- Neighbor (Spatial.hpp:613-704) ----------------------------------------------------------------------
@@ -657,31 +664,6 @@ __device__ __forceinline__ void face_flux(const Dev_mesh& m, const Face_ref& r, 
     }
 }
 
-// The faces' numerical fluxes of the workgroup's elements into dst[EPB][2ND][NV][NFQ] (element stride `per`), one thread
-// per face point (face-flux folding, in place of load_faces)
-template <int ND, int RS, bool DEF, int NT>
-__device__ inline void fold_fluxes(const Dev_mesh& m, int cls, int blk, double* dst, int per)
-{
-  using S = Shape<ND, RS>;
-  constexpr int NFP = 2 * ND * S::NFQ, NV = S::NV, NFQ = S::NFQ;
-  const int n = m.n_elem[cls];
-#pragma unroll
-  for (int k0 = 0; k0 < S::EPB * NFP; k0 += NT) {
-    // (threads past the last face point repeat the first one instead of branching)
-    const bool own = k0 + int(threadIdx.x) < S::EPB * NFP;
-    const int k = own ? k0 + int(threadIdx.x) : 0;
-    const int el = k / NFP, r = k % NFP, face = r / NFQ, p = r % NFQ;
-    const int e = blk * S::EPB + el;
-    double fl[NV], avg[NV];
-    const Face_ref fr = face_ref(m, cls, size_t(e < n ? e : n - 1) * 2 * ND + face);
-    Face_in<ND, RS> in;
-    face_in<ND, RS, DEF>(m, fr, p, in);
-    face_flux<ND, RS, false>(m, fr, p, own && e < n, in, fl, avg);
-    if (own)
-      for (int v = 0; v < NV; ++v) dst[el * per + (face * NV + v) * NFQ + p] = fl[v];
-  }
-}
-
 // ---- convective flux rows of the two forms ---------------------------------------------------------------------
 // FP64: the flux row x of direction i enters -(D x + L (b - B x)) as is.
 // FP32-MFMA: the FP32 operands carry only what FP32 holds accurately relative to the small residual of a nearly
@@ -770,33 +752,40 @@ __device__ inline void pressure_row(G&& ops, int i, int v, const double* prow, d
   }
 }
 
-// 1/time step at one quadrature point (Spatial.hpp:790-818): the convective scale over the interpolated vertex spacing,
-// plus the diffusive one for Navier-Stokes
+// 1/time step at one quadrature point (Spatial.hpp:790-818): the convective scale over the vertex spacing vs interpolated
+// to the point (coordinates x), plus the diffusive one for Navier-Stokes
+template <int ND, bool VISC>
+__device__ __forceinline__ double max_dt_scale_at(const Ns_params& ns, const double (&u)[ND + 2], double (&vs)[1 << ND],
+                                                  const double (&x)[ND], double bulk, double lap, double max_cfl_c,
+                                                  double max_cfl_d)
+{
+  // math::interp (math.hpp:207-218)
+  int stride = 1 << ND;
+#pragma unroll
+  for (int d = 0; d < ND; ++d) {
+    stride /= 2;
+#pragma unroll
+    for (int i = 0; i < stride; ++i) vs[i] += x[d] * (vs[i + stride] - vs[i]);
+  }
+  const double spacing = vs[0];
+  double scale = char_speed<ND>(u) / max_cfl_c / spacing;
+  if constexpr (VISC) scale += diffusivity<ND>(ns, u, bulk, lap) / max_cfl_d / spacing / spacing;
+  return scale;
+}
 template <int ND, int RS, bool VISC>
 __device__ inline double max_dt_scale_u(const Dev_mesh& m, const Ops<RS>* __restrict__ gops, const Ns_params& ns, int cls,
                                         size_t e, int q, const double (&u)[ND + 2], double max_cfl_c, double max_cfl_d)
 {
   constexpr int NQ = Shape<ND, RS>::NQ, NVERT = 1 << ND;
-  double vs[NVERT];
+  double vs[NVERT], x[ND];
   for (int i = 0; i < NVERT; ++i) vs[i] = m.vertex_tss[cls][e * NVERT + i];
-  // math::interp (math.hpp:207-218)
-  int stride = NVERT;
-  for (int d = 0; d < ND; ++d) {
-    stride /= 2;
-    const double x = gops->node[(q / ipow(RS, ND - 1 - d)) % RS];
-    for (int i = 0; i < stride; ++i) vs[i] += x * (vs[i + stride] - vs[i]);
+  for (int d = 0; d < ND; ++d) x[d] = gops->node[(q / ipow(RS, ND - 1 - d)) % RS];
+  double bulk = 0., lap = 0.;
+  if (VISC && m.av[cls]) {
+    bulk = m.av[cls][e * 2 * NQ + q];
+    lap = m.av[cls][e * 2 * NQ + NQ + q];
   }
-  const double spacing = vs[0];
-  double scale = char_speed<ND>(u) / max_cfl_c / spacing;
-  if constexpr (VISC) {
-    double bulk = 0., lap = 0.;
-    if (m.av[cls]) {
-      bulk = m.av[cls][e * 2 * NQ + q];
-      lap = m.av[cls][e * 2 * NQ + NQ + q];
-    }
-    scale += diffusivity<ND>(ns, u, bulk, lap) / max_cfl_d / spacing / spacing;
-  }
-  return scale;
+  return max_dt_scale_at<ND, VISC>(ns, u, vs, x, bulk, lap, max_cfl_c, max_cfl_d);
 }
 
 // The stage coefficient: `coef` itself, or with a device-resident time step (dtp not null) coef times that time step,
@@ -813,12 +802,19 @@ struct Euler_lds
   static constexpr int RT = F + S::NV * S::NQP;             // [NV][NQP] time rate
   static constexpr int PER_T = RT + S::NV * S::NQP;
   // arrays of double
-  static constexpr int SB = 0;                              // [2ND][NV][NFQ] numerical face fluxes
+  static constexpr int SB = 0;                              // [2ND][NV][NFQ] numerical face fluxes, the last face first
   static constexpr int PD = SB + 2 * ND * S::NV * S::NFQ;   // [ND][NQP] FP32-MFMA, deformed: pressure part p n_iv
   static constexpr int RP = PD + ND * S::NQP;               // [ND][NQP] FP32-MFMA, deformed: its derivative, summed
   static constexpr int LOOP_D = PD + (P::mfma && DEF ? 2 * ND * S::NQP : 0);
-  static constexpr int U = 0;                               // [NV][NQP] updated state, for Write_face (after the loop)
-  static constexpr int PER_D = LOOP_D > S::NV * S::NQP ? LOOP_D : S::NV * S::NQP;
+  static constexpr int U = 0;                                // [NV][NQP] updated state, for Write_face (after the loop)
+  // what the end of the tile reads of the element's tables: vertex time step scale [2^ND], face slots [2ND] (int), node
+  // coordinates [RS] (element 0). Written during the last direction's row phase, when every other direction's fluxes
+  // are done with; the last direction's come first in SB and so lie below it (at least two of the RS + 1 rows of NFQ
+  // points of U). It starts past U, which is written while slower waves still read it.
+  static constexpr int TB = S::NV * S::NQP;
+  static constexpr int TB_SLOT = TB + S::NVERT, TB_NODE = TB_SLOT + ND, TB_END = TB_NODE + RS;
+  static constexpr int PER_D = LOOP_D > TB_END ? LOOP_D : TB_END;
+  static constexpr __device__ int sb(int face) { return SB + (2 * ND - 1 - face) * S::NV * S::NFQ; }
 };
 
 // The Euler Local's workgroup: whole wavefronts in both forms (the fused time-step reduction shuffles across full
@@ -832,7 +828,7 @@ constexpr int euler_block()
 // Waves per SIMD that the workgroup's LDS allows (160 KB per CU, 4 SIMDs), at most 5: the register target given to
 // the compiler, so that registers do not lower the occupancy below what LDS permits. With face-flux folding, where a
 // thread computes more than one face point's flux, at most 4 (the registers of two face points' states and fluxes
-// would spill at 5), and so for the FP32-MFMA form at row size 8.
+// would spill at 5), and so for the FP32-MFMA form at row sizes 7 and 8.
 template <int ND, int RS, bool DEF, class P, bool FOLD = false>
 constexpr int euler_waves()
 {
@@ -840,7 +836,7 @@ constexpr int euler_waves()
   constexpr int lds = Shape<ND, RS>::EPB * (int(sizeof(typename P::T)) * L::PER_T + 8 * L::PER_D);
   constexpr int w = (163840 / lds) * (euler_block<ND, RS>() / 64) / 4;
   constexpr bool two = FOLD && Shape<ND, RS>::EPB * 2 * ND * Shape<ND, RS>::NFQ > euler_block<ND, RS>();
-  constexpr int cap = two || (P::mfma && RS == 8) ? 4 : 5;
+  constexpr int cap = two || (P::mfma && RS >= 7) ? 4 : 5;
   return w < 1 ? 1 : (w > cap ? cap : w);
 }
 
@@ -868,7 +864,9 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
   using L = Euler_lds<ND, RS, DEF, P>;
   using T = typename P::T;
   constexpr int NQ = S::NQ, NQP = S::NQP, NFQ = S::NFQ, NV = S::NV, EPB = S::EPB, NT = euler_block<ND, RS>();
+  constexpr int NVERT = S::NVERT;
   constexpr int cls = DEF ? HX_DEFORMED : HX_CARTESIAN;
+  constexpr bool EARLY_RC = true;
   const int t = threadIdx.x;
   const bool pt = t < EPB * NQ;
   const int el = pt ? t / NQ : 0, q = pt ? t % NQ : 0, qp = S::pad(q);
@@ -876,57 +874,104 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
   const int e = blk * EPB + el;
   const bool valid = pt && e < n;
   T* my = lt + el * L::PER_T;
-  // (the first contraction follows a barrier)
-  if constexpr (P::mfma) lds_mfma_operands<RS, NT>(od, mtab);
+  double* myd = ld + el * L::PER_D;
   const auto con = [&] {
     if constexpr (P::mfma) return Contraction_lds<RS>(mtab);
     else return Contraction<RS, P>(o, od);
   }();
 
+  // The loads go out in two steps, as in k_local_ns: the face table, then what it points at together with the point
+  // data. Threads past the last element or point read the last one's data instead of branching.
+  constexpr int NFP = 2 * ND * NFQ, FPT = (EPB * NFP + NT - 1) / NT;
+  const auto face_item = [&](int k, int& el2, int& e2, int& face, int& p) {
+    const int kk = t + k * NT < EPB * NFP ? t + k * NT : 0, r = kk % NFP;
+    el2 = kk / NFP;
+    e2 = blk * EPB + el2;
+    face = r / NFQ;
+    p = r % NFQ;
+  };
+  const int ec = e < n ? e : n - 1;
+  Face_ref fr[FPT];
+#pragma unroll
+  for (int k = 0; k < FPT; ++k) {
+    int el2, e2, face, p;
+    face_item(k, el2, e2, face, p);
+    fr[k] = face_ref(m, cls, size_t(e2 < n ? e2 : n - 1) * 2 * ND + face);
+  }
+  // (the first contraction follows a barrier)
+  if constexpr (P::mfma) lds_mfma_operands<RS, NT>(od, mtab);
+  __builtin_amdgcn_sched_barrier(0);
   double u[NV];
-  const double* st = m.state[cls] + size_t(e) * NV * NQ;
-  for (int v = 0; v < NV; ++v) u[v] = valid ? st[v * NQ + q] : (v >= ND ? 1. : 0.);
-  // what the stage update at the end reads from memory -- the residual cache (stage 1), the nominal size, the time
-  // step scale and (deformed) the Jacobian determinant. Folded kernels up to row size 6 load the last two at the start
-  // of the last direction, so that their latency overlaps that direction's phases; on Cartesian elements the first two
-  // as well (Euler Local 0.82 -> 0.78 ms per step on the 32^3 box, 0.48 -> 0.45 on the 16^3 tree). On deformed
-  // elements those are read at the update: earlier, they cost more registers than their latency saves (1.78 -> 1.84 ms
-  // on the 48^3 deformed mesh).
-  constexpr bool EARLY = !DEF && FOLD && RS <= 6;
-  double rcv[NV];
-  double tss_q = 0., nom = 1., det_q = 1.;
-  const auto load_update_operands = [&] {
-    const double* rc = m.rcache[cls] + size_t(e) * S::NRC * NQ;
-    for (int v = 0; v < NV; ++v) rcv[v] = (valid && stage) ? rc[v * NQ + q] : 0.;
-    if (valid) nom = m.nom_size[cls][e];
-  };
-  const auto load_scale = [&] {
-    if (valid) {
-      tss_q = m.tss[cls][size_t(e) * NQ + q];
-      if constexpr (DEF) det_q = m.metrics[size_t(e) * (ND * ND + 1) * NQ + ND * ND * NQ + q];
+  const double* st = m.state[cls] + size_t(ec) * NV * NQ;
+  // deformed: each direction's reference-level normals are loaded ahead of the row phase before it, so that only one
+  // direction's are held at a time
+  const double* mt = m.metrics + (DEF ? size_t(ec) * (ND * ND + 1) * NQ + q : 0);
+  double nrm[ND];
+#pragma unroll
+  for (int k = 0; k < FPT; ++k) {
+    int el2, e2, face, p;
+    face_item(k, el2, e2, face, p);
+    const bool own = t + k * NT < EPB * NFP;
+    double fl[NV], avg[NV];
+    Face_in<ND, RS> in;
+    if constexpr (FOLD) {
+      face_in<ND, RS, DEF>(m, fr[k], p, in);
+    } else {
+      const double* fs = state_ptr(m, fr[k].own, m.alt_rd);
+      for (int v = 0; v < NV; ++v) fl[v] = fs[v * NFQ + p];
     }
-  };
-  // deformed: each direction's reference-level normals are loaded in that direction's point phase, so that they
-  // are not held in registers across the row phases
-  const double* mt = m.metrics + (DEF ? size_t(e) * (ND * ND + 1) * NQ + q : 0);
+    if (k == FPT - 1) {
+      for (int v = 0; v < NV; ++v) u[v] = st[v * NQ + q];
+      if constexpr (DEF)
+        for (int j = 0; j < ND; ++j) nrm[j] = mt[j * NQ];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (FOLD) face_flux<ND, RS, false>(m, fr[k], p, own && e2 < n, in, fl, avg);
+    if (own)
+      for (int v = 0; v < NV; ++v) ld[el2 * L::PER_D + L::sb(face) + v * NFQ + p] = fl[v];
+  }
   const double p64 = P::mfma ? pressure_of<ND>(u) : 0.;
-  if constexpr (FOLD) fold_fluxes<ND, RS, DEF, NT>(m, cls, blk, ld + L::SB, L::PER_D);
-  else load_faces<ND, RS, NT>(m, cls, blk, 0, ld + L::SB, L::PER_D);
+  const bool fused_dt = (fuse.block_min || fuse.point_scale[cls]) && !compute_residual;
+  // what the end of the tile reads from memory: the residual cache (stage 1), the nominal size, the time step scale, the
+  // Jacobian determinant, and for the fused time step the viscosity coefficients; and the element's tables (L::TB),
+  // each thread fetching one entry of each. All are requested before the last direction's row phase.
+  double rcv[NV];
+  // (bulk and lap start as some loaded value: with a constant, the compiler moves their first use up to the load)
+  double tss_q = 0., nom = 1., det_q = 1., bulk = u[0], lap = u[0], vert = 0., node = 0.;
+  int slot = 0;
+  const auto load_update_operands = [&] {
+    if (stage) {
+      const double* rc = m.rcache[cls] + size_t(ec) * S::NRC * NQ;
+      for (int v = 0; v < NV; ++v) rcv[v] = rc[v * NQ + q];
+    } else {
+      for (int v = 0; v < NV; ++v) rcv[v] = 0.;
+    }
+  };
   for (int i = 0; i < ND; ++i) {
-    if (i == ND - 1) {
-      if constexpr (EARLY) load_update_operands();
-      if constexpr (FOLD && RS <= 6) load_scale();
-    }
     // volume flux along reference direction i (Spatial.hpp:404-419), in FP64
-    double nrm[ND];
-    for (int j = 0; j < ND; ++j) {
-      if constexpr (DEF) nrm[j] = valid ? mt[(i * ND + j) * NQ] : double(i == j);
-      else nrm[j] = double(i == j);
-    }
+    if constexpr (!DEF)
+      for (int j = 0; j < ND; ++j) nrm[j] = double(i == j);
     if (i || P::mfma) __syncthreads();
     if (pt)
-      conv_point<ND, DEF, P>(u, p64, nrm, ld + el * L::PER_D + L::SB + (2 * i) * NV * NFQ + Row<ND, RS>::fq(q, i), NFQ,
-                             my + L::F + qp, ld + el * L::PER_D + L::PD + qp, NQP);
+      conv_point<ND, DEF, P>(u, p64, nrm, myd + L::sb(2 * i) + Row<ND, RS>::fq(q, i), NFQ, my + L::F + qp, myd + L::PD + qp,
+                             NQP);
+    if constexpr (DEF)
+      if (i + 1 < ND)
+        for (int j = 0; j < ND; ++j) nrm[j] = mt[((i + 1) * ND + j) * NQ];
+    if (i == ND - 1) {
+      if constexpr (EARLY_RC) load_update_operands();
+      tss_q = m.tss[cls][size_t(ec) * NQ + q];
+      if constexpr (DEF) det_q = mt[ND * ND * NQ];
+      nom = m.nom_size[cls][ec];
+      if (fused_dt && fuse.visc && m.av[cls]) {
+        bulk = m.av[cls][size_t(ec) * 2 * NQ + q];
+        lap = m.av[cls][size_t(ec) * 2 * NQ + NQ + q];
+      }
+      const int ev = blk * EPB + t / NVERT, es = blk * EPB + t / (2 * ND);
+      vert = m.vertex_tss[cls][size_t(ev < n ? ev : n - 1) * NVERT + t % NVERT];
+      slot = m.face_slot[cls][size_t(es < n ? es : n - 1) * 2 * ND + t % (2 * ND)];
+      node = gops->node[t % RS];
+    }
     __syncthreads();
     // -derivative(row_f, face_f) (Spatial.hpp:444-457)
     for_columns<ND, RS, NV, NT, P::mfma>(i, [&](bool ok, int el2, int v, int r, int base, int sd) {
@@ -934,13 +979,16 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
       double* db = ld + el2 * L::PER_D;
       T y[RS];
       conv_row<ND, RS, DEF, P>(con, [&]() -> const Eops<RS, double>& { return o; }, v, b + L::F + v * NQP + base, db + L::PD + (v % ND) * NQP + base, sd,
-                               db[L::SB + ((2 * i) * NV + v) * NFQ + r], db[L::SB + ((2 * i + 1) * NV + v) * NFQ + r], y);
+                               db[L::sb(2 * i) + v * NFQ + r], db[L::sb(2 * i + 1) + v * NFQ + r], y);
       if (ok) {
         sub_row(b + L::RT + v * NQP + base, sd, y, i == 0);
         pressure_row<ND, RS, DEF, P>([&]() -> const Eops<RS, double>& { return o; }, i, v, db + L::PD + (v % ND) * NQP + base, db + L::RP + (v % ND) * NQP + base, sd);
       }
     });
   }
+  if (t < EPB * NVERT) ld[(t / NVERT) * L::PER_D + L::TB + t % NVERT] = vert;
+  if (t < EPB * 2 * ND) reinterpret_cast<int*>(ld + (t / (2 * ND)) * L::PER_D + L::TB_SLOT)[t % (2 * ND)] = slot;
+  if (t < RS) ld[L::TB_NODE + t] = node;
   if (use_filter) {
     filter_columns<ND, RS, NV, NT>(o, lt + L::RT, L::PER_T);
     if constexpr (P::mfma && DEF) filter_columns<ND, RS, ND, NT>(o, ld + L::RP, L::PER_D);
@@ -948,8 +996,7 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
     __syncthreads();
   }
   // stage update (Spatial.hpp:483-503)
-  if constexpr (!EARLY) load_update_operands();
-  if constexpr (!(FOLD && RS <= 6)) load_scale();
+  if constexpr (!EARLY_RC) load_update_operands();
   if (valid) {
     double mult = step_coef(coef, dtp) * tss_q / nom;
     if constexpr (DEF) mult /= det_q;
@@ -957,7 +1004,7 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
     double* sw = m.state[cls] + size_t(e) * NV * NQ;
     for (int v = 0; v < NV; ++v) {
       double r = double(my[L::RT + v * NQP + qp]);
-      if (has_pressure<ND, DEF>(v) && P::mfma) r -= ld[el * L::PER_D + L::RP + v * NQP + qp];
+      if (has_pressure<ND, DEF>(v) && P::mfma) r -= myd[L::RP + v * NQP + qp];
       if (stage) r -= rcv[v];
       else rcw[v * NQ + q] = r;
       r *= mult;
@@ -968,11 +1015,15 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
       for (int v = 0; v < NV; ++v) sw[v * NQ + q] = u[v];
   }
   // the next time step's Max_dt (Spatial.hpp:790-818, global time step) on the state just written: each point's
-  // 1/scale here (its loads then overlap the face writes below), the workgroup minimum after them
+  // 1/scale here, the workgroup minimum after the face writes below
   double c = DBL_MAX;
-  if ((fuse.block_min || fuse.point_scale[cls]) && valid && !compute_residual) {
-    const double scale = fuse.visc ? max_dt_scale_u<ND, RS, true>(m, gops, fuse.ns, cls, e, q, u, fuse.max_cfl_c, fuse.max_cfl_d)
-                                   : max_dt_scale_u<ND, RS, false>(m, gops, fuse.ns, cls, e, q, u, fuse.max_cfl_c, fuse.max_cfl_d);
+  if (fused_dt && valid) {
+    double vs[NVERT], x[ND];
+    for (int i = 0; i < NVERT; ++i) vs[i] = myd[L::TB + i];
+    for (int d = 0; d < ND; ++d) x[d] = ld[L::TB_NODE + Row<ND, RS>::node(q, d)];
+    const bool av = m.av[cls];
+    const double scale = fuse.visc ? max_dt_scale_at<ND, true>(fuse.ns, u, vs, x, av ? bulk : 0., av ? lap : 0., fuse.max_cfl_c, fuse.max_cfl_d)
+                                   : max_dt_scale_at<ND, false>(fuse.ns, u, vs, x, 0., 0., fuse.max_cfl_c, fuse.max_cfl_d);
     // folded as k_max_dt does: a NaN of this point never wins (std::min(dt, NaN) keeps dt in the reference)
     const double inv = 1. / scale;
     c = (inv < c) ? inv : c;
@@ -980,9 +1031,10 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
   }
   // Write_face of the updated state (Spatial.hpp:507)
   if (pt)
-    for (int v = 0; v < NV; ++v) ld[el * L::PER_D + L::U + v * NQP + qp] = u[v];
+    for (int v = 0; v < NV; ++v) myd[L::U + v * NQP + qp] = u[v];
   __syncthreads();
-  write_faces_from<ND, RS, NT>(m, cls, blk, o, ld + L::U, L::PER_D);
+  write_faces_to<ND, RS, NT, NV>(m, cls, blk, o, ld + L::U, L::PER_D,
+                                 [&](int el2) { return reinterpret_cast<const int*>(ld + el2 * L::PER_D + L::TB_SLOT); });
   if (fuse.block_min) {
     for (int off = 32; off > 0; off /= 2) {
       const double x = __shfl_xor(c, off, 64);
