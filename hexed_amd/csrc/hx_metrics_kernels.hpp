@@ -33,6 +33,9 @@ __device__ inline double det_unit_col(const double* a, int col, int row)
   return det_n(c, ND);
 }
 
+// LDS of k_set_jacobian, per element: positions and Jacobian first (padded), then in their place the metrics (unpadded)
+// and the two arrays their extrapolation to the vertices alternates between. 26 KB per 3D workgroup at row size 6: six
+// workgroups per compute unit, where all arrays side by side (44 KB) left three.
 template <int ND, int RS>
 struct Jac_lds
 {
@@ -40,14 +43,19 @@ struct Jac_lds
   static constexpr int NQP = S::NQP, NVERT = 1 << ND, NM = ND * ND + 1;
   static constexpr int POS = 0;                   // [ND][NQP] quadrature point positions
   static constexpr int JAC = POS + ND * NQP;      // [ND*ND][NQP] Jacobian
-  static constexpr int MET = JAC + ND * ND * NQP; // [ND*ND + 1][NQP] reference-level normals and determinant
-  static constexpr int VX = MET + NM * NQP;       // [NM][NVERT] metrics extrapolated to the vertices
-  static constexpr int PER = VX + NM * NVERT;
+  static constexpr int MET = 0;                   // [NM][NQ] reference-level normals and determinant
+  static constexpr int TMP = MET + NM * S::NQ;    // [NM][2][NFQ] after the first contraction
+  static constexpr int P1 = JAC + ND * ND * NQP, P2 = TMP + 2 * NM * S::NFQ;
+  static constexpr int PER = P1 > P2 ? P1 : P2;
 };
 
 // Deformed_element::set_jacobian of every deformed element. vert: [n][nvert][nd]; adj: [n][2 nd][nfq] or null.
 // Writes the metrics, the element's face normals into its face state blocks and its vertex time step scale into
 // vtss[(n_cartesian + e) * nvert + v].
+// Bound by its writes (10 values per point and 3 per face point at n_dim 3) once the contractions are rows: one thread
+// takes a whole row (or both faces of one) with the operator in scalar registers, and the metrics go to the vertices one
+// dimension at a time, as math::hypercube_matvec does (rows of RS values, instead of every vertex summing over
+// all NQ points: 216 terms at row size 6, each with three table reads). 32^3 elements, row size 6: 1150 -> 296 us (2.5 TB/s).
 template <int ND, int RS>
 __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_set_jacobian(Dev_mesh m, Metric_consts<RS> mc,
                                                                          const double* vert, const double* adj,
@@ -56,102 +64,130 @@ __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_set_jacobian(Dev_mes
   using S = Shape<ND, RS>;
   using R = Row<ND, RS>;
   using L = Jac_lds<ND, RS>;
-  constexpr int NQ = S::NQ, NQP = S::NQP, NFQ = S::NFQ, EPB = S::EPB, NVERT = L::NVERT, NM = L::NM;
+  constexpr int NQ = S::NQ, NQP = S::NQP, NFQ = S::NFQ, EPB = S::EPB, NT = S::BLOCK, NVERT = L::NVERT, NM = L::NM;
   __shared__ double lds[EPB * L::PER];
+  __shared__ double node[RS];
   const int t = threadIdx.x, el = t / NQ, q = t % NQ, qp = S::pad(q);
   const int n = m.n_elem[HX_DEFORMED];
   const int e = blockIdx.x * EPB + el;
   const bool valid = e < n;
+  const int ec = valid ? e : n - 1;
   double* my = lds + el * L::PER;
-  const double* vp = vert + size_t(valid ? e : 0) * NVERT * ND;
-  const double* ap = (adj && valid) ? adj + size_t(e) * 2 * ND * NFQ : nullptr;
+  const double nom = m.nom_size[HX_DEFORMED][ec];
+  double vp[NVERT][ND];
+  for (int v = 0; v < NVERT; ++v)
+    for (int i = 0; i < ND; ++i) vp[v][i] = vert[(size_t(ec) * NVERT + v) * ND + i];
+  // the node coordinates, per lane through LDS (a by-value array indexed per lane is a memory read each time)
+  if (t == 0)
+#pragma unroll
+    for (int k = 0; k < RS; ++k) node[k] = mc.node[k];
+  __syncthreads();
   // position (Deformed_element.cpp:15-58): the n-linear interpolation of the vertices plus, along each direction k,
   // the face adjustments interpolated between the faces (k, 0) and (k, 1) times the edge vector along k
   double x[ND];
-  for (int d = 0; d < ND; ++d) x[d] = mc.node[R::node(q, d)];
-  for (int i = 0; i < ND; ++i) {
-    double p = 0.;
-    for (int v = 0; v < NVERT; ++v) {
-      double w = 1.;
-      for (int d = 0; d < ND; ++d) w *= ((v >> (ND - 1 - d)) & 1) ? x[d] : 1. - x[d];
-      p += w * vp[v * ND + i];
-    }
-    if (ap) {
-      for (int k = 0; k < ND; ++k) {
-        const int f = R::fq(q, k);
-        const double a = ap[2 * k * NFQ + f] * (1. - x[k]) + ap[(2 * k + 1) * NFQ + f] * x[k];
-        double edge = 0.;
-        for (int v = 0; v < NVERT; ++v) {
-          double w = 1.;
-          for (int d = 0; d < ND; ++d)
-            if (d != k) w *= ((v >> (ND - 1 - d)) & 1) ? x[d] : 1. - x[d];
-          edge += (((v >> (ND - 1 - k)) & 1) ? w : -w) * vp[v * ND + i];
-        }
-        p += a * edge;
+  for (int d = 0; d < ND; ++d) x[d] = node[R::node(q, d)];
+  double p[ND] = {};
+#pragma unroll
+  for (int v = 0; v < NVERT; ++v) {
+    double w = 1.;
+    for (int d = 0; d < ND; ++d) w *= ((v >> (ND - 1 - d)) & 1) ? x[d] : 1. - x[d];
+    for (int i = 0; i < ND; ++i) p[i] += w * vp[v][i];
+  }
+  if (adj) {
+    const double* ap = adj + size_t(ec) * 2 * ND * NFQ;
+#pragma unroll
+    for (int k = 0; k < ND; ++k) {
+      const int f = R::fq(q, k);
+      const double a = ap[2 * k * NFQ + f] * (1. - x[k]) + ap[(2 * k + 1) * NFQ + f] * x[k];
+      double edge[ND] = {};
+#pragma unroll
+      for (int v = 0; v < NVERT; ++v) {
+        double w = 1.;
+        for (int d = 0; d < ND; ++d)
+          if (d != k) w *= ((v >> (ND - 1 - d)) & 1) ? x[d] : 1. - x[d];
+        for (int i = 0; i < ND; ++i) edge[i] += (((v >> (ND - 1 - k)) & 1) ? w : -w) * vp[v][i];
       }
+      for (int i = 0; i < ND; ++i) p[i] += a * edge[i];
     }
-    my[L::POS + i * NQP + qp] = valid ? p : 0.;
   }
+  for (int i = 0; i < ND; ++i) my[L::POS + i * NQP + qp] = p[i];
   __syncthreads();
-  // Jacobian: derivative along each reference direction over the nominal size, then determinant and cofactors
-  const double inv_h = valid ? 1. / m.nom_size[HX_DEFORMED][e] : 1.;
-  double J[ND * ND];
-  for (int j = 0; j < ND; ++j) {
-    const int kq = R::node(q, j), base = R::base(q, j), st = R::stride(j);
-    for (int i = 0; i < ND; ++i) {
-      double acc = 0.;
-      for (int k = 0; k < RS; ++k) acc += mc.diff[kq][k] * my[L::POS + i * NQP + S::pad(base + k * st)];
-      J[i * ND + j] = acc * inv_h;
-      my[L::JAC + (i * ND + j) * NQP + qp] = J[i * ND + j];
-    }
-  }
-  double met[NM];
+  // Jacobian: derivative along each reference direction over the nominal size, one row of one coordinate per thread
+#pragma unroll
+  for (int j = 0; j < ND; ++j)
+    for_columns<ND, RS, ND, NT, false>(j, [&](bool, int el2, int i, int, int base, int sd) {
+      double* b = lds + el2 * L::PER;
+      const int e2 = blockIdx.x * EPB + el2;
+      const double inv_h = 1. / m.nom_size[HX_DEFORMED][e2 < n ? e2 : n - 1];
+      double xr[RS], y[RS];
+      load_row(b + L::POS + i * NQP + base, sd, xr);
+      row_matvec(mc.diff, xr, y);
+      double* out = b + L::JAC + (i * ND + j) * NQP + base;
+#pragma unroll
+      for (int k = 0; k < RS; ++k) out[k * sd] = y[k] * inv_h;
+    });
+  __syncthreads();
+  // determinant and cofactors
+  double J[ND * ND], met[NM];
+  for (int a = 0; a < ND * ND; ++a) J[a] = my[L::JAC + a * NQP + qp];
   met[ND * ND] = det_n(J, ND);
   for (int i = 0; i < ND; ++i)
     for (int j = 0; j < ND; ++j) met[i * ND + j] = det_unit_col<ND>(J, i, j);
-  for (int k = 0; k < NM; ++k) my[L::MET + k * NQP + qp] = met[k];
   if (valid) {
     double* out = m.metrics + size_t(e) * NM * NQ;
     for (int k = 0; k < NM; ++k) out[k * NQ + q] = met[k];
   }
-  __syncthreads();
   // face normals (Deformed_element.cpp:91-113): the Jacobian extrapolated to the face, column i_dim replaced by each
-  // unit vector
-  if (valid) {
-    for (int k = q; k < 2 * ND * NFQ; k += NQ) {
-      const int f = k / NFQ, fq = k % NFQ, i_dim = f / 2, sign = f % 2;
-      const int base = R::base_of_fq(fq, i_dim), st = R::stride(i_dim);
-      double FJ[ND * ND];
+  // unit vector; one thread per row, for both faces it ends at
+#pragma unroll
+  for (int i_dim = 0; i_dim < ND; ++i_dim)
+    for_columns<ND, RS, 1, NT, false>(i_dim, [&](bool, int el2, int, int r, int base, int sd) {
+      const int e2 = blockIdx.x * EPB + el2;
+      if (e2 >= n) return;
+      const double* b = lds + el2 * L::PER + L::JAC + base;
+      double FJ[2][ND * ND];
       for (int a = 0; a < ND * ND; ++a) {
-        double acc = 0.;
-        for (int r = 0; r < RS; ++r) acc += mc.bound[sign][r] * my[L::JAC + a * NQP + S::pad(base + r * st)];
-        FJ[a] = acc;
+        double xr[RS];
+        load_row(b + a * NQP, sd, xr);
+        for (int s = 0; s < 2; ++s) FJ[s][a] = row_bound(mc, s, xr);
       }
-      double* face = slot_ptr(m, m.face_slot[HX_DEFORMED][e * 2 * ND + f]);
-      for (int j = 0; j < ND; ++j) face[j * NFQ + fq] = det_unit_col<ND>(FJ, i_dim, j);
+      const int* fs = m.face_slot[HX_DEFORMED] + size_t(e2) * 2 * ND + 2 * i_dim;
+      for (int s = 0; s < 2; ++s) {
+        double* face = slot_ptr(m, fs[s]);
+        for (int j = 0; j < ND; ++j) face[j * NFQ + r] = det_unit_col<ND>(FJ[s], i_dim, j);
+      }
+    });
+  __syncthreads();
+  for (int k = 0; k < NM; ++k) my[L::MET + k * NQ + q] = met[k];
+  // metrics extrapolated to the vertices (math::hypercube_matvec with the boundary matrix), dimension by dimension:
+  // [NM 2^d][RS][rest] -> [NM 2^d][2][rest], one thread per row
+  int src = L::MET, dst = L::TMP;
+#pragma unroll
+  for (int d = 0; d < ND; ++d) {
+    __syncthreads();
+    const int rest = ipow(RS, ND - 1 - d), rows = (NM << d) * rest;
+    for (int k = t; k < EPB * rows; k += NT) {
+      const int el2 = k / rows, kr = k % rows, a = kr / rest, r = kr % rest;
+      const double* in = lds + el2 * L::PER + src + a * RS * rest + r;
+      double* out = lds + el2 * L::PER + dst + a * 2 * rest + r;
+      double xr[RS];
+      load_row(in, rest, xr);
+      for (int s = 0; s < 2; ++s) out[s * rest] = row_bound(mc, s, xr);
     }
-  }
-  // metrics extrapolated to the vertices (math::hypercube_matvec with the boundary matrix)
-  for (int k = q; k < NM * NVERT; k += NQ) {
-    const int a = k / NVERT, v = k % NVERT;
-    double acc = 0.;
-    for (int p = 0; p < NQ; ++p) {
-      double w = 1.;
-      for (int d = 0; d < ND; ++d) w *= mc.bound[(v >> (ND - 1 - d)) & 1][R::node(p, d)];
-      acc += w * my[L::MET + a * NQP + S::pad(p)];
-    }
-    my[L::VX + a * NVERT + v] = acc;
+    const int next = src;
+    src = dst;
+    dst = next;
   }
   __syncthreads();
   if (valid && q < NVERT) {
+    const double* vx = my + src;
     double norm_sum = 0.;
     for (int i = 0; i < ND; ++i) {
       double sq = 0.;
-      for (int j = 0; j < ND; ++j) sq += my[L::VX + (i * ND + j) * NVERT + q] * my[L::VX + (i * ND + j) * NVERT + q];
+      for (int j = 0; j < ND; ++j) sq += vx[(i * ND + j) * NVERT + q] * vx[(i * ND + j) * NVERT + q];
       norm_sum += sqrt(sq);
     }
-    vtss[(size_t(m.n_elem[HX_CARTESIAN]) + e) * NVERT + q] =
-        m.nom_size[HX_DEFORMED][e] * my[L::VX + ND * ND * NVERT + q] / norm_sum;
+    vtss[(size_t(m.n_elem[HX_CARTESIAN]) + e) * NVERT + q] = nom * vx[ND * ND * NVERT + q] / norm_sum;
   }
 }
 
