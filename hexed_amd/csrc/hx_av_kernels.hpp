@@ -59,13 +59,17 @@ __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_av_write_face(Dev_me
   using S = Shape<ND, RS>;
   constexpr int NQ = S::NQ, NQP = S::NQP, EPB = S::EPB, NVAR = Av_vars<ND, RS, KIND>::N;
   __shared__ double lds[EPB * NVAR * NQP];
+  __shared__ int fsl[EPB * 2 * ND];
   const int t = threadIdx.x, el = t / NQ, q = t % NQ;
-  const int e = blockIdx.x * EPB + el;
-  const bool valid = e < m.n_elem[cls];
-  for (int v = 0; v < NVAR; ++v)
-    lds[el * NVAR * NQP + v * NQP + S::pad(q)] = valid ? av_extrap<ND, RS, KIND>(m, cls, e, v, q) : 0.;
+  const int n = m.n_elem[cls];
+  const int e = blockIdx.x * EPB + el, ec = e < n ? e : n - 1;
+  const int slot = staged_slot<ND, RS>(m, cls, blockIdx.x, t);
+  double u[NVAR];
+  for (int v = 0; v < NVAR; ++v) u[v] = av_extrap<ND, RS, KIND>(m, cls, ec, v, q);
+  if (t < EPB * 2 * ND) fsl[t] = slot;
+  for (int v = 0; v < NVAR; ++v) lds[el * NVAR * NQP + v * NQP + S::pad(q)] = u[v];
   __syncthreads();
-  write_faces_from<ND, RS, S::BLOCK, NVAR>(m, cls, blockIdx.x, o, lds, NVAR * NQP);
+  write_faces_to<ND, RS, S::BLOCK, NVAR>(m, cls, blockIdx.x, o, lds, NVAR * NQP, [&](int el2) { return fsl + el2 * 2 * ND; });
 }
 
 // ---- Neighbor<Advection / Smooth_art_visc / Fix_therm_admis> (Spatial.hpp:613-704) -----------------------------
@@ -149,6 +153,7 @@ __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_adv_local(Dev_mesh m
   constexpr int NQ = S::NQ, NQP = S::NQP, NFQ = S::NFQ, EPB = S::EPB, NT = S::BLOCK;
   constexpr int cls = DEF ? HX_DEFORMED : HX_CARTESIAN;
   __shared__ double lds[EPB * L::PER];
+  __shared__ int fsl[EPB * 2 * ND];
   const int t = threadIdx.x, el = t / NQ, q = t % NQ, qp = S::pad(q);
   const int n = m.n_elem[cls];
   const int e = blockIdx.x * EPB + el;
@@ -156,31 +161,39 @@ __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_adv_local(Dev_mesh m
   double* my = lds + el * L::PER;
   const Contraction<RS, Fp64_form> con(o, nullptr);
 
+  // loads in two steps, without branches, as in k_local_ns: the face slots and the point data, then the numerical face
+  // fluxes (the first rs variables of block 0 of every face), one face point per thread, held in registers and staged
+  // into LDS one direction at a time
+  using I = Face_items<ND, RS, NT>;
+  const int ec = valid ? e : n - 1;
+  int own[I::N];
+#pragma unroll
+  for (int k = 0; k < I::N; ++k) {
+    const I f(blockIdx.x, t, k);
+    own[k] = m.face_slot[cls][size_t(f.e2 < n ? f.e2 : n - 1) * 2 * ND + f.face];
+  }
   double vel[ND], a[RS];
-  for (int j = 0; j < ND; ++j) vel[j] = valid ? m.state[cls][(size_t(e) * (ND + 2) + j) * NQ + q] : 0.;
-  for (int i = 0; i < RS; ++i) a[i] = valid ? m.advection[cls][(size_t(e) * RS + i) * NQ + q] : 0.;
+  for (int j = 0; j < ND; ++j) vel[j] = m.state[cls][(size_t(ec) * (ND + 2) + j) * NQ + q];
+  for (int i = 0; i < RS; ++i) a[i] = m.advection[cls][(size_t(ec) * RS + i) * NQ + q];
   double det = 1.;
   double met[ND][ND];
   if constexpr (DEF) {
-    const double* mt = m.metrics + size_t(e) * (ND * ND + 1) * NQ;
+    const double* mt = m.metrics + size_t(ec) * (ND * ND + 1) * NQ;
     for (int i = 0; i < ND; ++i)
-      for (int j = 0; j < ND; ++j) met[i][j] = valid ? mt[(i * ND + j) * NQ + q] : double(i == j);
-    det = valid ? mt[ND * ND * NQ + q] : 1.;
+      for (int j = 0; j < ND; ++j) met[i][j] = mt[(i * ND + j) * NQ + q];
+    det = mt[ND * ND * NQ + q];
   }
-  // numerical face fluxes (the first rs variables of block 0 of every face), loaded now into registers, direction by
-  // direction, and staged into LDS one direction at a time: entry k of direction i's block [EPB][2][RS][NFQ] is held by
-  // thread k mod NT
-  constexpr int DB = EPB * 2 * RS * NFQ, FPD = (DB + NT - 1) / NT;
-  double sbr[ND][FPD];
+  double sbr[I::N][RS];
 #pragma unroll
-  for (int i = 0; i < ND; ++i)
-#pragma unroll
-    for (int j = 0; j < FPD; ++j) {
-      const int k = t + j * NT, el2 = k / (2 * RS * NFQ), r = k % (2 * RS * NFQ);
-      const int e2 = blockIdx.x * EPB + el2;
-      sbr[i][j] = k < DB && e2 < n ? slot_ptr(m, m.face_slot[cls][e2 * 2 * ND + 2 * i + r / (RS * NFQ)])[r % (RS * NFQ)]
-                                   : 0.;
-    }
+  for (int k = 0; k < I::N; ++k) {
+    const I f(blockIdx.x, t, k);
+    const double* s = slot_ptr(m, own[k]) + f.p;
+    for (int v = 0; v < RS; ++v) sbr[k][v] = s[v * NFQ];
+    if (f.own && f.p == 0) fsl[f.el2 * 2 * ND + f.face] = own[k];
+  }
+  // what the update at the end reads: requested ahead of the last direction's row phase
+  double rcv[RS];
+  double tss = 0., d_pos = 1.;
   for (int i = 0; i < ND; ++i) {
     double vn = 0;
     for (int j = 0; j < ND; ++j) {
@@ -190,9 +203,20 @@ __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_adv_local(Dev_mesh m
     if (i) __syncthreads();
     for (int v = 0; v < RS; ++v) my[L::F + v * NQP + qp] = ac.adv_node[v] * vn * a[v];
 #pragma unroll
-    for (int j = 0; j < FPD; ++j) {
-      const int k = t + j * NT;
-      if (k < DB) lds[(k / (2 * RS * NFQ)) * L::PER + L::SB + k % (2 * RS * NFQ)] = sbr[i][j];
+    for (int k = 0; k < I::N; ++k) {
+      const I f(blockIdx.x, t, k);
+      if (f.own && f.face / 2 == i)
+        for (int v = 0; v < RS; ++v) lds[f.el2 * L::PER + L::SB + (f.face % 2 * RS + v) * NFQ + f.p] = sbr[k][v];
+    }
+    if (i == ND - 1) {
+      tss = m.tss[cls][size_t(ec) * NQ + q];
+      d_pos = m.nom_size[cls][ec];
+      if (stage) {
+        const double* rc = m.rcache[cls] + size_t(ec) * S::NRC * NQ;
+        for (int v = 0; v < RS; ++v) rcv[v] = rc[v * NQ + q];
+      } else {
+        for (int v = 0; v < RS; ++v) rcv[v] = 0.;
+      }
     }
     __syncthreads();
     for_columns<ND, RS, RS, NT, false>(i, [&](bool, int el2, int v, int r, int base, int sd) {
@@ -205,8 +229,6 @@ __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_adv_local(Dev_mesh m
   }
   __syncthreads();
   if (valid) {
-    const double d_pos = m.nom_size[cls][e];
-    const double tss = m.tss[cls][size_t(e) * NQ + q];
     double mult = coef * tss / d_pos;
     if constexpr (DEF) mult /= det;
     double src_mult = d_pos;
@@ -216,7 +238,7 @@ __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_adv_local(Dev_mesh m
     for (int v = 0; v < RS; ++v) {
       double u = my[L::RT + v * NQP + qp];
       if (stage) {
-        u -= rc[v * NQ + q];
+        u -= rcv[v];
       } else {
         rc[v * NQ + q] = u;
         u += src_mult * (2 / advect_length);
@@ -243,7 +265,7 @@ __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_adv_local(Dev_mesh m
   for (int j = 0; j < ND; ++j) my[L::U + j * NQP + qp] = vel[j];
   for (int v = 0; v < RS; ++v) my[L::U + (ND + v) * NQP + qp] = a[v];
   __syncthreads();
-  write_faces_from<ND, RS, NT, ND + RS>(m, cls, blockIdx.x, o, lds + L::U, L::PER);
+  write_faces_to<ND, RS, NT, ND + RS>(m, cls, blockIdx.x, o, lds + L::U, L::PER, [&](int el2) { return fsl + el2 * 2 * ND; });
 }
 
 // ---- Local<Smooth_art_visc / Fix_therm_admis> (Spatial.hpp:326-509, stage 0) -----------------------------------
@@ -285,51 +307,58 @@ __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_sav_local(Dev_mesh m
   double* my = lds + el * L::PER;
   const Contraction<RS, Fp64_form> con(o, nullptr);
 
-  double uv[NS];
-  for (int v = 0; v < NS; ++v) uv[v] = valid ? diff_vars<ND, RS, KIND>(m, cls, e)[v * NQ + q] : 0.;
-  for (int v = 0; v < NS; ++v) my[L::U + v * NQP + qp] = uv[v];
-  // read with the first loads rather than where they are used: the source's forcing[0] (its forcing[1] and [2] are
-  // the first two diffused variables, held above), the update's time step scale, and the elements' face slots (into
-  // LDS, for the flux extrapolations)
-  const double f0 = (SAV && valid) ? m.forcing[cls][size_t(e) * 4 * NQ + q] : 0.;
-  const double tss_q = valid ? m.tss[cls][size_t(e) * NQ + q] : 0.;
-  // (the slots are staged where their LDS leaves the workgroups per compute unit as they are)
+  // loads in two steps, without branches, as in k_local_ns: the face tables and the point data (the source's forcing[0]
+  // among them; its forcing[1] and [2] are the first two diffused variables), then the face data, one face point per
+  // thread. (The face slots stay in LDS for the flux extrapolations where that leaves the workgroups per compute unit.)
   constexpr int LDS = 8 * EPB * L::PER, SLOTS = 4 * EPB * 2 * ND;
   constexpr bool STAGE = 163840 / (LDS + SLOTS) == 163840 / LDS;
   __shared__ int fsl[STAGE ? EPB * 2 * ND : 1];
-  if (STAGE && t < EPB * 2 * ND) {
-    const int e2 = blockIdx.x * EPB + t / (2 * ND);
-    fsl[t] = e2 < n ? m.face_slot[cls][e2 * 2 * ND + t % (2 * ND)] : 0;
+  using I = Face_items<ND, RS, NT>;
+  const int ec = valid ? e : n - 1;
+  int own[I::N], fns[I::N];
+#pragma unroll
+  for (int k = 0; k < I::N; ++k) {
+    const I f(blockIdx.x, t, k);
+    const size_t kf = size_t(f.e2 < n ? f.e2 : n - 1) * 2 * ND + f.face;
+    own[k] = m.face_slot[cls][kf];
+    if constexpr (DEF) fns[k] = m.face_nslot[kf];
   }
+  double uv[NS];
+  for (int v = 0; v < NS; ++v) uv[v] = diff_vars<ND, RS, KIND>(m, cls, ec)[v * NQ + q];
+  const double f0 = SAV ? m.forcing[cls][size_t(ec) * 4 * NQ + q] : 0.;
+  const double tss_q = m.tss[cls][size_t(ec) * NQ + q], d_pos = m.nom_size[cls][ec];
   double det = 1.;
   double met[ND][ND];
   if constexpr (DEF) {
-    const double* mt = m.metrics + size_t(e) * (ND * ND + 1) * NQ;
+    const double* mt = m.metrics + size_t(ec) * (ND * ND + 1) * NQ;
     for (int i = 0; i < ND; ++i)
-      for (int j = 0; j < ND; ++j) met[i][j] = valid ? mt[(i * ND + j) * NQ + q] : double(i == j);
-    // the column of the normals that gradient component 0 needs (each later component's replaces it)
-    for (int i = 0; i < ND; ++i) my[L::SN + i * NQP + qp] = met[i][0];
-    det = valid ? mt[ND * ND * NQ + q] : 1.;
+      for (int j = 0; j < ND; ++j) met[i][j] = mt[(i * ND + j) * NQ + q];
+    det = mt[ND * ND * NQ + q];
   }
-  for (int k = t; k < EPB * 2 * ND * NS * NFQ; k += NT) {
-    const int el2 = k / (2 * ND * NS * NFQ), r = k % (2 * ND * NS * NFQ), f = r / (NS * NFQ), vq = r % (NS * NFQ);
-    const int e2 = blockIdx.x * EPB + el2;
-    lds[el2 * L::PER + L::SL + r] = e2 < n ? slot_ptr(m, m.face_slot[cls][e2 * 2 * ND + f])[NV * NFQ + vq] : 0.;
-  }
-  if constexpr (DEF) {
-    for (int k = t; k < EPB * 2 * ND * ND * NFQ; k += NT) {
-      const int el2 = k / (2 * ND * ND * NFQ), r = k % (2 * ND * ND * NFQ), f = r / (ND * NFQ), jq = r % (ND * NFQ);
-      const int e2 = blockIdx.x * EPB + el2;
-      double val = 0.;
-      if (e2 < n) {
-        const int ns_ = m.face_nslot[e2 * 2 * ND + f];
-        val = ns_ >= 0 ? m.normals[size_t(ns_) * ND * NFQ + jq] : double(jq / NFQ == f / 2);
-      }
-      lds[el2 * L::PER + L::SFN + r] = val;
+#pragma unroll
+  for (int k = 0; k < I::N; ++k) {
+    const I f(blockIdx.x, t, k);
+    const double* l = slot_ptr(m, own[k]) + NV * NFQ;
+    double sl[NS], nf[ND];
+    for (int v = 0; v < NS; ++v) sl[v] = l[v * NFQ + f.p];
+    if constexpr (DEF) {
+      // (a face in a Cartesian connection uses the identity normal)
+      const double* np = fns[k] >= 0 ? m.normals + size_t(fns[k]) * ND * NFQ : l;
+      for (int j = 0; j < ND; ++j) nf[j] = np[j * NFQ + f.p];
+    }
+    if (f.own) {
+      double* b = lds + f.el2 * L::PER;
+      for (int v = 0; v < NS; ++v) b[L::SL + (f.face * NS + v) * NFQ + f.p] = sl[v];
+      if constexpr (DEF)
+        for (int j = 0; j < ND; ++j) b[L::SFN + (f.face * ND + j) * NFQ + f.p] = fns[k] >= 0 ? nf[j] : double(j == f.face / 2);
+      if (STAGE && f.p == 0) fsl[f.el2 * 2 * ND + f.face] = own[k];
     }
   }
+  for (int v = 0; v < NS; ++v) my[L::U + v * NQP + qp] = uv[v];
+  // the column of the normals that gradient component 0 needs (each later component's replaces it)
+  if constexpr (DEF)
+    for (int i = 0; i < ND; ++i) my[L::SN + i * NQP + qp] = met[i][0];
   __syncthreads();
-  const double d_pos = valid ? m.nom_size[cls][e] : 1.;
   const double inv_h = 1. / d_pos;
   double grad[NS][ND];
   for (int j = 0; j < ND; ++j) {
@@ -372,7 +401,7 @@ __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_sav_local(Dev_mesh m
     double src_mult = d_pos;
     if constexpr (DEF) src_mult *= det;
     for (int v = 0; v < NS; ++v) {
-      const double f = valid ? fabs(v == 0 ? f0 : uv[v - 1]) : 0.;
+      const double f = fabs(v == 0 ? f0 : uv[v - 1]);
       my[L::RT + v * NQP + qp] = src_mult * (((v == 1) ? sqrt(f) : f) / diff_time);
     }
   } else {
@@ -436,15 +465,30 @@ __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_sav_reconcile(Dev_me
   const int e = blockIdx.x * EPB + el;
   const bool valid = e < n;
   double* my = lds + el * PER;
-  // the point's own data are read with the face data, so that their latency overlaps it
+  // the point's own data are read with the face data, so that their latency overlaps it (without branches, as in
+  // k_local_ns)
+  __shared__ int fsl[EPB * 2 * ND];
+  using I = Face_items<ND, RS, S::BLOCK>;
+  const int ec = valid ? e : n - 1;
+  int own[I::N];
+#pragma unroll
+  for (int k = 0; k < I::N; ++k) {
+    const I f(blockIdx.x, t, k);
+    own[k] = m.face_slot[cls][size_t(f.e2 < n ? f.e2 : n - 1) * 2 * ND + f.face];
+    if (f.own && f.p == 0) fsl[f.el2 * 2 * ND + f.face] = own[k];
+  }
   double fv[NS];
-  for (int v = 0; v < NS; ++v) fv[v] = valid ? diff_vars<ND, RS, KIND>(m, cls, e)[v * NQ + q] : 0.;
-  const double tss = valid ? m.tss[cls][size_t(e) * NQ + q] : 0., nom = valid ? m.nom_size[cls][e] : 1.;
-  const double det = (DEF && valid) ? m.metrics[size_t(e) * (ND * ND + 1) * NQ + ND * ND * NQ + q] : 1.;
-  for (int k = t; k < EPB * PF; k += S::BLOCK) {
-    const int el2 = k / PF, r = k % PF, f = r / (NS * NFQ), vq = r % (NS * NFQ);
-    const int e2 = blockIdx.x * EPB + el2;
-    lds[el2 * PER + r] = e2 < n ? slot_ptr(m, m.face_slot[cls][e2 * 2 * ND + f])[NV * NFQ + vq] : 0.;
+  for (int v = 0; v < NS; ++v) fv[v] = diff_vars<ND, RS, KIND>(m, cls, ec)[v * NQ + q];
+  const double tss = m.tss[cls][size_t(ec) * NQ + q], nom = m.nom_size[cls][ec];
+  const double det = DEF ? m.metrics[size_t(ec) * (ND * ND + 1) * NQ + ND * ND * NQ + q] : 1.;
+#pragma unroll
+  for (int k = 0; k < I::N; ++k) {
+    const I f(blockIdx.x, t, k);
+    const double* l = slot_ptr(m, own[k]) + NV * NFQ;
+    double j[NS];
+    for (int v = 0; v < NS; ++v) j[v] = l[v * NFQ + f.p];
+    if (f.own)
+      for (int v = 0; v < NS; ++v) lds[f.el2 * PER + (f.face * NS + v) * NFQ + f.p] = j[v];
   }
   __syncthreads();
   double rate[NS] = {};
@@ -465,7 +509,7 @@ __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_sav_reconcile(Dev_me
   }
   for (int v = 0; v < NS; ++v) my[PF + v * NQP + S::pad(q)] = fv[v];
   __syncthreads();
-  write_faces_from<ND, RS, S::BLOCK, NS>(m, cls, blockIdx.x, o, lds + PF, PER);
+  write_faces_to<ND, RS, S::BLOCK, NS>(m, cls, blockIdx.x, o, lds + PF, PER, [&](int el2) { return fsl + el2 * 2 * ND; });
 }
 
 // ---- Max_dt<Advection / Smooth_art_visc> (Spatial.hpp:784-828) ------------------------------------------------

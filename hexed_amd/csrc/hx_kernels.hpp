@@ -427,26 +427,6 @@ __device__ inline void filter_columns(const Eops<RS, double>& o, T* buf, int per
   __syncthreads();
 }
 
-// Loads block `ldg` (0: state/flux, 1: LDG) of every face of the workgroup's elements into dst[EPB][2ND][NV][NFQ]
-// (element stride `per`).
-template <int ND, int RS, int NT>
-__device__ inline void load_faces(const Dev_mesh& m, int cls, int blk, int ldg, double* dst, int per)
-{
-  using S = Shape<ND, RS>;
-  constexpr int PF = 2 * ND * S::NV * S::NFQ;
-  const int n = m.n_elem[cls];
-  for (int k = threadIdx.x; k < S::EPB * PF; k += NT) {
-    const int el = k / PF, r = k % PF, f = r / (S::NV * S::NFQ), vq = r % (S::NV * S::NFQ);
-    const int e = blk * S::EPB + el;
-    if (e < n) {
-      const int slot = m.face_slot[cls][e * 2 * ND + f];
-      dst[el * per + r] = (ldg ? slot_ptr(m, slot) + S::NV * S::NFQ : state_ptr(m, slot, m.alt_rd))[vq];
-    } else {
-      dst[el * per + r] = 0.;
-    }
-  }
-}
-
 // Write_face of the FP64 padded [NVAR][NQP] arrays at `buf` (element stride `per`) into block 0 of every face
 // (Spatial.hpp:29-71); slots(el2) points at the 2 ND face slots of element el2 of the workgroup
 template <int ND, int RS, int NT, int NVAR, class F>
@@ -467,13 +447,35 @@ __device__ inline void write_faces_to(const Dev_mesh& m, int cls, int blk, const
     });
   }
 }
-template <int ND, int RS, int NT, int NVAR = Shape<ND, RS>::NV>
-__device__ inline void write_faces_from(const Dev_mesh& m, int cls, int blk, const Eops<RS, double>& o, const double* buf,
-                                        int per)
+// Entry t of the workgroup's face slots (t < EPB 2 ND: element t / 2 ND, face t % 2 ND), requested with a kernel's first
+// loads and kept in LDS for its face writes, so that these need no memory read of their own
+template <int ND, int RS>
+__device__ __forceinline__ int staged_slot(const Dev_mesh& m, int cls, int blk, int t)
 {
-  write_faces_to<ND, RS, NT, NVAR>(m, cls, blk, o, buf, per,
-                                   [&](int el) { return m.face_slot[cls] + (blk * Shape<ND, RS>::EPB + el) * 2 * ND; });
+  const int n = m.n_elem[cls], e = blk * Shape<ND, RS>::EPB + t / (2 * ND);
+  return m.face_slot[cls][size_t(e < n ? e : n - 1) * 2 * ND + t % (2 * ND)];
 }
+
+// The face points of a workgroup's elements dealt out to its NT threads, N per thread: item k of thread t is face point p
+// of face `face` of element el2 of the workgroup (element e2 of the class); `own` is false, and the item that of thread
+// 0, past the last one.
+template <int ND, int RS, int NT>
+struct Face_items
+{
+  using S = Shape<ND, RS>;
+  static constexpr int NFP = 2 * ND * S::NFQ, N = (S::EPB * NFP + NT - 1) / NT;
+  int el2, e2, face, p;
+  bool own;
+  __device__ __forceinline__ Face_items(int blk, int t, int k)
+  {
+    own = t + k * NT < S::EPB * NFP;
+    const int kk = own ? t + k * NT : 0, r = kk % NFP;
+    el2 = kk / NFP;
+    e2 = blk * S::EPB + el2;
+    face = r / S::NFQ;
+    p = r % S::NFQ;
+  }
+};
 
 // ---- Neighbor (Spatial.hpp:613-704) ----------------------------------------------------------------------
 // The numerical flux at face point f of connection con of class DEF, and where each side keeps it: side 0 at f, side
@@ -882,21 +884,14 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
 
   // The loads go out in two steps, as in k_local_ns: the face table, then what it points at together with the point
   // data. Threads past the last element or point read the last one's data instead of branching.
-  constexpr int NFP = 2 * ND * NFQ, FPT = (EPB * NFP + NT - 1) / NT;
-  const auto face_item = [&](int k, int& el2, int& e2, int& face, int& p) {
-    const int kk = t + k * NT < EPB * NFP ? t + k * NT : 0, r = kk % NFP;
-    el2 = kk / NFP;
-    e2 = blk * EPB + el2;
-    face = r / NFQ;
-    p = r % NFQ;
-  };
+  using I = Face_items<ND, RS, NT>;
+  constexpr int FPT = I::N;
   const int ec = e < n ? e : n - 1;
   Face_ref fr[FPT];
 #pragma unroll
   for (int k = 0; k < FPT; ++k) {
-    int el2, e2, face, p;
-    face_item(k, el2, e2, face, p);
-    fr[k] = face_ref(m, cls, size_t(e2 < n ? e2 : n - 1) * 2 * ND + face);
+    const I f(blk, t, k);
+    fr[k] = face_ref(m, cls, size_t(f.e2 < n ? f.e2 : n - 1) * 2 * ND + f.face);
   }
   // (the first contraction follows a barrier)
   if constexpr (P::mfma) lds_mfma_operands<RS, NT>(od, mtab);
@@ -909,9 +904,8 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
   double nrm[ND];
 #pragma unroll
   for (int k = 0; k < FPT; ++k) {
-    int el2, e2, face, p;
-    face_item(k, el2, e2, face, p);
-    const bool own = t + k * NT < EPB * NFP;
+    const I f(blk, t, k);
+    const int el2 = f.el2, face = f.face, p = f.p;
     double fl[NV], avg[NV];
     Face_in<ND, RS> in;
     if constexpr (FOLD) {
@@ -926,8 +920,8 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
         for (int j = 0; j < ND; ++j) nrm[j] = mt[j * NQ];
     }
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (FOLD) face_flux<ND, RS, false>(m, fr[k], p, own && e2 < n, in, fl, avg);
-    if (own)
+    if constexpr (FOLD) face_flux<ND, RS, false>(m, fr[k], p, f.own && f.e2 < n, in, fl, avg);
+    if (f.own)
       for (int v = 0; v < NV; ++v) ld[el2 * L::PER_D + L::sb(face) + v * NFQ + p] = fl[v];
   }
   const double p64 = P::mfma ? pressure_of<ND>(u) : 0.;
@@ -1160,22 +1154,15 @@ void k_local_ns(Dev_mesh m, Eops<RS, double> o,
   // it. (With a branch per operand the loads were waited for one after the other, about eleven memory latencies, a third
   // of the time an element stayed on its compute unit: FP64 3.10 -> 2.49 ms, FP32-MFMA 2.79 -> 2.36 ms per launch on the 48^3
   // deformed mesh.)
-  constexpr int NFP = 2 * ND * NFQ, FPT = (EPB * NFP + NT - 1) / NT;
-  const auto face_item = [&](int k, int& el2, int& e2, int& face, int& p) {
-    const int kk = t + k * NT < EPB * NFP ? t + k * NT : 0, r = kk % NFP;
-    el2 = kk / NFP;
-    e2 = blk * EPB + el2;
-    face = r / NFQ;
-    p = r % NFQ;
-  };
+  using I = Face_items<ND, RS, NT>;
+  constexpr int FPT = I::N;
   const int ec = e < n ? e : n - 1;
   Face_ref fr[FPT];
   int fns[FPT];
 #pragma unroll
   for (int k = 0; k < FPT; ++k) {
-    int el2, e2, face, p;
-    face_item(k, el2, e2, face, p);
-    const size_t kf = size_t(e2 < n ? e2 : n - 1) * 2 * ND + face;
+    const I f(blk, t, k);
+    const size_t kf = size_t(f.e2 < n ? f.e2 : n - 1) * 2 * ND + f.face;
     fr[k] = face_ref(m, cls, kf);
     if constexpr (DEF) fns[k] = m.face_nslot[kf];
   }
@@ -1190,9 +1177,8 @@ void k_local_ns(Dev_mesh m, Eops<RS, double> o,
   double sbf[FPT][NV];
 #pragma unroll
   for (int k = 0; k < FPT; ++k) {
-    int el2, e2, face, p;
-    face_item(k, el2, e2, face, p);
-    const bool own = t + k * NT < EPB * NFP;
+    const I f(blk, t, k);
+    const int el2 = f.el2, face = f.face, p = f.p;
     double nf[DEF ? ND : 1], avg[NV];
     Face_in<ND, RS> in;
     if constexpr (FOLD) {
@@ -1217,8 +1203,8 @@ void k_local_ns(Dev_mesh m, Eops<RS, double> o,
         for (int i = 0; i < ND; ++i) metd[i][0] = mt[i * ND * NQ + q];
     }
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (FOLD) face_flux<ND, RS, true>(m, fr[k], p, own && e2 < n, in, sbf[k], avg);
-    if (own) {
+    if constexpr (FOLD) face_flux<ND, RS, true>(m, fr[k], p, f.own && f.e2 < n, in, sbf[k], avg);
+    if (f.own) {
       for (int v = 0; v < NV; ++v) ld[el2 * L::PER_D + L::SL + (face * NV + v) * NFQ + p] = avg[v];
       if constexpr (DEF)
         for (int j = 0; j < ND; ++j)
@@ -1341,10 +1327,9 @@ void k_local_ns(Dev_mesh m, Eops<RS, double> o,
   if constexpr (!L::SB_EARLY) {
 #pragma unroll
     for (int k = 0; k < FPT; ++k) {
-      int el2, e2, face, p;
-      face_item(k, el2, e2, face, p);
-      if (t + k * NT < EPB * NFP)
-        for (int v = 0; v < NV; ++v) ld[el2 * L::PER_D + L::SB + (face * NV + v) * NFQ + p] = sbf[k][v];
+      const I f(blk, t, k);
+      if (f.own)
+        for (int v = 0; v < NV; ++v) ld[f.el2 * L::PER_D + L::SB + (f.face * NV + v) * NFQ + f.p] = sbf[k][v];
     }
   }
   // residual along each direction (Spatial.hpp:444-470). The viscous flux goes first (it is also extrapolated to the
@@ -1446,17 +1431,19 @@ struct Reconcile_lds
   static constexpr int PER = U + S::NV * S::NQP;
 };
 
-// waves per SIMD that Reconcile_ldg_flux's LDS allows, at most 8: the register target follows it
+// waves per SIMD that Reconcile_ldg_flux's LDS allows, at most 8 (7 at row size 8, which spills at 8): the register
+// target follows it
 template <int ND, int RS>
 constexpr int reconcile_waves()
 {
   constexpr int lds = Shape<ND, RS>::EPB * 8 * Reconcile_lds<ND, RS>::PER;
   constexpr int w = (163840 / lds) * ((Shape<ND, RS>::BLOCK + 63) / 64) / 4;
-  return w < 1 ? 1 : (w > 8 ? 8 : w);
+  constexpr int cap = RS == 8 ? 7 : 8;
+  return w < 1 ? 1 : (w > cap ? cap : w);
 }
 
 template <int ND, int RS>
-__device__ __forceinline__ void ldg_jump(const Dev_mesh& m, int cls, int e, int face, int p, double (&out)[ND + 2]);
+__device__ __forceinline__ void ldg_jump(const Dev_mesh& m, const Face_ref& r, int p, double (&out)[ND + 2]);
 
 // FOLD: the jumps are formed here from both sides' LDG blocks (ldg_jump) instead of read from the slots
 template <int ND, int RS, bool DEF, bool FOLD = false>
@@ -1470,28 +1457,40 @@ void k_reconcile_ldg(Dev_mesh m, Eops<RS, double> o, double dt, const double* __
   constexpr int NQ = S::NQ, NFQ = S::NFQ, NV = S::NV, EPB = S::EPB;
   constexpr int cls = DEF ? HX_DEFORMED : HX_CARTESIAN;
   __shared__ double lds[EPB * L::PER];
+  __shared__ int fsl[EPB * 2 * ND];
   const int t = threadIdx.x, el = t / NQ, q = t % NQ;
   const int blk = blockIdx.x;
   const int n = m.n_elem[cls];
   const int e = blk * EPB + el;
   const bool valid = e < n;
   double* my = lds + el * L::PER;
+  // loads in two steps, without branches, as in k_local_ns: the face table, then the face and point data
+  using I = Face_items<ND, RS, S::BLOCK>;
+  const int ec = valid ? e : n - 1;
+  Face_ref fr[I::N];
+#pragma unroll
+  for (int k = 0; k < I::N; ++k) {
+    const I f(blk, t, k);
+    fr[k] = face_ref(m, cls, size_t(f.e2 < n ? f.e2 : n - 1) * 2 * ND + f.face);
+    if (f.own && f.p == 0) fsl[f.el2 * 2 * ND + f.face] = fr[k].own;
+  }
   double u[NV];
-  const double* st = m.state[cls] + size_t(e) * NV * NQ;
-  for (int v = 0; v < NV; ++v) u[v] = valid ? st[v * NQ + q] : 0.;
-  if constexpr (FOLD) {
-    constexpr int NFP = 2 * ND * NFQ;
-    for (int k = t; k < EPB * NFP; k += S::BLOCK) {
-      const int el2 = k / NFP, r = k % NFP, face = r / NFQ, p = r % NFQ;
-      const int e2 = blk * EPB + el2;
-      double jv[NV];
-      if (e2 < n) ldg_jump<ND, RS>(m, cls, e2, face, p, jv);
-      else
-        for (int v = 0; v < NV; ++v) jv[v] = 0.;
-      for (int v = 0; v < NV; ++v) lds[el2 * L::PER + L::SL + (face * NV + v) * NFQ + p] = jv[v];
+  const double* st = m.state[cls] + size_t(ec) * NV * NQ;
+  for (int v = 0; v < NV; ++v) u[v] = st[v * NQ + q];
+  const double tss_q = m.tss[cls][size_t(ec) * NQ + q], nom = m.nom_size[cls][ec];
+  const double det = DEF ? m.metrics[size_t(ec) * (ND * ND + 1) * NQ + ND * ND * NQ + q] : 1.;
+#pragma unroll
+  for (int k = 0; k < I::N; ++k) {
+    const I f(blk, t, k);
+    double jv[NV];
+    if constexpr (FOLD) {
+      ldg_jump<ND, RS>(m, fr[k], f.p, jv);
+    } else {
+      const double* l = slot_ptr(m, fr[k].own) + NV * NFQ;
+      for (int v = 0; v < NV; ++v) jv[v] = l[v * NFQ + f.p];
     }
-  } else {
-    load_faces<ND, RS, S::BLOCK>(m, cls, blk, 1, lds + L::SL, L::PER);
+    if (f.own)
+      for (int v = 0; v < NV; ++v) lds[f.el2 * L::PER + L::SL + (f.face * NV + v) * NFQ + f.p] = jv[v];
   }
   __syncthreads();
   // -boundary_term(jump) (Spatial.hpp:560-570)
@@ -1508,8 +1507,8 @@ void k_reconcile_ldg(Dev_mesh m, Eops<RS, double> o, double dt, const double* __
     for (int v = 0; v < NV; ++v) rate[v] = my[L::U + v * S::NQP + S::pad(q)];
   }
   if (valid) {
-    double mult = step_coef(dt, dtp) * m.tss[cls][size_t(e) * NQ + q] / m.nom_size[cls][e];
-    if constexpr (DEF) mult /= m.metrics[size_t(e) * (ND * ND + 1) * NQ + ND * ND * NQ + q];
+    double mult = step_coef(dt, dtp) * tss_q / nom;
+    if constexpr (DEF) mult /= det;
     if (compute_residual) {
       double* rc = m.rcache[cls] + size_t(e) * S::NRC * NQ;
       for (int v = 0; v < NV; ++v) rc[v * NQ + q] += rate[v] * mult;
@@ -1525,12 +1524,12 @@ void k_reconcile_ldg(Dev_mesh m, Eops<RS, double> o, double dt, const double* __
   __syncthreads();
   for (int v = 0; v < NV; ++v) my[L::U + v * S::NQP + S::pad(q)] = u[v];
   __syncthreads();
-  write_faces_from<ND, RS, S::BLOCK>(m, cls, blk, o, lds + L::U, L::PER);
+  write_faces_to<ND, RS, S::BLOCK, NV>(m, cls, blk, o, lds + L::U, L::PER, [&](int el2) { return fsl + el2 * 2 * ND; });
 }
 
 // ---- Write_face (Spatial.hpp:60-70) ----------------------------------------------------------------------
 // Write_face (Spatial.hpp:29-71) of the state: staged in LDS in the padded layout, then one thread per column of each
-// direction in turn extrapolating it to both of that direction's faces (write_faces_from, the operator constants
+// direction in turn extrapolating it to both of that direction's faces (write_faces_to, the operator constants
 // taken by value). scale_velocity 1: first divide the momentum by sqrt(2 rho E) in the state itself, the advection
 // velocity of Solver::update_art_visc_smoothness (Solver.cpp:468-478); 2: multiply it back (Solver.cpp:570-574).
 // Either way the Write_face that follows it in the reference reads the state once.
@@ -1541,19 +1540,23 @@ __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_write_face(Dev_mesh 
   using S = Shape<ND, RS>;
   constexpr int NQ = S::NQ, NQP = S::NQP, NV = S::NV, EPB = S::EPB;
   __shared__ double su[EPB * NV * NQP];
+  __shared__ int fsl[EPB * 2 * ND];
   const int t = threadIdx.x, el = t / NQ, q = t % NQ;
+  const int n = m.n_elem[cls];
   const int e = blockIdx.x * EPB + el;
-  const bool valid = e < m.n_elem[cls];
-  double* st = m.state[cls] + size_t(e) * NV * NQ;
+  const bool valid = e < n;
+  double* st = m.state[cls] + size_t(valid ? e : n - 1) * NV * NQ;
+  const int slot = staged_slot<ND, RS>(m, cls, blockIdx.x, t);
   double u[NV];
-  for (int v = 0; v < NV; ++v) u[v] = valid ? st[v * NQ + q] : 0.;
+  for (int v = 0; v < NV; ++v) u[v] = st[v * NQ + q];
+  if (t < EPB * 2 * ND) fsl[t] = slot;
   if (scale_velocity && valid) {
     const double scale = sqrt(2 * u[ND] * u[ND + 1]);
     for (int d = 0; d < ND; ++d) st[d * NQ + q] = u[d] = scale_velocity == 1 ? u[d] / scale : u[d] * scale;
   }
   for (int v = 0; v < NV; ++v) su[el * NV * NQP + v * NQP + S::pad(q)] = u[v];
   __syncthreads();
-  write_faces_from<ND, RS, S::BLOCK>(m, cls, blockIdx.x, o, su, NV * NQP);
+  write_faces_to<ND, RS, S::BLOCK, NV>(m, cls, blockIdx.x, o, su, NV * NQP, [&](int el2) { return fsl + el2 * 2 * ND; });
 }
 
 // ---- Neighbor_reconcile (Spatial.hpp:716-759) ------------------------------------------------------------
@@ -1604,40 +1607,34 @@ __global__ __launch_bounds__(256) void k_neighbor_reconcile_mortar(Dev_mesh m)
   if (i < m.n_mortar_con[cls]) neighbor_reconcile_con<ND, RS, DEF, ND + 2>(m, m.mortar_con[cls][i], f);
 }
 
-// Neighbor_reconcile folded into Reconcile_ldg_flux: the reconciled viscous-flux jump of face point p of face `face`
-// of element e, this side's value of what Neighbor_reconcile writes (the same operations on the two sides' LDG blocks,
-// in the connection's side order), from the partner table (Dev_mesh::partner). A face whose partner is -1 (hanging
-// faces) reads the jump a launch before wrote into its own slot.
+// Neighbor_reconcile folded into Reconcile_ldg_flux: the reconciled viscous-flux jump of face point p of the face with
+// table entry r, this side's value of what Neighbor_reconcile writes (the same operations on the two sides' LDG blocks,
+// in the connection's side order). A face whose partner is -1 (hanging faces) takes the jump a launch before wrote into
+// its own slot. Branch-free, as face_in.
 template <int ND, int RS>
-__device__ __forceinline__ void ldg_jump(const Dev_mesh& m, int cls, int e, int face, int p, double (&out)[ND + 2])
+__device__ __forceinline__ void ldg_jump(const Dev_mesh& m, const Face_ref& r, int p, double (&out)[ND + 2])
 {
   constexpr int NFQ = Shape<ND, RS>::NFQ, NV = ND + 2;
-  const size_t k = size_t(e) * 2 * ND + face;
-  const int* pi = m.partner[cls] + 4 * k;
-  const double* own = slot_ptr(m, m.face_slot[cls][k]) + NV * NFQ;
-  const int ps = pi[0];
-  if (ps < 0) {
-    for (int v = 0; v < NV; ++v) out[v] = own[v * NFQ + p];
-    return;
-  }
-  const int info = pi[1];
+  const bool pre = r.ps < 0;
+  const int info = pre ? 0 : r.info;
   const Dir dir(info & 63);
   const bool side1 = (info >> 6) & 1, def = (info >> 7) & 1;
-  int fp = p;
-  double sg0 = 1., sg1 = 1.;
-  if (def) {
-    fp = side1 ? face0_index<ND, RS>(dir, p) : face1_index<ND, RS>(dir, p);
-    sg0 = 1 - 2 * int(dir.flip_normal(0));
-    sg1 = 1 - 2 * int(dir.flip_normal(1));
-  }
-  const double* par = slot_ptr(m, ps) + NV * NFQ;
+  int fp = side1 ? face0_index<ND, RS>(dir, p) : face1_index<ND, RS>(dir, p);
+  fp = def ? fp : p;
+  const double sg0 = def ? 1 - 2 * int(dir.flip_normal(0)) : 1, sg1 = def ? 1 - 2 * int(dir.flip_normal(1)) : 1;
+  const double* own = slot_ptr(m, r.own) + NV * NFQ;
+  const double* par = slot_ptr(m, pre ? r.own : r.ps) + NV * NFQ;
+  double ao[NV], ap[NV];
   for (int v = 0; v < NV; ++v) {
-    const double ao = own[v * NFQ + p], ap = par[v * NFQ + fp];
-    const double a0 = side1 ? ap : ao, a1 = side1 ? ao : ap;
+    ao[v] = own[v * NFQ + p];
+    ap[v] = par[v * NFQ + fp];
+  }
+  for (int v = 0; v < NV; ++v) {
+    const double a0 = side1 ? ap[v] : ao[v], a1 = side1 ? ao[v] : ap[v];
     double avg = 0;
     avg += .5 * sg0 * a0;
     avg += .5 * sg1 * a1;
-    out[v] = side1 ? sg1 * avg - a1 : sg0 * avg - a0;
+    out[v] = pre ? ao[v] : side1 ? sg1 * avg - a1 : sg0 * avg - a0;
   }
 }
 
