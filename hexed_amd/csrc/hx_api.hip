@@ -18,13 +18,16 @@
 using namespace hx;
 
 // Scratch memory of hx_update_no_alloc, for callers that cannot allocate device memory: [0, 32) holds the reduction
-// scalar of the time step, [32, 32 + no_alloc_max_blocks) one fused Max_dt minimum per Euler Local workgroup (a mesh
+// words and the time step, [32, 32 + no_alloc_max_blocks) one fused Max_dt minimum per Euler Local workgroup (a mesh
 // of up to 262,144 workgroups: 262,144 elements at 3D row size 5 to 8). Each GPU holds its own copy (2 MiB) until the
 // process ends. Host code uses the address hipGetSymbolAddress returns for the current device (hx_ctx::scratch), never
 // the array's name.
 namespace {
 constexpr long long no_alloc_max_blocks = 1LL << 18;
 constexpr long long scratch_minima_offset = 32;
+constexpr int scratch_step_offset = 8 + dt_final_blocks;  // the step's Step_dev, after the reduction words
+static_assert(scratch_step_offset + sizeof(Step_dev) / sizeof(double) <= scratch_minima_offset, "the words fit");
+constexpr int ctx_words = 8 + dt_final_blocks;
 }  // namespace
 static __device__ __align__(256) double scratch[scratch_minima_offset + no_alloc_max_blocks];
 
@@ -69,9 +72,13 @@ struct hx_ctx
   std::string err;
   void* ops[HX_MAX_ROW_SIZE + 1] = {};  // device Ops<rs> tables
   std::vector<char> host_ops[HX_MAX_ROW_SIZE + 1];  // host copies, for kernels taking constants by value
+  std::vector<char> host_eops[HX_MAX_ROW_SIZE + 1];
   void* eops[HX_MAX_ROW_SIZE + 1] = {};             // device Eops<rs, double> tables
-  double* scalar = nullptr;             // device scratch for reductions
-  double* host_scalar = nullptr;        // pinned host memory the per-step reductions are read back into
+  double* scalar = nullptr;             // device words for reductions (ctx_words of them, Dt_final::scalar)
+  // pinned host memory: [0..4) readbacks, [4] the time step and [5] its sequence number (Dt_final::host), [6] the two flags
+  // of the admissibility check
+  double* host_scalar = nullptr;
+  unsigned long long dt_seq = 0;        // sequence number of the last time step sent to host_scalar
   // per-category event timing
   struct Pending
   {
@@ -93,15 +100,6 @@ struct hx_ctx
   bool events_off = false;       // no per-launch events (a graph capture, or a call that may not create any)
   double* scratch = nullptr;     // this device's address of the file-scope scratch array (hx_update_no_alloc)
   hipError_t scratch_err = hipSuccess;
-};
-
-// status of the updates enqueued by hx_update_async, kept on the device
-struct Step_dev
-{
-  double dt;          // the time step the stage kernels of the current step read
-  double time_step;   // hx_update_status::time_step
-  double flow_time;   // hx_update_status::flow_time
-  long long iteration;
 };
 
 struct hx_mesh
@@ -127,7 +125,7 @@ struct hx_mesh
   double* dt_block_min = nullptr;  // one minimum per workgroup of the Euler Local, both classes
   long long n_dt_blocks = 0;
   Dt_fuse fuse{};                  // the fusion the next Euler Local launch performs (block_min == nullptr: none)
-  int* admis_flags = nullptr;      // [2] results of the admissibility check (hx_is_admissible)
+  Dt_final dtf{};                  // the time step the next state_bcs launch forms (blocks == 0: none)
   struct
   {
     bool valid = false;
@@ -151,6 +149,7 @@ struct hx_mesh
   // hx_update_async: the device status, the time step the stage kernels read while an update is enqueued with it
   // (null otherwise), and the captured steady-state update with the options and form it was captured for
   Step_dev* step = nullptr;
+  Step_dev* sync_step = nullptr;   // hx_update's own, of which it uses dt only
   const double* dt_dev = nullptr;
   // the reduction scalar the mesh's calls use: the context's, or the file-scope scratch array during
   // hx_update_no_alloc; and the scratch epoch of the last hx_update_no_alloc on this mesh (its fused minima sit in the
@@ -248,8 +247,8 @@ void release_mesh_memory(hx_mesh* mesh)
   mesh->case_min = nullptr;
   mesh->case_dt = nullptr;
   mesh->dt_block_min = nullptr;
-  mesh->admis_flags = nullptr;
-  mesh->step = nullptr;
+  mesh->step = mesh->sync_step = nullptr;
+  mesh->dtf = Dt_final{};
   mesh->dt_dev = nullptr;
   mesh->fuse = Dt_fuse{};
   mesh->dt_cache.valid = mesh->case_cache.valid = false;
@@ -329,6 +328,8 @@ hx_status upload_ops(hx_ctx* ctx, void** out)
   const Eops<RS, double> e = make_eops<RS, double>(o);
   HX_TRY(ctx, hipMalloc(&ctx->eops[RS], sizeof(e)), "hipMalloc(eops)");
   HX_TRY(ctx, hipMemcpy(ctx->eops[RS], &e, sizeof(e), hipMemcpyHostToDevice), "hipMemcpy(eops)");
+  const char* eb = reinterpret_cast<const char*>(&e);
+  ctx->host_eops[RS].assign(eb, eb + sizeof(e));
   return HX_OK;
 }
 
@@ -546,9 +547,11 @@ Launch make_launch(hx_mesh* mesh, bool writes = true)
   l.ops = mesh->ctx->ops[mesh->dm.rs];
   l.hops = mesh->ctx->host_ops[mesh->dm.rs].data();
   l.eops = mesh->ctx->eops[mesh->dm.rs];
+  l.heops = mesh->ctx->host_eops[mesh->dm.rs].data();
   l.scalar = mesh->scalar ? mesh->scalar : mesh->ctx->scalar;
   l.precision = mesh->precision;
   l.fuse = mesh->fuse;
+  l.dtf = mesh->dtf;
   l.dtp = mesh->dt_dev;
   l.fold = mesh->fold;
   l.m.alt_rd = mesh->alt_rd;
@@ -660,20 +663,6 @@ void resolve_timing(hx_ctx* ctx)
 
 __global__ void k_fill(double* p, double v) { p[threadIdx.x] = v; }
 
-// one step's time step on the device, min(Max_dt, max_time_step) * chebyshev_step (Solver.cpp:843-848), with
-// Max_dt from *mdt (or 1 with local time stepping), and the status it advances (Solver.cpp:872-876)
-__global__ void k_step_dt(const double* mdt, int unit, double max_time_step, double cheby, Step_dev* s, int count)
-{
-  const double m = unit ? 1. : *mdt;
-  double dt = (max_time_step < m ? max_time_step : m) * cheby;
-  // the product is rounded before it is accumulated, as the host's flow_time += dt does (no fused multiply-add)
-  asm volatile("" : "+v"(dt));
-  s->dt = dt;
-  s->time_step = dt;
-  s->flow_time += dt;
-  if (count) ++s->iteration;
-}
-
 __global__ void k_set_status(Step_dev* s, double time_step, double flow_time, long long iteration)
 {
   s->dt = time_step;
@@ -728,24 +717,6 @@ __global__ __launch_bounds__(256) void k_fill_u64(unsigned long long* p, unsigne
 {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i < n) p[i] = v;
-}
-
-// minimum of v[0..n) by atomic minimum into *out (prefilled with DBL_MAX), one atomic per workgroup
-__global__ __launch_bounds__(256) void k_min_reduce(const double* __restrict__ v, long long n, double* out)
-{
-  __shared__ double w[4];
-  double m = DBL_MAX;
-  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) m = v[i] < m ? v[i] : m;
-  for (int off = 32; off > 0; off /= 2) {
-    const double x = __shfl_xor(m, off, 64);
-    m = x < m ? x : m;
-  }
-  if ((threadIdx.x & 63) == 0) w[threadIdx.x / 64] = m;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int k = 1; k < 4; ++k) m = w[k] < m ? w[k] : m;
-    if (m < DBL_MAX) atomicMin(reinterpret_cast<unsigned long long*>(out), (unsigned long long)__double_as_longlong(m));
-  }
 }
 
 // plain streaming copy: each workgroup moves chunks of 4 x 256 16-byte items, every lane with its four loads in flight
@@ -893,12 +864,14 @@ hx_status hx_ctx_create(int device, hx_ctx** out)
   auto* ctx = new hx_ctx;
   ctx->device = device;
   if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess ||
-      hipMalloc(&ctx->scalar, 8 * sizeof(double)) != hipSuccess ||
-      hipHostMalloc(&ctx->host_scalar, 8 * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+      hipMalloc(&ctx->scalar, ctx_words * sizeof(double)) != hipSuccess ||
+      hipMemset(ctx->scalar, 0, ctx_words * sizeof(double)) != hipSuccess ||
+      hipHostMalloc(&ctx->host_scalar, 8 * sizeof(double), hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
     if (ctx->scalar) (void)hipFree(ctx->scalar);
     delete ctx;
     return HX_ERR_HIP;
   }
+  std::memset(ctx->host_scalar, 0, 8 * sizeof(double));
   // the scratch array of hx_update_no_alloc, with this device current; a failure is reported by that entry point
   ctx->scratch = scratch_on(device, &ctx->scratch_err);
   *out = ctx;
@@ -1311,8 +1284,12 @@ hx_status hx_max_dt(hx_mesh* mesh, int cls, const hx_pde* pde, int is_local, int
   if (hx_status s = pde_check(mesh, pde, &visc, &l)) return s;
   const double max_cfl_c = hx_basis_max_cfl(mesh->dm.rs) * safety_conv;
   const double max_cfl_d = -2 / hx_basis_tables::eigenvalss[mesh->dm.rs - 2][1] * safety_diff;
-  hipLaunchKernelGGL(k_fill, dim3(1), dim3(1), 0, l.stream, l.scalar, DBL_MAX);
-  HX_TRY(mesh->ctx, hipGetLastError(), "fill");
+  *dt_out = is_local ? 1. : DBL_MAX;
+  if (!mesh->dm.n_elem[cls]) return HX_OK;
+  if (!is_local) {
+    hipLaunchKernelGGL(k_fill, dim3(1), dim3(1), 0, l.stream, l.scalar, DBL_MAX);
+    HX_TRY(mesh->ctx, hipGetLastError(), "fill");
+  }
   {
     Timer tm(mesh->ctx, std::string(cls_name(cls)) + "/compute time step/" + pde_name(pde), mesh->dm.n_elem[cls]);
     // Smooth_art_visc and Fix_therm_admis share Max_dt's diffusivity-1 form (pde.hpp:412-416, 486-490)
@@ -1321,11 +1298,12 @@ hx_status hx_max_dt(hx_mesh* mesh, int cls, const hx_pde* pde, int is_local, int
              "max_dt");
     else HX_TRY(mesh->ctx, mesh->ks->max_dt(l, cls, visc, is_local, max_cfl_c, max_cfl_d), "max_dt");
   }
+  // with local time stepping the result is 1 whatever the device holds: nothing to wait for
+  if (is_local) return HX_OK;
   HX_TRY(mesh->ctx, hipMemcpyAsync(mesh->ctx->host_scalar, l.scalar, sizeof(double), hipMemcpyDeviceToHost, l.stream),
          "max_dt readback");
   HX_TRY(mesh->ctx, hipStreamSynchronize(l.stream), "max_dt sync");
-  const double dt = *mesh->ctx->host_scalar;
-  *dt_out = is_local ? 1. : dt;
+  *dt_out = *mesh->ctx->host_scalar;
   return HX_OK;
 }
 
@@ -1488,7 +1466,8 @@ struct Update_setup
   double* block_min; // the fused per-workgroup minima: the mesh's buffer, or the scratch array
   long long n_blocks;
   bool in_scratch;
-  double* scalar;    // the reduction scalar
+  double* scalar;    // the reduction words (Dt_final::scalar)
+  Step_dev* step;    // where the time step is formed on the device
 };
 
 // workgroups of the Euler Local over both classes, each storing one fused minimum
@@ -1498,8 +1477,10 @@ long long euler_local_blocks(const hx_mesh* mesh)
   return (mesh->dm.n_elem[0] + epb - 1) / epb + (mesh->dm.n_elem[1] + epb - 1) / epb;
 }
 
-// no_alloc: the minima and the reduction scalar go to the file-scope scratch array, and nothing is allocated
-hx_status update_setup(hx_mesh* mesh, const hx_update_options* o, Update_setup* u, bool no_alloc = false)
+// no_alloc: the minima, the reduction words and the time step go to the file-scope scratch array, and nothing is
+// allocated; `async`: the time step and the status it advances are those of hx_update_async
+hx_status update_setup(hx_mesh* mesh, const hx_update_options* o, Update_setup* u, bool no_alloc = false,
+                       bool async = false)
 {
   hx_ctx* ctx = mesh->ctx;
   // the state that stage 1's Local writes is the state that Max_dt would read next; local time stepping writes the
@@ -1513,7 +1494,18 @@ hx_status update_setup(hx_mesh* mesh, const hx_update_options* o, Update_setup* 
                                            " Euler Local workgroups, at most " + std::to_string(no_alloc_max_blocks));
     u->block_min = ctx->scratch + scratch_minima_offset;
     u->scalar = ctx->scratch;
+    u->step = reinterpret_cast<Step_dev*>(ctx->scratch + scratch_step_offset);
   } else {
+    Step_dev*& step = async ? mesh->step : mesh->sync_step;
+    if (!step) {
+      void* p = nullptr;
+      HX_TRY(ctx, hipMalloc(&p, sizeof(Step_dev)), "hipMalloc(update status)");
+      mesh->allocs.push_back(p);
+      step = static_cast<Step_dev*>(p);
+      hipLaunchKernelGGL(k_set_status, dim3(1), dim3(1), 0, ctx->stream, step, 0., 0., 0LL);
+      HX_TRY(ctx, hipGetLastError(), "status");
+    }
+    u->step = step;
     if (u->fusable && !mesh->dt_block_min) {
       mesh->n_dt_blocks = u->n_blocks;
       void* p = nullptr;
@@ -1564,14 +1556,17 @@ void remember_fused(hx_mesh* mesh, const hx_update_options* o, const Update_setu
   c.in_scratch = u.in_scratch;
 }
 
-// Max_dt of both classes into the context's reduction scalar, without reading it back (kernels_max_dt.cpp:8-17)
+// Max_dt of both classes into the reduction words, without reading it back (kernels_max_dt.cpp:8-17); with local time
+// stepping only the time step scale, which needs no reduction
 hx_status enqueue_max_dt(hx_mesh* mesh, const hx_update_options* o, const Update_setup& u)
 {
   hx_ctx* ctx = mesh->ctx;
   const double max_cfl_c = hx_basis_max_cfl(mesh->dm.rs) * u.msc;
   const double max_cfl_d = -2 / hx_basis_tables::eigenvalss[mesh->dm.rs - 2][1] * u.msd;
-  hipLaunchKernelGGL(k_fill, dim3(1), dim3(1), 0, ctx->stream, u.scalar, DBL_MAX);
-  HX_TRY(ctx, hipGetLastError(), "fill");
+  if (!o->local_time) {
+    hipLaunchKernelGGL(k_fill, dim3(1), dim3(1), 0, ctx->stream, u.scalar, DBL_MAX);
+    HX_TRY(ctx, hipGetLastError(), "fill");
+  }
   for (int cls = 0; cls < 2; ++cls) {
     Launch l = make_launch(mesh);
     l.ns = u.ns;
@@ -1581,15 +1576,23 @@ hx_status enqueue_max_dt(hx_mesh* mesh, const hx_update_options* o, const Update
   return HX_OK;
 }
 
-// the fused minima of the previous stage 1 reduced into the context's reduction scalar
-hx_status enqueue_fused_reduce(hx_mesh* mesh, const Update_setup& u)
+// Waits for the time step with sequence number `seq` that a launch of this context sends to the pinned host words
+// (Dt_final::host): it arrives while the stage kernels queued behind it run. Ends with an error if the stream drains, or
+// fails, without it.
+hx_status wait_dt(hx_ctx* ctx, unsigned long long seq, double* dt)
 {
-  hx_ctx* ctx = mesh->ctx;
-  Timer tm(ctx, "fused/compute time step/reduce", u.n_blocks);
-  hipLaunchKernelGGL(k_fill, dim3(1), dim3(1), 0, ctx->stream, u.scalar, DBL_MAX);
-  const unsigned g = unsigned(std::min<long long>(256, (u.n_blocks + 255) / 256));
-  if (g) hipLaunchKernelGGL(k_min_reduce, dim3(g), dim3(256), 0, ctx->stream, u.block_min, u.n_blocks, u.scalar);
-  HX_TRY(ctx, hipGetLastError(), "time step reduction");
+  const auto* arrived = reinterpret_cast<const unsigned long long*>(ctx->host_scalar + 5);
+  for (unsigned spin = 1; __atomic_load_n(arrived, __ATOMIC_ACQUIRE) != seq; ++spin) {
+    if (spin % 1024) {
+      __builtin_ia32_pause();
+      continue;
+    }
+    const hipError_t e = hipStreamQuery(ctx->stream);
+    if (e == hipErrorNotReady) continue;
+    HX_TRY(ctx, e, "time step");
+    if (__atomic_load_n(arrived, __ATOMIC_ACQUIRE) != seq) return fail(ctx, HX_ERR_HIP, "the time step did not arrive");
+  }
+  *dt = ctx->host_scalar[4];
   return HX_OK;
 }
 
@@ -1615,88 +1618,96 @@ struct Stage_fold
   ~Stage_fold() { mesh->fold = mesh->alt_rd = mesh->alt_wr = 0; }
 };
 
+// sets the time step the stage kernels read from the device (null: their coefficient holds it) for a scope
+struct Device_dt
+{
+  hx_mesh* mesh;
+  Device_dt(hx_mesh* m, const double* dt) : mesh{m} { mesh->dt_dev = dt; }
+  ~Device_dt() { mesh->dt_dev = nullptr; }
+};
+
 // The kernels of one Solver::update (Solver.cpp:834-886), with fix_admissibility after each stage when enabled
-// (Solver.cpp:867). Host form (st not null): each step's Max_dt is read back and the time step passed by value.
-// Device form (st null): the time step stays in mesh->step, formed by k_step_dt, and the stage kernels read it; nothing
-// here waits for the device. `pending`: the previous stage 1's fused Max_dt minima hold the current state's.
+// (Solver.cpp:867). The time step is formed on the device, beside stage 0's boundary conditions, and read there by the
+// stage kernels. Host form (st not null): it also goes to pinned host memory, and the host picks it up once the stage
+// kernels are queued, so that the device never waits for the host (with local time stepping it is 1, up to the maximum,
+// and the host needs nothing). Device form (st null): nothing here waits for the device. `pending`: the previous stage 1's
+// fused Max_dt minima hold the current state's.
 hx_status update_once(hx_mesh* mesh, const hx_update_options* o, const Update_setup& u, hx_update_status* st, bool& pending)
 {
   hx_ctx* ctx = mesh->ctx;
-  const bool device_dt = st == nullptr;
+  const bool device_form = st == nullptr, device_dt = device_form || !o->local_time;
   for (int i_flow = 0; i_flow < o->flow_iters; ++i_flow) {
     for (int i_cheby = 0; i_cheby < u.n_cheby; ++i_cheby) {
       hx_status s;
-      double dt = 1.;
-      if (pending) {
-        if ((s = enqueue_fused_reduce(mesh, u))) return s;
-      } else if (device_dt) {
+      const double cheby = cheby_step(u.n_cheby, i_cheby);
+      double dt = device_dt ? 1. : std::min(1., o->max_time_step) * cheby;
+      if (!pending)
         if ((s = enqueue_max_dt(mesh, o, u))) return s;
-      } else {
-        hx_kernel_options ko{0., 0, 0, o->use_filter};
-        double mdt;
-        s = o->use_ldg ? hx_max_dt_navier_stokes(mesh, &ko, u.msc, u.msd, o->local_time, o->visc, o->cond, &mdt)
-                       : hx_max_dt_euler(mesh, &ko, u.msc, u.msd, o->local_time, &mdt);
-        if (s) return s;
-        dt = std::min(mdt, o->max_time_step) * cheby_step(u.n_cheby, i_cheby);
-      }
+      Dt_final f{};
       if (device_dt) {
-        hipLaunchKernelGGL(k_step_dt, dim3(1), dim3(1), 0, ctx->stream, u.scalar, pending ? 0 : o->local_time,
-                           o->max_time_step, cheby_step(u.n_cheby, i_cheby), mesh->step, int(i_flow == 0 && i_cheby == 0));
-        HX_TRY(ctx, hipGetLastError(), "time step");
-      } else if (pending) {
-        HX_TRY(ctx, hipMemcpyAsync(ctx->host_scalar, u.scalar, sizeof(double), hipMemcpyDeviceToHost, ctx->stream),
-               "max_dt readback");
-        HX_TRY(ctx, hipStreamSynchronize(ctx->stream), "max_dt sync");
-        dt = std::min(*ctx->host_scalar, o->max_time_step) * cheby_step(u.n_cheby, i_cheby);
+        f.v = pending ? u.block_min : u.scalar;
+        f.n = o->local_time ? 0 : pending ? u.n_blocks : 1;
+        f.blocks = dt_blocks_for(f.n);
+        f.scalar = u.scalar;
+        f.unit = o->local_time;
+        f.max_time_step = o->max_time_step;
+        f.cheby = cheby;
+        f.step = u.step;
+        f.accumulate = device_form;
+        f.count = i_flow == 0 && i_cheby == 0;
+        if (!device_form) {
+          f.host = ctx->host_scalar + 4;
+          f.seq = ++ctx->dt_seq;
+        }
       }
       bool fixed = false;
-      for (int i = 0; i < 2; ++i) {
-        hx_kernel_options opts{dt, i, 0, o->use_filter};
-        // face-flux folding (not with the admissibility fix, which reads the faces between the stages): stage 0 reads
-        // the face states from the primary buffer and extrapolates into the second, stage 1 the other way round, so
-        // that an update leaves the faces where the reference's sequence leaves them
-        Stage_fold sf(mesh, !o->fix_admis && folds_faces(mesh), i);
-        if ((s = hx_apply_state_bcs(mesh))) return s;
-        if (o->use_ldg && !i) {
-          s = hx_compute_navier_stokes(mesh, &opts, o->visc, o->cond);
-        } else {
-          if (i == 1 && u.fusable)
-            mesh->fuse = Dt_fuse{u.block_min, 0, o->use_ldg ? 1 : 0, hx_basis_max_cfl(mesh->dm.rs) * u.msc,
-                                 -2 / hx_basis_tables::eigenvalss[mesh->dm.rs - 2][1] * u.msd, u.ns};
-          s = hx_compute_euler(mesh, &opts);
-          mesh->fuse = Dt_fuse{};
-        }
-        if (s) return s;
-        if (o->fix_admis) {
-          int iters = 0;
-          if ((s = hx_fix_admissibility(mesh, o, o->fix_admis_max_safety, &iters))) return s;
-          st->fix_admis_iters += iters;
-          fixed = iters || fixed;
+      {
+        Device_dt in_use(mesh, device_dt ? &u.step->dt : nullptr);
+        for (int i = 0; i < 2; ++i) {
+          hx_kernel_options opts{dt, i, 0, o->use_filter};
+          // face-flux folding (not with the admissibility fix, which reads the faces between the stages): stage 0 reads
+          // the face states from the primary buffer and extrapolates into the second, stage 1 the other way round, so
+          // that an update leaves the faces where the reference's sequence leaves them
+          Stage_fold sf(mesh, !o->fix_admis && folds_faces(mesh), i);
+          if (i == 0) mesh->dtf = f;
+          s = hx_apply_state_bcs(mesh);
+          mesh->dtf = Dt_final{};
+          if (s) return s;
+          if (o->use_ldg && !i) {
+            s = hx_compute_navier_stokes(mesh, &opts, o->visc, o->cond);
+          } else {
+            if (i == 1 && u.fusable)
+              mesh->fuse = Dt_fuse{u.block_min, 0, o->use_ldg ? 1 : 0, hx_basis_max_cfl(mesh->dm.rs) * u.msc,
+                                   -2 / hx_basis_tables::eigenvalss[mesh->dm.rs - 2][1] * u.msd, u.ns};
+            s = hx_compute_euler(mesh, &opts);
+            mesh->fuse = Dt_fuse{};
+          }
+          if (s) return s;
+          if (o->fix_admis) {
+            int iters = 0;
+            if ((s = hx_fix_admissibility(mesh, o, o->fix_admis_max_safety, &iters))) return s;
+            st->fix_admis_iters += iters;
+            fixed = iters || fixed;
+          }
         }
       }
+      if (f.host)
+        if ((s = wait_dt(ctx, f.seq, &dt))) return s;
       // a fix changed the state after the fused Max_dt read it, and ends this Chebyshev sequence (Solver.cpp:869)
       if (fixed) {
         pending = false;
         break;
       }
       pending = u.fusable;
-      if (!device_dt) {
+      if (!device_form) {
         st->time_step = dt;
         st->flow_time += dt;
       }
     }
   }
-  if (!device_dt) ++st->iteration;
+  if (!device_form) ++st->iteration;
   return HX_OK;
 }
-
-// sets mesh->dt_dev for the duration of a device-form update
-struct Device_dt
-{
-  hx_mesh* mesh;
-  Device_dt(hx_mesh* m) : mesh{m} { mesh->dt_dev = &mesh->step->dt; }
-  ~Device_dt() { mesh->dt_dev = nullptr; }
-};
 
 // the steady-state update (the fused minima pending when it starts, or local time stepping) captured into a graph
 hx_status capture_update(hx_mesh* mesh, const hx_update_options* o, const Update_setup& u)
@@ -1706,11 +1717,7 @@ hx_status capture_update(hx_mesh* mesh, const hx_update_options* o, const Update
   HX_TRY(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
   ctx->events_off = true;
   bool pending = u.fusable;
-  hx_status s;
-  {
-    Device_dt d(mesh);
-    s = update_once(mesh, o, u, nullptr, pending);
-  }
+  const hx_status s = update_once(mesh, o, u, nullptr, pending);
   ctx->events_off = false;
   hipGraph_t g = nullptr;
   const hipError_t e = hipStreamEndCapture(ctx->stream, &g);
@@ -1752,15 +1759,7 @@ hx_status hx_update_async(hx_mesh* mesh, const hx_update_options* o, int n_updat
     return fail(ctx, HX_ERR_UNSUPPORTED, "the admissibility fix reads its verdict on the host; use hx_update");
   if (mesh->n_cases) return fail(ctx, HX_ERR_INVALID, "the mesh holds a batch of cases; use hx_update_cases");
   Update_setup u;
-  if (hx_status s = update_setup(mesh, o, &u)) return s;
-  if (!mesh->step) {
-    void* p = nullptr;
-    HX_TRY(ctx, hipMalloc(&p, sizeof(Step_dev)), "hipMalloc(update status)");
-    mesh->allocs.push_back(p);
-    mesh->step = static_cast<Step_dev*>(p);
-    hipLaunchKernelGGL(k_set_status, dim3(1), dim3(1), 0, ctx->stream, mesh->step, 0., 0., 0LL);
-    HX_TRY(ctx, hipGetLastError(), "status");
-  }
+  if (hx_status s = update_setup(mesh, o, &u, false, true)) return s;
   if (from) {
     hipLaunchKernelGGL(k_set_status, dim3(1), dim3(1), 0, ctx->stream, mesh->step, from->time_step, from->flow_time,
                        (long long)from->iteration);
@@ -1771,7 +1770,6 @@ hx_status hx_update_async(hx_mesh* mesh, const hx_update_options* o, int n_updat
   for (int k = 0; k < n_updates; ++k) {
     if (u.fusable && !pending) {
       // the first update of a sequence computes Max_dt itself; every later one starts from the fused minima
-      Device_dt d(mesh);
       if (hx_status s = update_once(mesh, o, u, nullptr, pending)) return s;
       continue;
     }
@@ -2678,8 +2676,8 @@ hx_status share_vertices(hx_mesh* mesh, double* vert, bool maximum)
 }
 
 // Stab_art_visc (stabilizing_art_visc.cpp:8-61) over both classes into a device array [n_tot][2^nd] (each element's
-// value in all its vertex slots), and the element values copied to `uncert` when it is not null
-hx_status stab_into(hx_mesh* mesh, double char_speed, double* vert, double* uncert)
+// value in all its vertex slots), and with `values` the element values into the mesh's work array
+hx_status stab_into(hx_mesh* mesh, double char_speed, double* vert, bool values)
 {
   hx_ctx* ctx = mesh->ctx;
   const Dev_mesh& dm = mesh->dm;
@@ -2690,16 +2688,26 @@ hx_status stab_into(hx_mesh* mesh, double char_speed, double* vert, double* unce
     Timer tm(ctx, std::string(cls_name(cls)) + "/stabilizing art visc/indicator", dm.n_elem[cls]);
     HX_TRY(ctx, mesh->ks->stab_indicator(l, cls, char_speed, vert), "stab_art_visc");
   }
-  if (uncert && n_tot) {
+  if (values && n_tot) {
     // each element's value is in all its vertex slots: the first slot of each, gathered on the device
     double* elem = mesh->vc.elem;
     hipLaunchKernelGGL(k_gather_stride, dim3(unsigned((n_tot + 255) / 256)), dim3(256), 0, ctx->stream, vert, nvert,
                        n_tot, elem);
     HX_TRY(ctx, hipGetLastError(), "element values");
-    HX_TRY(ctx, hipMemcpyAsync(uncert, elem, size_t(n_tot) * sizeof(double), hipMemcpyDeviceToHost, ctx->stream),
-           "element values readback");
-    HX_TRY(ctx, hipStreamSynchronize(ctx->stream), "stab_art_visc sync");
   }
+  return HX_OK;
+}
+
+// the element values that stab_into left in the mesh's work array copied to the host, when the stream reaches this; ends
+// synchronized
+hx_status stab_readback(hx_mesh* mesh, double* uncert)
+{
+  hx_ctx* ctx = mesh->ctx;
+  const long long n_tot = (long long)mesh->dm.n_elem[0] + mesh->dm.n_elem[1];
+  if (uncert && n_tot)
+    HX_TRY(ctx, hipMemcpyAsync(uncert, mesh->vc.elem, size_t(n_tot) * sizeof(double), hipMemcpyDeviceToHost, ctx->stream),
+           "element values readback");
+  HX_TRY(ctx, hipStreamSynchronize(ctx->stream), "stab_art_visc sync");
   return HX_OK;
 }
 
@@ -2765,7 +2773,8 @@ hx_status hx_stab_art_visc(hx_mesh* mesh, double char_speed, double* uncert)
   const long long n_tot = (long long)mesh->dm.n_elem[0] + mesh->dm.n_elem[1];
   HX_TRY(mesh->ctx, vc_buffer(&vc.vert, size_t(n_tot) << mesh->dm.nd, false), "hipMalloc(vertex values)");
   HX_TRY(mesh->ctx, vc_buffer(&vc.elem, size_t(n_tot), false), "hipMalloc(element values)");
-  return stab_into(mesh, char_speed, vc.vert, uncert);
+  if (hx_status s = stab_into(mesh, char_speed, vc.vert, true)) return s;
+  return stab_readback(mesh, uncert);
 }
 
 hx_status hx_set_art_visc_admis(hx_mesh* mesh, const hx_vertex_data* v, double char_speed, double* uncert)
@@ -2778,7 +2787,7 @@ hx_status hx_set_art_visc_admis(hx_mesh* mesh, const hx_vertex_data* v, double c
   if (hx_status s = sync_vertices(mesh, v)) return s;
   const long long n_tot = (long long)dm.n_elem[0] + dm.n_elem[1];
   double* vert = mesh->vc.vert;
-  if (hx_status s = stab_into(mesh, char_speed, vert, uncert)) return s;
+  if (hx_status s = stab_into(mesh, char_speed, vert, uncert != nullptr)) return s;
   {
     Timer tm(ctx, "stabilizing art visc/vertices", n_tot);
     if (hx_status s = share_vertices(mesh, vert, true)) return s;
@@ -2788,8 +2797,7 @@ hx_status hx_set_art_visc_admis(hx_mesh* mesh, const hx_vertex_data* v, double c
     Timer tm(ctx, std::string(cls_name(cls)) + "/stabilizing art visc/interpolate", dm.n_elem[cls]);
     HX_TRY(ctx, mesh->ks->vertex_interp_lap(l, cls, vert), "vertex interpolation");
   }
-  HX_TRY(ctx, hipStreamSynchronize(ctx->stream), "set_art_visc_admis sync");
-  return HX_OK;
+  return stab_readback(mesh, uncert);
 }
 
 // compute_fix_therm_admis (kernels_diffusive.cpp:32): the COMPUTE_DIFFUSION sequence with pde::Fix_therm_admis; the
@@ -2839,22 +2847,14 @@ hx_status hx_is_admissible(hx_mesh* mesh, int* admissible)
   if (!live(mesh) || !admissible) return HX_ERR_INVALID;
   hx_ctx* ctx = mesh->ctx;
   // reads the fields only, so a fused Max_dt stays valid
-  if (!mesh->admis_flags) {
-    void* p = nullptr;
-    HX_TRY(ctx, hipMalloc(&p, 2 * sizeof(int)), "hipMalloc(admissibility flags)");
-    mesh->allocs.push_back(p);
-    mesh->admis_flags = static_cast<int*>(p);
-  }
+  // (every use of the flags ends with a wait for the stream, so no kernel writes them now)
+  int* const h = reinterpret_cast<int*>(ctx->host_scalar + 6);
+  h[0] = h[1] = 0;
   Launch l = make_launch(mesh, false);
-  hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(256), 0, ctx->stream, reinterpret_cast<unsigned long long*>(mesh->admis_flags),
-                     0ull, 1);
-  HX_TRY(ctx, hipGetLastError(), "fill");
   {
     Timer tm(ctx, "check admis.", (long long)mesh->dm.n_elem[0] + mesh->dm.n_elem[1]);
-    HX_TRY(ctx, mesh->ks->admissible(l, mesh->admis_flags), "is_admissible");
+    HX_TRY(ctx, mesh->ks->admissible(l, h), "is_admissible");
   }
-  int h[2] = {0, 0};
-  HX_TRY(ctx, hipMemcpyAsync(h, mesh->admis_flags, sizeof(h), hipMemcpyDeviceToHost, ctx->stream), "admissibility readback");
   HX_TRY(ctx, hipStreamSynchronize(ctx->stream), "admissibility sync");
   if (h[1]) return fail(ctx, HX_ERR_NOT_FINITE, "state is not finite");
   *admissible = !h[0];
@@ -3005,10 +3005,10 @@ hx_status hx_update_art_visc_smoothness(hx_mesh* mesh, const hx_av_options* o, d
   }
   if ((s = hx_compute_prolong(mesh, 0, 0))) return s;
   if (residual) {
-    double r = 0;
-    HX_TRY(ctx, hipMemcpyAsync(&r, resid_dev, sizeof(double), hipMemcpyDeviceToHost, l.stream), "residual readback");
+    HX_TRY(ctx, hipMemcpyAsync(ctx->host_scalar, resid_dev, sizeof(double), hipMemcpyDeviceToHost, l.stream),
+           "residual readback");
     HX_TRY(ctx, hipStreamSynchronize(l.stream), "residual sync");
-    *residual = std::sqrt(r);
+    *residual = std::sqrt(*ctx->host_scalar);
   }
   return HX_OK;
 }

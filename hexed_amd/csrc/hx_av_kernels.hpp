@@ -610,9 +610,11 @@ __global__ __launch_bounds__(256) void k_av_bcs(Dev_mesh m, int mode)
 
 // ---- Solver::is_admissible (Solver.cpp:921-959) with thermo::admissible (thermo.cpp:6-18) ----------------------
 // Density and energy must be positive at every quadrature point of the element and of its faces (state block);
-// flags[0] |= 1 when some element is not, flags[1] |= 1 when a checked value is not finite (the reference's "state is
-// not finite" assertion). Per element the reference stops at the first inadmissible array: the state, then the faces
+// flags[0] = 1 when some element is not, flags[1] = 1 when a checked value is not finite (the reference's "state is
+// not finite" assertion); both in pinned host memory. Per element the reference stops at the first inadmissible array: the state, then the faces
 // in order; a face after that one is not checked for finiteness.
+__device__ inline void raise_flag(int* f) { __hip_atomic_store(f, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
+
 template <int ND, int RS>
 __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_admissible(Dev_mesh m, int cls, int* flags)
 {
@@ -646,8 +648,8 @@ __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_admissible(Dev_mesh 
       if ((face_nonfinite[el] >> f) & 1) fin = false;
       if ((face_bad[el] >> f) & 1) admis = false;
     }
-    if (!admis) atomicOr(flags, 1);
-    if (!fin) atomicOr(flags + 1, 1);
+    if (!admis) raise_flag(flags);
+    if (!fin) raise_flag(flags + 1);
   }
 }
 
@@ -667,8 +669,8 @@ __global__ __launch_bounds__(256) void k_admissible_ref(Dev_mesh m, int* flags)
   const double* fc = slot_ptr(m, m.ref_slot[5 * i + 1 + f]);
   bool fin = true;
   for (int v = 0; v < NV; ++v) fin = fin && isfinite(fc[v * NFQ + p]);
-  if (!(fc[ND * NFQ + p] > 0.) || !(fc[(ND + 1) * NFQ + p] > 0.)) atomicOr(flags, 1);
-  if (!fin) atomicOr(flags + 1, 1);
+  if (!(fc[ND * NFQ + p] > 0.) || !(fc[(ND + 1) * NFQ + p] > 0.)) raise_flag(flags);
+  if (!fin) raise_flag(flags + 1);
 }
 
 // The artificial-viscosity swap around one iteration of Solver::fix_admissibility (Solver.cpp:1040-1047,

@@ -165,6 +165,79 @@ struct Dt_fuse
   double* point_scale[2];  // per class, each point's 1/scale (the batch's per-case time steps), or null
 };
 
+// The status of the updates whose time step stays on the device
+struct Step_dev
+{
+  double dt;          // the time step the stage kernels of the current step read
+  double time_step;   // hx_update_status::time_step
+  double flow_time;   // hx_update_status::flow_time
+  long long iteration;
+};
+
+// One step's time step, min(Max_dt, max_time_step) * chebyshev_step (Solver.cpp:843-848), with Max_dt the minimum of
+// v[0..n), formed by `blocks` workgroups (dt_final)
+struct Dt_final
+{
+  int blocks;               // 0: no time step to form
+  const double* v;
+  long long n;
+  double* scalar;           // reduction words: [0] the minimum, [2] workgroup counter (zero between launches), [8..) minima
+  int unit;                 // local time stepping: Max_dt is 1
+  double max_time_step, cheby;
+  Step_dev* step;           // receives dt; with `accumulate` also the status it advances (Solver.cpp:872-876)
+  int accumulate, count;    // count: the step starts an iteration
+  double* host;             // pinned memory receiving dt, then `seq` (as an integer) one word on; or null
+  unsigned long long seq;
+};
+constexpr int dt_final_blocks = 16;  // at most; the reduction words hold this many minima
+inline int dt_blocks_for(long long n) { return n <= 4096 ? 1 : dt_final_blocks; }
+
+// Workgroup b (256 threads) of the time step: each reduces its share, the last to arrive combines their minima. A NaN never
+// wins. One launch, usually shared with the state boundary conditions (k_state_bcs), where a fill, a reduction and a
+// one-thread kernel took three (13 us of a graph-replayed step).
+__device__ inline void dt_final(const Dt_final& f, int b)
+{
+  __shared__ double w[4];
+  double m = 1.7976931348623157e308;  // DBL_MAX
+  for (long long i = (long long)b * 256 + threadIdx.x; i < f.n; i += (long long)f.blocks * 256) {
+    const double x = f.v[i];
+    m = x < m ? x : m;
+  }
+  for (int off = 32; off > 0; off /= 2) {
+    const double x = __shfl_xor(m, off, 64);
+    m = x < m ? x : m;
+  }
+  if ((threadIdx.x & 63) == 0) w[threadIdx.x / 64] = m;
+  __syncthreads();
+  if (threadIdx.x) return;
+  for (int k = 1; k < 4; ++k) m = w[k] < m ? w[k] : m;
+  if (f.blocks > 1) {
+    unsigned* count = reinterpret_cast<unsigned*>(f.scalar + 2);
+    __hip_atomic_store(f.scalar + 8 + b, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__hip_atomic_fetch_add(count, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) != unsigned(f.blocks - 1)) return;
+    for (int k = 0; k < f.blocks; ++k) {
+      const double x = __hip_atomic_load(f.scalar + 8 + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      m = x < m ? x : m;
+    }
+    __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (f.unit) m = 1.;
+  double dt = (f.max_time_step < m ? f.max_time_step : m) * f.cheby;
+  // the product is rounded before it is accumulated, as the host's flow_time += dt does (no fused multiply-add)
+  asm volatile("" : "+v"(dt));
+  f.step->dt = dt;
+  if (f.accumulate) {
+    f.step->time_step = dt;
+    f.step->flow_time += dt;
+    if (f.count) ++f.step->iteration;
+  }
+  if (f.host) {
+    __hip_atomic_store(f.host, dt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(reinterpret_cast<unsigned long long*>(f.host) + 1, f.seq, __ATOMIC_RELEASE,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
 // Connection_direction (Kernel_connection.hpp:7-37) from the packed form of hx_host_mesh::con_dir
 struct Dir
 {

@@ -2154,10 +2154,12 @@ __device__ __forceinline__ void state_bcs_at(const Dev_mesh& m, int gid)
   }
 }
 
+// the first f.blocks workgroups form the step's time step
 template <int ND, int RS>
-__global__ __launch_bounds__(256) void k_state_bcs(Dev_mesh m)
+__global__ __launch_bounds__(256) void k_state_bcs(Dev_mesh m, Dt_final f)
 {
-  state_bcs_at<ND, RS>(m, blockIdx.x * 256 + threadIdx.x);
+  if (int(blockIdx.x) < f.blocks) dt_final(f, blockIdx.x);
+  else state_bcs_at<ND, RS>(m, (blockIdx.x - f.blocks) * 256 + threadIdx.x);
 }
 
 template <int ND, int RS>
@@ -2239,12 +2241,13 @@ struct Launchers
   using S = Shape<ND, RS>;
   static const Ops<RS>* ops(const Launch& l) { return static_cast<const Ops<RS>*>(l.ops); }
   static const Ops<RS>& hops(const Launch& l) { return *static_cast<const Ops<RS>*>(l.hops); }
+  static const Eops<RS, double>& heops(const Launch& l) { return *static_cast<const Eops<RS, double>*>(l.heops); }
 
   static hipError_t write_face(const Launch& l, int cls, int scale_velocity)
   {
     const int n = l.m.n_elem[cls];
     if (n == 0) return hipSuccess;
-    const Eops<RS, double> o = make_eops<RS, double>(hops(l));
+    const Eops<RS, double>& o = heops(l);
     hipLaunchKernelGGL((k_write_face<ND, RS>), dim3(blocks_for(n, S::EPB)), dim3(S::BLOCK), 0, l.stream, l.m, o, cls,
                        scale_velocity);
     return hipGetLastError();
@@ -2283,7 +2286,7 @@ struct Launchers
     const int n = l.m.n_elem[cls];
     if (n == 0) return hipSuccess;
     dim3 g(blocks_for(n, S::EPB)), b(form_block<ND, RS, P>());
-    const Eops<RS, double> o = make_eops<RS, double>(hops(l));
+    const Eops<RS, double>& o = heops(l);
     const Eops<RS, double>* od = static_cast<const Eops<RS, double>*>(l.eops);
     if (l.fold) return local_fold<P, true>(l, cls, visc, coef, stage, cr, uf, g, b, o, od);
     return local_fold<P, false>(l, cls, visc, coef, stage, cr, uf, g, b, o, od);
@@ -2337,7 +2340,7 @@ struct Launchers
     const int n = l.m.n_elem[cls];
     if (n == 0) return hipSuccess;
     dim3 g(blocks_for(n, S::EPB)), b(S::BLOCK);
-    const Eops<RS, double> o = make_eops<RS, double>(hops(l));
+    const Eops<RS, double>& o = heops(l);
     if (l.fold) {
       if (cls == HX_DEFORMED)
         hipLaunchKernelGGL((k_reconcile_ldg<ND, RS, true, true>), g, b, 0, l.stream, l.m, o, dt, l.dtp, cr, uf);
@@ -2398,8 +2401,9 @@ struct Launchers
   }
   static hipError_t state_bcs(const Launch& l)
   {
-    if (l.m.n_bc_con == 0) return hipSuccess;
-    hipLaunchKernelGGL((k_state_bcs<ND, RS>), dim3(blocks_for(size_t(l.m.n_bc_con) * S::NFQ, 256)), dim3(256), 0, l.stream, l.m);
+    const unsigned g = blocks_for(size_t(l.m.n_bc_con) * S::NFQ, 256) + l.dtf.blocks;
+    if (g == 0) return hipSuccess;
+    hipLaunchKernelGGL((k_state_bcs<ND, RS>), dim3(g), dim3(256), 0, l.stream, l.m, l.dtf);
     return hipGetLastError();
   }
   static hipError_t flux_bcs(const Launch& l)
@@ -2425,7 +2429,7 @@ struct Launchers
   {
     const int n = l.m.n_elem[cls];
     if (n == 0) return hipSuccess;
-    const Eops<RS, double> o = make_eops<RS, double>(hops(l));
+    const Eops<RS, double>& o = heops(l);
     dim3 g(blocks_for(n, S::EPB)), b(S::BLOCK);
     if (kind == av_kind_adv) hipLaunchKernelGGL((k_av_write_face<ND, RS, av_kind_adv>), g, b, 0, l.stream, l.m, o, cls);
     else if (kind == av_kind_sav) hipLaunchKernelGGL((k_av_write_face<ND, RS, av_kind_sav>), g, b, 0, l.stream, l.m, o, cls);
@@ -2455,7 +2459,7 @@ struct Launchers
   {
     const int n = l.m.n_elem[cls];
     if (n == 0) return hipSuccess;
-    const Eops<RS, double> o = make_eops<RS, double>(hops(l));
+    const Eops<RS, double>& o = heops(l);
     const Av_consts<RS> c = av_consts(l, project_av_rs > 0 ? project_av_rs : RS);
     const int project = project_av_rs > 0;
     dim3 g(blocks_for(n, S::EPB)), b(S::BLOCK);
@@ -2468,7 +2472,7 @@ struct Launchers
   template <int KIND>
   static void diff_local_as(const Launch& l, int cls, double dt, double diff_time)
   {
-    const Eops<RS, double> o = make_eops<RS, double>(hops(l));
+    const Eops<RS, double>& o = heops(l);
     dim3 g(blocks_for(l.m.n_elem[cls], S::EPB)), b(S::BLOCK);
     if (cls == HX_DEFORMED) hipLaunchKernelGGL((k_sav_local<ND, RS, true, KIND>), g, b, 0, l.stream, l.m, o, dt, diff_time);
     else hipLaunchKernelGGL((k_sav_local<ND, RS, false, KIND>), g, b, 0, l.stream, l.m, o, dt, diff_time);
@@ -2498,7 +2502,7 @@ struct Launchers
   template <int KIND>
   static void diff_reconcile_as(const Launch& l, int cls, double dt, double diff_time, double cheby)
   {
-    const Eops<RS, double> o = make_eops<RS, double>(hops(l));
+    const Eops<RS, double>& o = heops(l);
     dim3 g(blocks_for(l.m.n_elem[cls], S::EPB)), b(S::BLOCK);
     if (cls == HX_DEFORMED)
       hipLaunchKernelGGL((k_sav_reconcile<ND, RS, true, KIND>), g, b, 0, l.stream, l.m, o, dt, diff_time, cheby);

@@ -15,11 +15,13 @@ struct Launch
   const void* ops;   // device Ops<row_size>
   const void* hops;  // host copy of the same Ops<row_size>
   const void* eops;  // device Eops<row_size, double>
+  const void* heops; // host copy of the same, for kernels taking it by value
   Ns_params ns;      // transport models (Navier-Stokes)
   double* scalar;    // device scratch: [0] time step reduction
   int precision;     // hx_precision
   Dt_fuse fuse;      // next step's Max_dt fused into the Euler Local (slots == nullptr: not fused)
   const double* dtp; // device-resident time step the stage kernels multiply their coefficient by, or null
+  Dt_final dtf;      // the time step state_bcs forms beside the boundary conditions (blocks == 0: none)
   int fold;          // face-flux folding: the Local computes its faces' fluxes, Neighbor covers only mortar connections
 };
 
@@ -50,7 +52,7 @@ struct Kernel_set
   // batch of independent cases: global-time-step Max_dt with a minimum per case
   hipError_t (*max_dt_cases)(const Launch&, int cls, bool visc, double max_cfl_c, double max_cfl_d, const int* case_id,
                              unsigned long long* case_min);
-  // Solver::is_admissible (flags[0]: some state inadmissible, flags[1]: some value not finite; zero them first) and
+  // Solver::is_admissible (flags[0] = 1: some state inadmissible, flags[1] = 1: some value not finite; zero them first) and
   // the artificial-viscosity swap of Solver::fix_admissibility
   hipError_t (*admissible)(const Launch&, int* flags);
   hipError_t (*fix_av)(const Launch&, int mode);
