@@ -118,6 +118,8 @@ struct hx_mesh
   // when each class lists its cases in order (non-decreasing ids): first element of every case, [n_cases + 1]
   int* case_start[2] = {};
   int case_split[2] = {};  // workgroups per case of the per-case reduction
+  int case_biggest = 0;    // elements of the largest case, over both classes
+  double* case_host = nullptr;  // pinned: every case's time step, then its sequence number (Case_step::host)
   // Max_dt fused into the last stage of hx_update: every call that can change device data (a kernel launch, an
   // upload, handing out a device pointer) advances `gen`; the next hx_update takes the fused minimum only if `gen` is
   // where the previous hx_update left it and its time-step settings are the same
@@ -135,8 +137,8 @@ struct hx_mesh
     hx_transport visc{}, cond{};
     bool in_scratch = false;  // the minima are in the scratch array (hx_update_no_alloc), not in dt_block_min
   } dt_cache;
-  // the same fusion for hx_update_cases (cases listed in order): stage 1's Local writes each point's 1/scale into
-  // case_scale, which the next call's per-case minimum reads instead of running Max_dt
+  // the same fusion for hx_update_cases (cases listed in order): stage 1's Local writes each element's minimum
+  // of 1/scale into case_scale, which the next call's per-case minimum reads instead of running Max_dt
   double* case_scale[2] = {};
   struct
   {
@@ -200,7 +202,7 @@ struct hx_group
   hx::Fused_plan* plans = nullptr;      // device [3]: state BCs, Neighbor, Local
   hx::Fused_plan hplan[3]{};
   std::vector<hx::Fused_member> hmem;   // host copy of `mem`
-  double* dts = nullptr;                // pinned host: every case's time step
+  double* dts = nullptr;                // pinned host: every case's time step, then the sequence number
   int order = 2, per_cu = 0;            // launch shape of the fused Local (hx_group_set_shape)
   int n_cu = 0;
   const void* hops[HX_MAX_ROW_SIZE + 1] = {};  // the context's host Ops<rs> tables, by row size
@@ -246,6 +248,8 @@ void release_mesh_memory(hx_mesh* mesh)
   mesh->case_scale[0] = mesh->case_scale[1] = nullptr;
   mesh->case_min = nullptr;
   mesh->case_dt = nullptr;
+  if (mesh->case_host) (void)hipHostFree(mesh->case_host);
+  mesh->case_host = nullptr;
   mesh->dt_block_min = nullptr;
   mesh->step = mesh->sync_step = nullptr;
   mesh->dtf = Dt_final{};
@@ -711,6 +715,65 @@ __global__ __launch_bounds__(256) void k_case_tss(double* __restrict__ tss, cons
 {
   for (size_t i = size_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += size_t(gridDim.x) * 256)
     tss[i] = case_dt[case_id[i / nq]];
+}
+
+// The time steps of a step of several batch meshes, every case's per-element minima of 1/scale being those of the current
+// state (Dt_fuse::elem_scale): `split` workgroups per case, each of which takes the minimum over the case's elements and
+// writes its share of the case's time step scale; the first also stores the time step. One launch where each mesh took
+// four (fill, minimum over every point's 1/scale, time step, time step scale: about 35 us per mesh and step).
+struct Case_member
+{
+  const double* emin[2];  // per class
+  const int* start[2];    // per class, [n_cases + 1], or null (no elements)
+  double* tss[2];
+  double* case_dt;
+  int n_cases, nq, split, first_block, off;  // off: its first case among the launch's
+};
+struct Case_step
+{
+  int n, n_cases;
+  Case_member m[hx::fused_max_seg / 2];
+  double max_time_step, cheby;
+  unsigned* count;  // zero between launches
+  double* host;     // pinned: [n_cases] time steps, then `seq` (as an integer) once all are there
+  unsigned long long seq;
+};
+__global__ __launch_bounds__(256) void k_case_step(Case_step s)
+{
+  __shared__ double w[4];
+  int k = 0;
+  while (k + 1 < s.n && int(blockIdx.x) >= s.m[k + 1].first_block) ++k;
+  const Case_member& m = s.m[k];
+  const int b = blockIdx.x - m.first_block, ic = b / m.split, slice = b % m.split;
+  double mdt = DBL_MAX;
+  for (int c = 0; c < 2; ++c)
+    if (m.start[c])
+      for (int e = m.start[c][ic] + threadIdx.x; e < m.start[c][ic + 1]; e += 256) {
+        const double x = m.emin[c][e];
+        mdt = x < mdt ? x : mdt;
+      }
+  for (int off = 32; off > 0; off /= 2) {
+    const double x = __shfl_xor(mdt, off, 64);
+    mdt = x < mdt ? x : mdt;
+  }
+  if ((threadIdx.x & 63) == 0) w[threadIdx.x / 64] = mdt;
+  __syncthreads();
+  for (int j = 0; j < 4; ++j) mdt = w[j] < mdt ? w[j] : mdt;
+  const double dt = (s.max_time_step < mdt ? s.max_time_step : mdt) * s.cheby;
+  for (int c = 0; c < 2; ++c)
+    if (m.start[c]) {
+      const long long lo = (long long)m.start[c][ic] * m.nq, hi = (long long)m.start[c][ic + 1] * m.nq;
+      const long long per = (hi - lo + m.split - 1) / m.split, a = lo + slice * per, z = a + per < hi ? a + per : hi;
+      for (long long i = a + threadIdx.x; i < z; i += 256) m.tss[c][i] = dt;
+    }
+  if (slice || threadIdx.x) return;
+  m.case_dt[ic] = dt;
+  __hip_atomic_store(s.host + m.off + ic, dt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __threadfence_system();
+  if (__hip_atomic_fetch_add(s.count, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) != unsigned(s.n_cases - 1)) return;
+  __hip_atomic_store(s.count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(reinterpret_cast<unsigned long long*>(s.host) + s.n_cases, s.seq, __ATOMIC_RELEASE,
+                     __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 __global__ __launch_bounds__(256) void k_fill_u64(unsigned long long* p, unsigned long long v, int n)
@@ -1576,12 +1639,12 @@ hx_status enqueue_max_dt(hx_mesh* mesh, const hx_update_options* o, const Update
   return HX_OK;
 }
 
-// Waits for the time step with sequence number `seq` that a launch of this context sends to the pinned host words
-// (Dt_final::host): it arrives while the stage kernels queued behind it run. Ends with an error if the stream drains, or
-// fails, without it.
-hx_status wait_dt(hx_ctx* ctx, unsigned long long seq, double* dt)
+// Waits until a launch of this context has written sequence number `seq` to pinned host memory, behind the time steps it
+// sends (Dt_final::host, Case_step::host): they arrive while the stage kernels queued behind that launch run. Ends with an
+// error if the stream drains, or fails, without it.
+hx_status wait_seq(hx_ctx* ctx, const double* word, unsigned long long seq)
 {
-  const auto* arrived = reinterpret_cast<const unsigned long long*>(ctx->host_scalar + 5);
+  const auto* arrived = reinterpret_cast<const unsigned long long*>(word);
   for (unsigned spin = 1; __atomic_load_n(arrived, __ATOMIC_ACQUIRE) != seq; ++spin) {
     if (spin % 1024) {
       __builtin_ia32_pause();
@@ -1592,7 +1655,6 @@ hx_status wait_dt(hx_ctx* ctx, unsigned long long seq, double* dt)
     HX_TRY(ctx, e, "time step");
     if (__atomic_load_n(arrived, __ATOMIC_ACQUIRE) != seq) return fail(ctx, HX_ERR_HIP, "the time step did not arrive");
   }
-  *dt = ctx->host_scalar[4];
   return HX_OK;
 }
 
@@ -1691,8 +1753,10 @@ hx_status update_once(hx_mesh* mesh, const hx_update_options* o, const Update_se
           }
         }
       }
-      if (f.host)
-        if ((s = wait_dt(ctx, f.seq, &dt))) return s;
+      if (f.host) {
+        if ((s = wait_seq(ctx, f.host + 1, f.seq))) return s;
+        dt = f.host[0];
+      }
       // a fix changed the state after the fused Max_dt read it, and ends this Chebyshev sequence (Solver.cpp:869)
       if (fixed) {
         pending = false;
@@ -1906,6 +1970,7 @@ hx_status hx_mesh_set_cases(hx_mesh* mesh, int n_cases, const int* case_cartesia
   if (!alloc(&cmin, size_t(n_cases) * 8) || !alloc(&cdt, size_t(n_cases) * 8))
     return fail(ctx, HX_ERR_HIP, "hipMalloc(case time steps)");
   // cases listed in order within each class: their element ranges, for the streaming per-case reduction
+  mesh->case_biggest = 0;
   for (int c = 0; c < 2; ++c) {
     mesh->case_start[c] = nullptr;
     bool sorted = true;
@@ -1923,7 +1988,13 @@ hx_status hx_mesh_set_cases(hx_mesh* mesh, int n_cases, const int* case_cartesia
     HX_TRY(ctx, hipMemcpy(d, start.data(), start.size() * sizeof(int), hipMemcpyHostToDevice), "upload case ranges");
     mesh->case_start[c] = d;
     mesh->case_split[c] = int(std::max<long long>(1, (long long)biggest * m.nq / 8192));
+    mesh->case_biggest = std::max(mesh->case_biggest, biggest);
   }
+  if (mesh->case_host) (void)hipHostFree(mesh->case_host);
+  mesh->case_host = nullptr;
+  HX_TRY(ctx, hipHostMalloc(&mesh->case_host, size_t(n_cases + 1) * 8, hipHostMallocMapped | hipHostMallocCoherent),
+         "hipHostMalloc(case time steps)");
+  std::memset(mesh->case_host, 0, size_t(n_cases + 1) * 8);
   mesh->n_cases = n_cases;
   mesh->case_id[0] = dev_ids[0];
   mesh->case_id[1] = dev_ids[1];
@@ -1951,8 +2022,8 @@ struct Cases_step
   const char* name;
   double cc, cd;       // the constants of Max_dt with safety_conv = max_safety / max Chebyshev step, safety_diff = max_safety
   double n_cheby;
-  bool fusable;        // every class lists its cases in order: stage 1's Local computes the next step's 1/scale per point
-  bool pending;        // the previous call's per-point 1/scale is still that of the current state
+  bool fusable;        // every class lists its cases in order: stage 1's Local computes the next step's minima per element
+  bool pending;        // the previous call's per-element minima are still those of the current state
   long long gen_at_entry;
 };
 
@@ -1972,15 +2043,15 @@ hx_status cases_setup(hx_mesh* mesh, const hx_update_options* o, Cases_step& c)
   const double max_cheby = cheby_step(c.n_cheby, c.n_cheby - 1);
   c.cc = hx_basis_max_cfl(rs) * (o->max_safety / max_cheby);
   c.cd = -2 / hx_basis_tables::eigenvalss[rs - 2][1] * o->max_safety;
-  // with every class's cases in order, stage 1's Local also computes the next step's per-point 1/scale (the state it
-  // writes is the state the next Max_dt reads); the next call uses it if nothing changed the mesh in between and the
+  // with every class's cases in order, stage 1's Local also computes the next step's minimum of 1/scale per element (the
+  // state it writes is the state the next Max_dt reads); the next call uses it if nothing changed the mesh in between and the
   // time-step settings are the same
   c.fusable = true;
   for (int k = 0; k < 2; ++k) c.fusable = c.fusable && (!mesh->dm.n_elem[k] || mesh->case_start[k]);
   for (int k = 0; k < 2 && c.fusable; ++k)
     if (mesh->dm.n_elem[k] && !mesh->case_scale[k]) {
       void* q = nullptr;
-      HX_TRY(ctx, hipMalloc(&q, size_t(mesh->dm.n_elem[k]) * mesh->dm.nq * sizeof(double)), "hipMalloc(case scale)");
+      HX_TRY(ctx, hipMalloc(&q, size_t(mesh->dm.n_elem[k]) * sizeof(double)), "hipMalloc(case scale)");
       mesh->allocs.push_back(q);
       mesh->case_scale[k] = static_cast<double*>(q);
     }
@@ -2003,12 +2074,11 @@ hx_status cases_dt(hx_mesh* mesh, const hx_update_options* o, const Cases_step& 
     if (!mesh->dm.n_elem[k]) continue;
     Timer tm(ctx, std::string(cls_name(k)) + "/compute time step/" + c.name, mesh->dm.n_elem[k]);
     if (mesh->case_start[k]) {
-      // each point's 1/scale into the time step scale (Max_dt in local mode), or the fused values of the previous
-      // stage 1, then a streaming minimum per case
-      if (!c.pending) HX_TRY(ctx, mesh->ks->max_dt(c.l, k, c.visc, 1, c.cc, c.cd), "max_dt");
-      hipLaunchKernelGGL(k_case_min_tss, dim3(nc * mesh->case_split[k]), dim3(256), 0, c.l.stream,
-                         c.pending ? mesh->case_scale[k] : mesh->dm.tss[k], mesh->case_start[k], mesh->dm.nq,
-                         mesh->case_split[k], mesh->case_min);
+      // each point's 1/scale into the time step scale (Max_dt in local mode), then a streaming minimum per case (the
+      // fused minima of the previous stage 1 are taken by k_case_step)
+      HX_TRY(ctx, mesh->ks->max_dt(c.l, k, c.visc, 1, c.cc, c.cd), "max_dt");
+      hipLaunchKernelGGL(k_case_min_tss, dim3(nc * mesh->case_split[k]), dim3(256), 0, c.l.stream, mesh->dm.tss[k],
+                         mesh->case_start[k], mesh->dm.nq, mesh->case_split[k], mesh->case_min);
       HX_TRY(ctx, hipGetLastError(), "case minimum");
     } else {
       HX_TRY(ctx, mesh->ks->max_dt_cases(c.l, k, c.visc, c.cc, c.cd, mesh->case_id[k], mesh->case_min), "max_dt_cases");
@@ -2027,7 +2097,44 @@ hx_status cases_dt(hx_mesh* mesh, const hx_update_options* o, const Cases_step& 
   return HX_OK;
 }
 
-// the stage-1 fusion of the Euler Local in a batch step: each point's next-step 1/scale into case_scale
+// every case's time step of meshes whose fused minima are current, formed by one launch that also sends them to `host`
+// (all the meshes' cases in order, then the sequence number `seq`)
+hx_status cases_dt_fused(hx_ctx* ctx, hx_mesh* const* meshes, int n, const hx_update_options* o, double cheby, double* host,
+                         unsigned long long seq)
+{
+  Case_step s{};
+  s.n = n;
+  int blocks = 0;
+  for (int k = 0; k < n; ++k) {
+    hx_mesh* mesh = meshes[k];
+    Case_member& m = s.m[k];
+    for (int c = 0; c < 2; ++c) {
+      m.emin[c] = mesh->case_scale[c];
+      m.start[c] = mesh->dm.n_elem[c] ? mesh->case_start[c] : nullptr;
+      m.tss[c] = mesh->dm.tss[c];
+    }
+    m.case_dt = mesh->case_dt;
+    m.n_cases = mesh->n_cases;
+    m.nq = mesh->dm.nq;
+    m.split = int(std::max<long long>(1, (long long)mesh->case_biggest * m.nq / 16384));
+    m.first_block = blocks;
+    m.off = s.n_cases;
+    blocks += m.n_cases * m.split;
+    s.n_cases += m.n_cases;
+    ++mesh->gen;
+  }
+  s.max_time_step = o->max_time_step;
+  s.cheby = cheby;
+  s.count = reinterpret_cast<unsigned*>(ctx->scalar + 3);
+  s.host = host;
+  s.seq = seq;
+  Timer tm(ctx, "fused/compute time step/cases", s.n_cases);
+  hipLaunchKernelGGL(k_case_step, dim3(blocks), dim3(256), 0, ctx->stream, s);
+  HX_TRY(ctx, hipGetLastError(), "case time steps");
+  return HX_OK;
+}
+
+// the stage-1 fusion of the Euler Local in a batch step: each element's next-step minimum of 1/scale into case_scale
 Dt_fuse cases_fuse(const hx_mesh* mesh, const hx_update_options* o, const Cases_step& c)
 {
   Dt_fuse f{};
@@ -2035,8 +2142,8 @@ Dt_fuse cases_fuse(const hx_mesh* mesh, const hx_update_options* o, const Cases_
   f.max_cfl_c = c.cc;
   f.max_cfl_d = c.cd;
   f.ns = c.l.ns;
-  f.point_scale[0] = mesh->case_scale[0];
-  f.point_scale[1] = mesh->case_scale[1];
+  f.elem_scale[0] = mesh->case_scale[0];
+  f.elem_scale[1] = mesh->case_scale[1];
   return f;
 }
 
@@ -2107,10 +2214,21 @@ hx_status hx_update_cases(hx_mesh* mesh, const hx_update_options* o, hx_update_s
   for (int i_flow = 0; i_flow < o->flow_iters; ++i_flow) {
     for (int i_cheby = 0; i_cheby < c.n_cheby; ++i_cheby) {
       c.pending = pending;
-      if (hx_status s = cases_dt(mesh, o, c, i_cheby)) return s;
+      const bool fused = pending;
+      const unsigned long long seq = ++ctx->dt_seq;
+      if (fused) {
+        if (hx_status s = cases_dt_fused(ctx, &mesh, 1, o, cheby_step(c.n_cheby, i_cheby), mesh->case_host, seq)) return s;
+      } else {
+        if (hx_status s = cases_dt(mesh, o, c, i_cheby)) return s;
+      }
       for (int i = 0; i < 2; ++i)
         if (hx_status s = cases_stage(mesh, o, c, i)) return s;
       pending = c.fusable;
+      if (fused) {
+        if (hx_status s = wait_seq(ctx, mesh->case_host + nc, seq)) return s;
+        cases_status(mesh, mesh->case_host, st);
+        continue;
+      }
       HX_TRY(ctx, hipMemcpyAsync(dts.data(), mesh->case_dt, nc * sizeof(double), hipMemcpyDeviceToHost, c.l.stream),
              "case dt readback");
       HX_TRY(ctx, hipStreamSynchronize(c.l.stream), "case dt sync");
@@ -2273,8 +2391,10 @@ hx_status hx_group_create(hx_ctx* ctx, hx_mesh* const* meshes, int n_meshes, hx_
     delete g;
     return s;
   };
-  if (hipHostMalloc(reinterpret_cast<void**>(&g->dts), std::max(1, g->n_cases) * sizeof(double), hipHostMallocDefault) != hipSuccess)
+  if (hipHostMalloc(reinterpret_cast<void**>(&g->dts), (g->n_cases + 1) * sizeof(double),
+                    hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
     return bail(fail(ctx, HX_ERR_HIP, "hipHostMalloc(group time steps)"));
+  std::memset(g->dts, 0, (g->n_cases + 1) * sizeof(double));
   if (fusable) {
     g->fs = hx::fused_set_nd3();
     if (hipMalloc(reinterpret_cast<void**>(&g->mem), 2 * n_meshes * sizeof(hx::Fused_member)) != hipSuccess ||
@@ -2346,12 +2466,28 @@ hx_status hx_group_update(hx_group* g, const hx_update_options* o, hx_update_sta
   if (hx_status s = upload_members(g, fuse)) return s;
   for (int i_flow = 0; i_flow < o->flow_iters; ++i_flow) {
     for (int i_cheby = 0; i_cheby < c[0].n_cheby; ++i_cheby) {
+      bool fused = true;
       for (int k = 0; k < n; ++k) {
         c[k].pending = pending[k];
-        if (hx_status s = cases_dt(g->meshes[k], o, c[k], i_cheby)) return s;
+        fused = fused && pending[k];
+      }
+      const unsigned long long seq = ++ctx->dt_seq;
+      if (fused) {
+        if (hx_status s = cases_dt_fused(ctx, g->meshes.data(), n, o, cheby_step(c[0].n_cheby, i_cheby), g->dts, seq)) return s;
+      } else {
+        for (int k = 0; k < n; ++k)
+          if (hx_status s = cases_dt(g->meshes[k], o, c[k], i_cheby)) return s;
       }
       for (int i = 0; i < 2; ++i)
         if (hx_status s = group_stage(g, o, i)) return s;
+      if (fused) {
+        if (hx_status s = wait_seq(ctx, g->dts + g->n_cases, seq)) return s;
+        for (int k = 0, off = 0; k < n; off += g->meshes[k]->n_cases, ++k) {
+          pending[k] = c[k].fusable;
+          cases_status(g->meshes[k], g->dts + off, st + off);
+        }
+        continue;
+      }
       for (int k = 0, off = 0; k < n; off += g->meshes[k]->n_cases, ++k) {
         pending[k] = c[k].fusable;
         HX_TRY(ctx, hipMemcpyAsync(g->dts + off, g->meshes[k]->case_dt, g->meshes[k]->n_cases * sizeof(double),

@@ -162,7 +162,7 @@ struct Dt_fuse
   int visc;  // include the diffusive scale (Max_dt of Navier-Stokes)
   double max_cfl_c, max_cfl_d;
   Ns_params ns;
-  double* point_scale[2];  // per class, each point's 1/scale (the batch's per-case time steps), or null
+  double* elem_scale[2];  // per class, each element's minimum of 1/scale (the batch's per-case time steps), or null
 };
 
 // The status of the updates whose time step stays on the device

@@ -925,7 +925,7 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
       for (int v = 0; v < NV; ++v) ld[el2 * L::PER_D + L::sb(face) + v * NFQ + p] = fl[v];
   }
   const double p64 = P::mfma ? pressure_of<ND>(u) : 0.;
-  const bool fused_dt = (fuse.block_min || fuse.point_scale[cls]) && !compute_residual;
+  const bool fused_dt = (fuse.block_min || fuse.elem_scale[cls]) && !compute_residual;
   // what the end of the tile reads from memory: the residual cache (stage 1), the nominal size, the time step scale, the
   // Jacobian determinant, and for the fused time step the viscosity coefficients; and the element's tables (L::TB),
   // each thread fetching one entry of each. All are requested before the last direction's row phase.
@@ -1021,7 +1021,6 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
     // folded as k_max_dt does: a NaN of this point never wins (std::min(dt, NaN) keeps dt in the reference)
     const double inv = 1. / scale;
     c = (inv < c) ? inv : c;
-    if (fuse.point_scale[cls]) fuse.point_scale[cls][size_t(e) * NQ + q] = inv;
   }
   // Write_face of the updated state (Spatial.hpp:507)
   if (pt)
@@ -1029,6 +1028,24 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
   __syncthreads();
   write_faces_to<ND, RS, NT, NV>(m, cls, blk, o, ld + L::U, L::PER_D,
                                  [&](int el2) { return reinterpret_cast<const int*>(ld + el2 * L::PER_D + L::TB_SLOT); });
+  if (fused_dt && fuse.elem_scale[cls]) {
+    // one wavefront per element takes its points' minimum (every wave of the workgroup is whole)
+    __syncthreads();
+    if (pt) myd[q] = c;
+    __syncthreads();
+    for (int el2 = t / 64; el2 < EPB; el2 += NT / 64) {
+      double b = DBL_MAX;
+      for (int k = t & 63; k < NQ; k += 64) {
+        const double x = ld[el2 * L::PER_D + k];
+        b = (x < b) ? x : b;
+      }
+      for (int off = 32; off > 0; off /= 2) {
+        const double x = __shfl_xor(b, off, 64);
+        b = (x < b) ? x : b;
+      }
+      if ((t & 63) == 0 && blk * EPB + el2 < n) fuse.elem_scale[cls][blk * EPB + el2] = b;
+    }
+  }
   if (fuse.block_min) {
     for (int off = 32; off > 0; off /= 2) {
       const double x = __shfl_xor(c, off, 64);
