@@ -117,9 +117,10 @@ def algorithmic_bytes(category, nd, nq, n_elem):
 FORMS = {"fp64": (abi.HX_FP64, "Fp64_form"), "fp32_mfma": (abi.HX_FP32_MFMA, "Fp32_mfma_form")}
 
 
-def folds_faces(nd, rs, mode):
-    """Whether hx_update folds the face fluxes into the Local (hx_mesh_set_face_fold)."""
-    return mode == 1 or (mode == -1 and rs >= 2 * nd)
+def folds_faces(nd, rs, mode, visc=True):
+    """Whether hx_update folds the faces into the element kernels (hx_mesh_set_face_fold): all of them with `visc`, the
+    face fluxes alone without (an Euler update has no others)."""
+    return mode == 1 or (mode == -1 and (not visc or rs >= 2 * nd))
 
 
 def kernel_symbol(category, nd, rs, form, fold):
@@ -371,7 +372,8 @@ def main():
     ap.add_argument("--setup", type=int, default=1,
                     help="ns48: also time calc_jacobian, is_admissible and fix_admissibility (0 to skip)")
     ap.add_argument("--face-fold", type=int, default=-1, choices=(-1, 0, 1),
-                    help="fold the face fluxes into the Local: 1 always, 0 never, -1 where 2 n_dim <= row_size")
+                    help="fold the faces into the element kernels: 1 all, 0 none, -1 the fluxes always, the viscous jumps "
+                         "where 2 n_dim <= row_size")
     args = ap.parse_args()
     world = int(os.environ.get("WORLD_SIZE", "1"))
     if args.gpus != 1 or world != 1:
@@ -463,7 +465,7 @@ def main():
         symbol = (f"k_fused_local_euler<{nd}, {FORMS[args.precision][1]}, {'true' if with_def else 'false'}, "
                   f"{'true' if persist else 'false'}, 4, 5, 6>")
     else:
-        symbol = (kernel_symbol(dominant, nd, rs0, args.precision, folds_faces(nd, rs0, args.face_fold))
+        symbol = (kernel_symbol(dominant, nd, rs0, args.precision, folds_faces(nd, rs0, args.face_fold, False))
                   if len(hosts) == 1 else None)
     roofline = {"bound": "hbm", "kernel": dominant, "symbol": symbol, "launch_ms": round(ms / launches, 5),
                 "peak": HBM_PEAK_GBS, "unit": "GB/s",

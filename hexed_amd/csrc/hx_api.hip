@@ -161,8 +161,8 @@ struct hx_mesh
   int n_groups = 0;  // groups (hx_group) holding the mesh, which must be destroyed first
   // face-flux folding of the current stage of an update (Dev_mesh::partner): the buffer holding the face states the
   // stage reads (alt_rd) and the one its face extrapolations go to (alt_wr)
-  int fold = 0, alt_rd = 0, alt_wr = 0;
-  int face_fold_mode = -1;  // hx_mesh_set_face_fold: 1 fold, 0 do not, -1 fold where rs >= 2 n_dim
+  int fold = 0, fold_ldg = 0, alt_rd = 0, alt_wr = 0;
+  int face_fold_mode = -1;  // hx_mesh_set_face_fold: 1 fold, 0 do not, -1 as Stage_fold decides
   bool mortar_fusable = false;  // every refined face's mortars are in connections (k_mortar_restrict applies)
   hipGraphExec_t graph = nullptr;
   hx_update_options graph_opts{};
@@ -558,6 +558,7 @@ Launch make_launch(hx_mesh* mesh, bool writes = true)
   l.dtf = mesh->dtf;
   l.dtp = mesh->dt_dev;
   l.fold = mesh->fold;
+  l.fold_ldg = mesh->fold_ldg;
   l.m.alt_rd = mesh->alt_rd;
   l.m.alt_wr = mesh->alt_wr;
   return l;
@@ -1658,26 +1659,28 @@ hx_status wait_seq(hx_ctx* ctx, const double* word, unsigned long long seq)
   return HX_OK;
 }
 
-// Whether hx_update folds the face fluxes into the Local: by default where an element has no more face points than
-// volume points (2 n_dim rs^(n_dim-1) <= rs^n_dim, i.e. rs >= 2 n_dim), where the neighbour's face states the Local
-// then reads cost less than the Neighbor launch saves (measured: 3D row size 6 folded is 20-28% faster per step, row
-// size 4 on a tree mesh 8% slower)
-bool folds_faces(const hx_mesh* mesh)
-{
-  return mesh->face_fold_mode == 1 || (mesh->face_fold_mode == -1 && mesh->dm.rs >= 2 * mesh->dm.nd);
-}
-
-// the face-flux folding flags of one stage of an update, reset when the stage ends
+// The face-flux folding flags of one stage of an update, reset when the stage ends. By default the Local always folds:
+// with its face loads in one step it is faster at every row size and n_dim (whole steps of Cartesian Euler boxes of 2e5
+// points, not folded -> folded: 3D row size 2 449 -> 331 us, 3 344 -> 239, 4 316 -> 253, 5 304 -> 236, 6 280 -> 215; 2D
+// row size 2 352 -> 222, 3 321 -> 217, 4 237 -> 165). Reconcile_ldg_flux folds its jumps where an element has no more
+// face points than volume points (rs >= 2 n_dim); below, an update leaves the reconciled jumps in the LDG blocks, as the
+// reference does.
 struct Stage_fold
 {
   hx_mesh* mesh;
-  Stage_fold(hx_mesh* m, bool on, int stage) : mesh{m}
+  Stage_fold(hx_mesh* m, bool on, bool ldg, int stage) : mesh{m}
   {
     mesh->fold = on ? 1 : 0;
+    mesh->fold_ldg = on && ldg ? 1 : 0;
     mesh->alt_rd = on ? stage : 0;
     mesh->alt_wr = on ? 1 - stage : 0;
   }
-  ~Stage_fold() { mesh->fold = mesh->alt_rd = mesh->alt_wr = 0; }
+  ~Stage_fold() { mesh->fold = mesh->fold_ldg = mesh->alt_rd = mesh->alt_wr = 0; }
+  static bool local(const hx_mesh* m) { return m->face_fold_mode != 0; }
+  static bool ldg(const hx_mesh* m)
+  {
+    return m->face_fold_mode == 1 || (m->face_fold_mode == -1 && m->dm.rs >= 2 * m->dm.nd);
+  }
 };
 
 // sets the time step the stage kernels read from the device (null: their coefficient holds it) for a scope
@@ -1687,6 +1690,34 @@ struct Device_dt
   Device_dt(hx_mesh* m, const double* dt) : mesh{m} { mesh->dt_dev = dt; }
   ~Device_dt() { mesh->dt_dev = nullptr; }
 };
+
+// Solver::is_admissible, the face states read from the buffer `alt` selects
+hx_status check_admissible(hx_mesh* mesh, int alt, bool* admissible)
+{
+  hx_ctx* ctx = mesh->ctx;
+  // (every use of the flags ends with a wait for the stream, so no kernel writes them now)
+  int* const h = reinterpret_cast<int*>(ctx->host_scalar + 6);
+  h[0] = h[1] = 0;
+  Launch l = make_launch(mesh, false);  // reads the fields only, so a fused Max_dt stays valid
+  l.m.alt_rd = alt;
+  {
+    Timer tm(ctx, "check admis.", (long long)mesh->dm.n_elem[0] + mesh->dm.n_elem[1]);
+    HX_TRY(ctx, mesh->ks->admissible(l, h), "is_admissible");
+  }
+  HX_TRY(ctx, hipStreamSynchronize(ctx->stream), "admissibility sync");
+  if (h[1]) return fail(ctx, HX_ERR_NOT_FINITE, "state is not finite");
+  *admissible = !h[0];
+  return HX_OK;
+}
+
+// the state blocks of every face slot from the second buffer into the primary one
+__global__ __launch_bounds__(256) void k_faces_to_primary(Dev_mesh m, long long n)
+{
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int per = m.nv * m.nfq;
+  state_ptr(m, int(i / per), 0)[i % per] = state_ptr(m, int(i / per), 1)[i % per];
+}
 
 // The kernels of one Solver::update (Solver.cpp:834-886), with fix_admissibility after each stage when enabled
 // (Solver.cpp:867). The time step is formed on the device, beside stage 0's boundary conditions, and read there by the
@@ -1722,15 +1753,14 @@ hx_status update_once(hx_mesh* mesh, const hx_update_options* o, const Update_se
           f.seq = ++ctx->dt_seq;
         }
       }
-      bool fixed = false;
+      bool fixed = false, fold = Stage_fold::local(mesh);
       {
         Device_dt in_use(mesh, device_dt ? &u.step->dt : nullptr);
         for (int i = 0; i < 2; ++i) {
           hx_kernel_options opts{dt, i, 0, o->use_filter};
-          // face-flux folding (not with the admissibility fix, which reads the faces between the stages): stage 0 reads
-          // the face states from the primary buffer and extrapolates into the second, stage 1 the other way round, so
-          // that an update leaves the faces where the reference's sequence leaves them
-          Stage_fold sf(mesh, !o->fix_admis && folds_faces(mesh), i);
+          // face-flux folding: stage 0 reads the face states from the primary buffer and extrapolates into the second,
+          // stage 1 the other way round, so that an update leaves the faces where the reference's sequence leaves them
+          Stage_fold sf(mesh, fold, Stage_fold::ldg(mesh), i);
           if (i == 0) mesh->dtf = f;
           s = hx_apply_state_bcs(mesh);
           mesh->dtf = Dt_final{};
@@ -1746,10 +1776,25 @@ hx_status update_once(hx_mesh* mesh, const hx_update_options* o, const Update_se
           }
           if (s) return s;
           if (o->fix_admis) {
-            int iters = 0;
-            if ((s = hx_fix_admissibility(mesh, o, o->fix_admis_max_safety, &iters))) return s;
-            st->fix_admis_iters += iters;
-            fixed = iters || fixed;
+            // the check reads the faces where the stage left them; a fix works on the primary buffer, so after a folded
+            // stage 0 that needs one the faces move there and stage 1 goes without folding
+            bool admissible = false;
+            if ((s = check_admissible(mesh, mesh->alt_wr, &admissible))) return s;
+            if (!admissible) {
+              if (mesh->alt_wr) {
+                const long long n = (long long)mesh->dm.n_slot * mesh->dm.nv * mesh->dm.nfq;
+                if (n)
+                  hipLaunchKernelGGL(k_faces_to_primary, dim3(unsigned((n + 255) / 256)), dim3(256), 0, ctx->stream,
+                                     mesh->dm, n);
+                HX_TRY(ctx, hipGetLastError(), "faces to the primary buffer");
+              }
+              fold = fold && i;
+              Stage_fold off(mesh, false, false, 0);
+              int iters = 0;
+              if ((s = hx_fix_admissibility(mesh, o, o->fix_admis_max_safety, &iters))) return s;
+              st->fix_admis_iters += iters;
+              fixed = iters || fixed;
+            }
           }
         }
       }
@@ -2151,7 +2196,7 @@ Dt_fuse cases_fuse(const hx_mesh* mesh, const hx_update_options* o, const Cases_
 hx_status cases_stage(hx_mesh* mesh, const hx_update_options* o, const Cases_step& c, int i)
 {
   hx_kernel_options opts{1., i, 0, o->use_filter};
-  Stage_fold sf(mesh, true, i);
+  Stage_fold sf(mesh, true, true, i);
   hx_status s;
   if ((s = hx_apply_state_bcs(mesh))) return s;
   if (o->use_ldg && !i) return hx_compute_navier_stokes(mesh, &opts, o->visc, o->cond);
@@ -2326,14 +2371,14 @@ hx_status group_stage(hx_group* g, const hx_update_options* o, int i)
     Group_fold(const std::vector<hx_mesh*>& m, int stage) : ms{m}
     {
       for (hx_mesh* x : ms) {
-        x->fold = 1;
+        x->fold = x->fold_ldg = 1;
         x->alt_rd = stage;
         x->alt_wr = 1 - stage;
       }
     }
     ~Group_fold()
     {
-      for (hx_mesh* x : ms) x->fold = x->alt_rd = x->alt_wr = 0;
+      for (hx_mesh* x : ms) x->fold = x->fold_ldg = x->alt_rd = x->alt_wr = 0;
     }
   } folds(g->meshes, i);
   {
@@ -2981,19 +3026,9 @@ hx_status hx_max_dt_fix_therm_admis(hx_mesh* mesh, const hx_kernel_options* o, d
 hx_status hx_is_admissible(hx_mesh* mesh, int* admissible)
 {
   if (!live(mesh) || !admissible) return HX_ERR_INVALID;
-  hx_ctx* ctx = mesh->ctx;
-  // reads the fields only, so a fused Max_dt stays valid
-  // (every use of the flags ends with a wait for the stream, so no kernel writes them now)
-  int* const h = reinterpret_cast<int*>(ctx->host_scalar + 6);
-  h[0] = h[1] = 0;
-  Launch l = make_launch(mesh, false);
-  {
-    Timer tm(ctx, "check admis.", (long long)mesh->dm.n_elem[0] + mesh->dm.n_elem[1]);
-    HX_TRY(ctx, mesh->ks->admissible(l, h), "is_admissible");
-  }
-  HX_TRY(ctx, hipStreamSynchronize(ctx->stream), "admissibility sync");
-  if (h[1]) return fail(ctx, HX_ERR_NOT_FINITE, "state is not finite");
-  *admissible = !h[0];
+  bool ok = false;
+  if (hx_status s = check_admissible(mesh, 0, &ok)) return s;
+  *admissible = ok;
   return HX_OK;
 }
 

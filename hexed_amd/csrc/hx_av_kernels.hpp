@@ -634,7 +634,7 @@ __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_admissible(Dev_mesh 
     if (!fin) atomicOr(&nonfinite[el], 1);
     for (int k = q; k < NF * NFQ; k += NQ) {
       const int f = k / NFQ, p = k % NFQ;
-      const double* fc = slot_ptr(m, m.face_slot[cls][e * NF + f]);
+      const double* fc = state_ptr(m, m.face_slot[cls][e * NF + f], m.alt_rd);
       bool ffin = true;
       for (int v = 0; v < NV; ++v) ffin = ffin && isfinite(fc[v * NFQ + p]);
       if (!(fc[ND * NFQ + p] > 0.) || !(fc[(ND + 1) * NFQ + p] > 0.)) atomicOr(&face_bad[el], 1 << f);
@@ -666,7 +666,7 @@ __global__ __launch_bounds__(256) void k_admissible_ref(Dev_mesh m, int* flags)
   for (int d = 0; d < ND - 1; ++d)
     if (m.ref_stretch[2 * i + d]) n_fine /= 2;
   if (f >= n_fine) return;
-  const double* fc = slot_ptr(m, m.ref_slot[5 * i + 1 + f]);
+  const double* fc = state_ptr(m, m.ref_slot[5 * i + 1 + f], m.alt_rd);
   bool fin = true;
   for (int v = 0; v < NV; ++v) fin = fin && isfinite(fc[v * NFQ + p]);
   if (!(fc[ND * NFQ + p] > 0.) || !(fc[(ND + 1) * NFQ + p] > 0.)) raise_flag(flags);

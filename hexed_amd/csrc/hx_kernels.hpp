@@ -2336,7 +2336,7 @@ struct Launchers
   }
   static hipError_t neighbor_reconcile(const Launch& l, int cls)
   {
-    if (l.fold) {
+    if (l.fold_ldg) {
       // folded into Reconcile_ldg_flux: only the connections touching a hanging-face mortar
       const int n = l.m.n_mortar_con[cls];
       if (n == 0) return hipSuccess;
@@ -2358,7 +2358,7 @@ struct Launchers
     if (n == 0) return hipSuccess;
     dim3 g(blocks_for(n, S::EPB)), b(S::BLOCK);
     const Eops<RS, double>& o = heops(l);
-    if (l.fold) {
+    if (l.fold_ldg) {
       if (cls == HX_DEFORMED)
         hipLaunchKernelGGL((k_reconcile_ldg<ND, RS, true, true>), g, b, 0, l.stream, l.m, o, dt, l.dtp, cr, uf);
       else

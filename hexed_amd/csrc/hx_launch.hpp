@@ -23,6 +23,7 @@ struct Launch
   const double* dtp; // device-resident time step the stage kernels multiply their coefficient by, or null
   Dt_final dtf;      // the time step state_bcs forms beside the boundary conditions (blocks == 0: none)
   int fold;          // face-flux folding: the Local computes its faces' fluxes, Neighbor covers only mortar connections
+  int fold_ldg;      // Reconcile_ldg_flux forms its jumps, Neighbor_reconcile covers only mortar connections
 };
 
 struct Kernel_set

@@ -114,8 +114,9 @@ class Device_mesh:
         self.ctx.check(self.lib.hx_mesh_set_precision(self.ptr, precision), "set_precision")
 
     def set_face_fold(self, mode):
-        """Whether update folds the face fluxes into the Local: 1 always, 0 never (Neighbor then Local, as the
-        reference sequences them), -1 where 2 n_dim <= row_size (the default)."""
+        """Whether update folds the face fluxes into the Local and the viscous jumps into Reconcile_ldg_flux: 1 both, 0
+        neither (Neighbor then Local, as the reference sequences them), -1 the fluxes always and the jumps where
+        2 n_dim <= row_size (the default)."""
         self.ctx.check(self.lib.hx_mesh_set_face_fold(self.ptr, int(mode)), "set_face_fold")
 
     def _field_array(self, name, cls):
