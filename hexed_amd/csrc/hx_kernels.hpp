@@ -24,10 +24,15 @@ struct Shape
   static constexpr int BLOCK = EPB * NQ;
   static constexpr int NFACE_DOF = 2 * ND * NV * NFQ;  // face values per element
   static constexpr int NRC = NV > RS ? NV : RS;         // residual-cache variables per point
-  // LDS copies of per-point arrays carry one pad slot after every row along the last dimension, so that the
-  // columns of that dimension (rows rs apart) fall on different banks
-  static constexpr int NQP = NQ + NQ / RS;
-  static __device__ int pad(int q) { return q + q / RS; }
+  // LDS copies of per-point arrays. Pairs of doubles are read and written 16 lanes at a time over 16 banks of 8 bytes,
+  // so rows (along the last dimension) of an even row size collide with each other and carry one pad slot; of an odd row
+  // size they spread over the banks as they are, and padding would put them an even pitch apart (whole Navier-Stokes
+  // steps, padded -> not: 3D row size 7 1124 -> 961 us, 5 515 -> 504; 2D row size 7 137 -> 119, 5 108 -> 105, 3 198 -> 186).
+  // 3D row size 3 keeps the pad: 727 us with, 735 without.
+  static constexpr int PITCH = RS % 2 && !(ND == 3 && RS == 3) ? RS : RS + 1;
+  static constexpr int NQP = NFQ * PITCH;
+  static __device__ int pad(int q) { return PITCH == RS ? q : q + q / RS; }
+  static __device__ int row_stride(int i_dim) { return i_dim == ND - 1 ? 1 : ipow(RS, ND - 2 - i_dim) * PITCH; }
 };
 
 template <int RS>
@@ -109,8 +114,7 @@ __device__ inline void for_columns(int i_dim, F&& f)
   using S = Shape<ND, RS>;
   using R = Row<ND, RS>;
   constexpr int PER = NVAR * S::NFQ, TOTAL = S::EPB * PER;
-  const int sd = R::stride(i_dim);
-  const int sdp = i_dim == ND - 1 ? 1 : sd + sd / RS;
+  const int sdp = S::row_stride(i_dim);
   if constexpr (UNIFORM) {
     for (int c0 = 0; c0 < TOTAL; c0 += NT) {
       const int c = c0 + int(threadIdx.x);
