@@ -120,7 +120,7 @@ __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_set_jacobian(Dev_mes
       const int e2 = blockIdx.x * EPB + el2;
       const double inv_h = 1. / m.nom_size[HX_DEFORMED][e2 < n ? e2 : n - 1];
       double xr[RS], y[RS];
-      load_row(b + L::POS + i * NQP + base, sd, xr);
+      for (int k = 0; k < RS; ++k) xr[k] = b[L::POS + i * NQP + base + k * sd];  // (pairs: 8% faster here than load_row)
       row_matvec(mc.diff, xr, y);
       double* out = b + L::JAC + (i * ND + j) * NQP + base;
 #pragma unroll
@@ -148,7 +148,7 @@ __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_set_jacobian(Dev_mes
       double FJ[2][ND * ND];
       for (int a = 0; a < ND * ND; ++a) {
         double xr[RS];
-        load_row(b + a * NQP, sd, xr);
+        for (int k = 0; k < RS; ++k) xr[k] = b[a * NQP + k * sd];
         for (int s = 0; s < 2; ++s) FJ[s][a] = row_bound(mc, s, xr);
       }
       const int* fs = m.face_slot[HX_DEFORMED] + size_t(e2) * 2 * ND + 2 * i_dim;
@@ -171,7 +171,7 @@ __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_set_jacobian(Dev_mes
       const double* in = lds + el2 * L::PER + src + a * RS * rest + r;
       double* out = lds + el2 * L::PER + dst + a * 2 * rest + r;
       double xr[RS];
-      load_row(in, rest, xr);
+      for (int k = 0; k < RS; ++k) xr[k] = in[k * rest];
       for (int s = 0; s < 2; ++s) out[s * rest] = row_bound(mc, s, xr);
     }
     const int next = src;
