@@ -13,7 +13,8 @@
 
 namespace hx {
 
-template <int ND, int RS>
+// F32: of a kernel that holds its rows in FP32
+template <int ND, int RS, bool F32 = false>
 struct Shape
 {
   static constexpr int NQ = ipow(RS, ND);
@@ -28,8 +29,9 @@ struct Shape
   // so rows (along the last dimension) of an even row size collide with each other and carry one pad slot; of an odd row
   // size they spread over the banks as they are, and padding would put them an even pitch apart (whole Navier-Stokes
   // steps, padded -> not: 3D row size 7 1124 -> 961 us, 5 515 -> 504; 2D row size 7 137 -> 119, 5 108 -> 105, 3 198 -> 186).
-  // 3D row size 3 keeps the pad: 727 us with, 735 without.
-  static constexpr int PITCH = RS % 2 && !(ND == 3 && RS == 3) ? RS : RS + 1;
+  // 3D row size 3 keeps the pad: 727 us with, 735 without. 3D row size 6 goes without where the rows are doubles: the pairs
+  // collide as often either way, and without it the in-place gradient of the Navier-Stokes Local fits the LDS four times.
+  static constexpr int PITCH = (RS % 2 && !(ND == 3 && RS == 3)) || (ND == 3 && RS == 6 && !F32) ? RS : RS + 1;
   static constexpr int NQP = NFQ * PITCH;
   static __device__ int pad(int q) { return PITCH == RS ? q : q + q / RS; }
   static __device__ int row_stride(int i_dim) { return i_dim == ND - 1 ? 1 : ipow(RS, ND - 2 - i_dim) * PITCH; }
@@ -108,10 +110,9 @@ constexpr int form_block()
 // qpoint), base the row's first point and sd its stride in the padded LDS layout (Row_index.hpp:14-64). With
 // UNIFORM, every thread takes part in each round (ok is false past the last column and the indices are then those of
 // column 0).
-template <int ND, int RS, int NVAR, int NT, bool UNIFORM, class F>
+template <int ND, int RS, int NVAR, int NT, bool UNIFORM, class S = Shape<ND, RS>, class F>
 __device__ inline void for_columns(int i_dim, F&& f)
 {
-  using S = Shape<ND, RS>;
   using R = Row<ND, RS>;
   constexpr int PER = NVAR * S::NFQ, TOTAL = S::EPB * PER;
   const int sdp = S::row_stride(i_dim);
@@ -136,14 +137,17 @@ __device__ inline void for_columns(int i_dim, F&& f)
 // of a direction collide half as often, each collision costs half as much, and the lanes served per cycle are the same
 // (deformed Navier-Stokes Local at 48^3, row size 6: 2.49 -> 2.29 ms per launch). Not where a value is read to be added to:
 // the loads keep their order among themselves, and there it exposes their latency (2.29 -> 2.32 ms).
+template <class T>
+__device__ __forceinline__ T lds_get(const T* p)
+{
+  if constexpr (std::is_same_v<T, double>) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  else return *p;
+}
 template <int RS, class T>
 __device__ inline void load_row(const T* p, int sd, T (&x)[RS])
 {
 #pragma unroll
-  for (int k = 0; k < RS; ++k) {
-    if constexpr (std::is_same_v<T, double>) x[k] = __hip_atomic_load(p + k * sd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    else x[k] = p[k * sd];
-  }
+  for (int k = 0; k < RS; ++k) x[k] = lds_get(p + k * sd);
 }
 
 // y = M x for an rs x rs matrix M
@@ -418,16 +422,15 @@ __device__ inline void lds_mfma_operands(const Eops<RS, double>* od, float* tab)
 
 // Modal filter of NVAR padded [NQP] arrays per element at `buf` (element stride `per`), in place, one direction at a
 // time (Spatial.hpp:472-481). Ends synchronized.
-template <int ND, int RS, int NVAR, int NT, class T>
+template <int ND, int RS, int NVAR, int NT, class S = Shape<ND, RS>, class T>
 __device__ inline void filter_columns(const Eops<RS, double>& o, T* buf, int per)
 {
-  using S = Shape<ND, RS>;
   T filt[RS][RS];
   for (int i = 0; i < RS; ++i)
     for (int k = 0; k < RS; ++k) filt[i][k] = T(o.filt[i][k]);
   for (int i = 0; i < ND; ++i) {
     __syncthreads();
-    for_columns<ND, RS, NVAR, NT, false>(i, [&](bool, int el, int v, int, int base, int sd) {
+    for_columns<ND, RS, NVAR, NT, false, S>(i, [&](bool, int el, int v, int, int base, int sd) {
       T* row = buf + el * per + v * S::NQP + base;
       T x[RS], y[RS];
       load_row(row, sd, x);
@@ -441,14 +444,13 @@ __device__ inline void filter_columns(const Eops<RS, double>& o, T* buf, int per
 
 // Write_face of the FP64 padded [NVAR][NQP] arrays at `buf` (element stride `per`) into block 0 of every face
 // (Spatial.hpp:29-71); slots(el2) points at the 2 ND face slots of element el2 of the workgroup
-template <int ND, int RS, int NT, int NVAR, class F>
+template <int ND, int RS, int NT, int NVAR, class S = Shape<ND, RS>, class F>
 __device__ inline void write_faces_to(const Dev_mesh& m, int cls, int blk, const Eops<RS, double>& o, const double* buf,
                                       int per, F&& slots)
 {
-  using S = Shape<ND, RS>;
   const int n = m.n_elem[cls];
   for (int i = 0; i < ND; ++i) {
-    for_columns<ND, RS, NVAR, NT, false>(i, [&](bool, int el, int v, int r, int base, int sd) {
+    for_columns<ND, RS, NVAR, NT, false, S>(i, [&](bool, int el, int v, int r, int base, int sd) {
       const int e = blk * S::EPB + el;
       if (e >= n) return;
       double x[RS];
@@ -810,7 +812,7 @@ __device__ inline double step_coef(double coef, const double* dtp) { return dtp 
 template <int ND, int RS, bool DEF, class P>
 struct Euler_lds
 {
-  using S = Shape<ND, RS>;
+  using S = Shape<ND, RS, P::mfma>;
   // arrays of T (padded)
   static constexpr int F = 0;                               // [NV][NQP] flux along the current direction
   static constexpr int RT = F + S::NV * S::NQP;             // [NV][NQP] time rate
@@ -874,7 +876,7 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
                                                  const double* __restrict__ dtp, int stage, int compute_residual,
                                                  int use_filter, const Dt_fuse& fuse, const Ops<RS>* __restrict__ gops)
 {
-  using S = Shape<ND, RS>;
+  using S = Shape<ND, RS, P::mfma>;
   using L = Euler_lds<ND, RS, DEF, P>;
   using T = typename P::T;
   constexpr int NQ = S::NQ, NQP = S::NQP, NFQ = S::NFQ, NV = S::NV, EPB = S::EPB, NT = euler_block<ND, RS>();
@@ -980,7 +982,7 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
     }
     __syncthreads();
     // -derivative(row_f, face_f) (Spatial.hpp:444-457)
-    for_columns<ND, RS, NV, NT, P::mfma>(i, [&](bool ok, int el2, int v, int r, int base, int sd) {
+    for_columns<ND, RS, NV, NT, P::mfma, S>(i, [&](bool ok, int el2, int v, int r, int base, int sd) {
       T* b = lt + el2 * L::PER_T;
       double* db = ld + el2 * L::PER_D;
       T y[RS];
@@ -996,8 +998,8 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
   if (t < EPB * 2 * ND) reinterpret_cast<int*>(ld + (t / (2 * ND)) * L::PER_D + L::TB_SLOT)[t % (2 * ND)] = slot;
   if (t < RS) ld[L::TB_NODE + t] = node;
   if (use_filter) {
-    filter_columns<ND, RS, NV, NT>(o, lt + L::RT, L::PER_T);
-    if constexpr (P::mfma && DEF) filter_columns<ND, RS, ND, NT>(o, ld + L::RP, L::PER_D);
+    filter_columns<ND, RS, NV, NT, S>(o, lt + L::RT, L::PER_T);
+    if constexpr (P::mfma && DEF) filter_columns<ND, RS, ND, NT, S>(o, ld + L::RP, L::PER_D);
   } else {
     __syncthreads();
   }
@@ -1038,7 +1040,7 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
   if (pt)
     for (int v = 0; v < NV; ++v) myd[L::U + v * NQP + qp] = u[v];
   __syncthreads();
-  write_faces_to<ND, RS, NT, NV>(m, cls, blk, o, ld + L::U, L::PER_D,
+  write_faces_to<ND, RS, NT, NV, S>(m, cls, blk, o, ld + L::U, L::PER_D,
                                  [&](int el2) { return reinterpret_cast<const int*>(ld + el2 * L::PER_D + L::TB_SLOT); });
   if (fused_dt && fuse.elem_scale[cls]) {
     // one wavefront per element takes its points' minimum (every wave of the workgroup is whole)
@@ -1095,17 +1097,17 @@ void k_local_euler(Dev_mesh m, Eops<RS, double> o, const Eops<RS, double>* od, d
 template <int ND, int RS, bool DEF, class P>
 struct Ns_lds
 {
-  using S = Shape<ND, RS>;
+  using S = Shape<ND, RS, P::mfma>;
   static constexpr int NQP = S::NQP, NFQ = S::NFQ, NV = S::NV;
-  // arrays of T (padded), gradient phase. FP64 form: the state, one gradient component and the column of the
-  // reference-level normals that component j needs, contracted row by row. FP32-MFMA form: the face-referenced
-  // products u n_ij of the directions i that contribute to one physical component j, contracted in place.
+  // arrays of T (padded), gradient phase: the products u n_ij (FP32-MFMA form: face-referenced) of the directions i that
+  // contribute to one physical component j, contracted in place: two barriers per component (with the state kept and the
+  // directions summed one by one in an array of their own there were four; 48^3, row size 6: 2.22 -> 2.14 ms per launch)
   static constexpr int NI = DEF ? ND : 1;                         // reference directions per physical component
-  static constexpr int U = 0;                                     // [NV][NQP] state (FP64 form)
-  static constexpr int G = U + NV * NQP;                          // [NV][NQP] one gradient component (FP64 form)
-  static constexpr int SN = G + NV * NQP;                         // [ND][NQP] normals n_ij of one j (FP64 form)
-  static constexpr int X = 0;                                     // [NI][NV][NQP] row operands (FP32-MFMA form)
-  static constexpr int P1_T = P::mfma ? NI * NV * NQP : SN + (DEF ? ND * NQP : 0);
+  // (FP64 on Cartesian elements keeps the operand, the state, for every component and has the derivatives elsewhere)
+  static constexpr bool IN_PLACE = P::mfma || DEF;
+  static constexpr int X = 0;                                     // [NI][NV][NQP] row operands
+  static constexpr int Y = IN_PLACE ? X : X + NV * NQP;           // [NI][NV][NQP] derivatives
+  static constexpr int P1_T = Y + NI * NV * NQP;
   // arrays of T (padded), residual phase. FP64 form: one rate array, the viscous rate moving to registers before the
   // convective pass (so that four workgroups of 3D row size 6 fit a compute unit's LDS); FP32-MFMA form: both rates.
   static constexpr int F = 0;                                     // [NV][NQP] viscous, then convective flux
@@ -1151,7 +1153,7 @@ void k_local_ns(Dev_mesh m, Eops<RS, double> o,
                 const Eops<RS, double>* od, Ns_params ns, double coef, const double* __restrict__ dtp,
                 int compute_residual, int use_filter)
 {
-  using S = Shape<ND, RS>;
+  using S = Shape<ND, RS, P::mfma>;
   using L = Ns_lds<ND, RS, DEF, P>;
   using T = typename P::T;
   constexpr int NQ = S::NQ, NQP = S::NQP, NFQ = S::NFQ, NV = S::NV, EPB = S::EPB, NT = form_block<ND, RS, P>();
@@ -1252,12 +1254,6 @@ void k_local_ns(Dev_mesh m, Eops<RS, double> o,
   const double nom = m.nom_size[cls][ec];
   const double det = DEF ? mt[ND * ND * NQ + q] : 1.;
   const T bulk = m.av[cls] ? T(bulk_d) : T(0), lap = m.av[cls] ? T(lap_d) : T(0);
-  if constexpr (!P::mfma)
-    if (pt) {
-      for (int v = 0; v < NV; ++v) my[L::U + v * NQP + qp] = T(u[v]);
-      if constexpr (DEF)
-        for (int i = 0; i < ND; ++i) my[L::SN + i * NQP + qp] = T(metd[i][0]);
-    }
   auto metric = [&](int i, int j) -> double {
     if constexpr (DEF) return metd[i][j];
     else return double(i == j);
@@ -1267,78 +1263,54 @@ void k_local_ns(Dev_mesh m, Eops<RS, double> o,
   // component j at a time
   const double inv_h = 1. / nom;
   T grad[NV][ND];
-  if constexpr (!P::mfma) {
-    for (int j = 0; j < ND; ++j) {
-      for (int i = DEF ? 0 : j; i < (DEF ? ND : j + 1); ++i) {
-        for_columns<ND, RS, NV, NT, false>(i, [&](bool ok, int el2, int v, int r, int base, int sd) {
-          T* b = lt + el2 * L::PER_T;
-          const double* db = ld + el2 * L::PER_D;
-          T x[RS], y[RS];
-          load_row(b + L::U + v * NQP + base, sd, x);
-          double b0 = db[L::SL + ((2 * i) * NV + v) * NFQ + r], b1 = db[L::SL + ((2 * i + 1) * NV + v) * NFQ + r];
-          if constexpr (DEF) {
-            T nk[RS];
-            load_row(b + L::SN + i * NQP + base, sd, nk);
-#pragma unroll
-            for (int k = 0; k < RS; ++k) x[k] *= nk[k];
-            b0 *= db[L::SFN + ((2 * i) * ND + j) * NFQ + r];
-            b1 *= db[L::SFN + ((2 * i + 1) * ND + j) * NFQ + r];
-          }
-          con.faces(x, b0, b1, y);
-          T* out = b + L::G + v * NQP + base;
-#pragma unroll
-          for (int k = 0; k < RS; ++k) out[k * sd] = (i == 0 || !DEF) ? y[k] : out[k * sd] + y[k];
-        });
-        __syncthreads();
-      }
-      for (int v = 0; v < NV; ++v) grad[v][j] = my[L::G + v * NQP + qp] * T(inv_h);
-      // the next component's column of the normals (every row of this one was read before the barrier above)
-      if constexpr (DEF)
-        if (pt && j + 1 < ND)
-          for (int i = 0; i < ND; ++i) my[L::SN + i * NQP + qp] = T(metric(i, j + 1));
-      __syncthreads();
-    }
-  } else {
-    for (int j = 0; j < ND; ++j) {
-      // u n_ij minus its value at the row's face 0 (face state times face normal), in FP64, then rounded
-      if (pt) {
-        const double* db = ld + el * L::PER_D;
-        for (int ii = 0; ii < L::NI; ++ii) {
-          const int i = DEF ? ii : j, r = Row<ND, RS>::fq(q, i);
-          const double nf = DEF ? db[L::SFN + ((2 * i) * ND + j) * NFQ + r] : 1.;
-          const double nq = metric(i, j);
-          for (int v = 0; v < NV; ++v)
-            my[L::X + (ii * NV + v) * NQP + qp] = T(u[v] * nq - db[L::SL + ((2 * i) * NV + v) * NFQ + r] * nf);
-        }
-      }
-      __syncthreads();
-      // every direction's rows in one pass, each row replaced by its derivative (a row is read and written by the
-      // one thread that owns it)
+  for (int j = 0; j < ND; ++j) {
+    // the row operands: u n_ij (Cartesian: u, once); FP32-MFMA form: minus its value at the row's face 0 (face state times
+    // face normal), in FP64, then rounded
+    if (pt && (j == 0 || L::IN_PLACE)) {
+      const double* db = ld + el * L::PER_D;
       for (int ii = 0; ii < L::NI; ++ii) {
         const int i = DEF ? ii : j;
-        for_columns<ND, RS, NV, NT, true>(i, [&](bool ok, int el2, int v, int r, int base, int sd) {
-          T* row = lt + el2 * L::PER_T + L::X + (ii * NV + v) * NQP + base;
-          const double* db = ld + el2 * L::PER_D;
-          double b0 = db[L::SL + ((2 * i) * NV + v) * NFQ + r], b1 = db[L::SL + ((2 * i + 1) * NV + v) * NFQ + r];
-          if constexpr (DEF) {
-            b0 *= db[L::SFN + ((2 * i) * ND + j) * NFQ + r];
-            b1 *= db[L::SFN + ((2 * i + 1) * ND + j) * NFQ + r];
-          }
-          T x[RS], y[RS];
-          load_row(row, sd, x);
-          con.faces(x, 0., b1 - b0, y);
-          if (ok)
+        const double nq = metric(i, j);
+        if constexpr (P::mfma) {
+          const int r = Row<ND, RS>::fq(q, i);
+          const double nf = DEF ? db[L::SFN + ((2 * i) * ND + j) * NFQ + r] : 1.;
+          for (int v = 0; v < NV; ++v)
+            my[L::X + (ii * NV + v) * NQP + qp] = T(u[v] * nq - db[L::SL + ((2 * i) * NV + v) * NFQ + r] * nf);
+        } else {
+          for (int v = 0; v < NV; ++v) my[L::X + (ii * NV + v) * NQP + qp] = DEF ? u[v] * nq : u[v];
+        }
+      }
+    }
+    __syncthreads();
+    // every direction's rows in one pass, each row's derivative in its place or in Y (a row is read and written by the
+    // one thread that owns it)
+    for (int ii = 0; ii < L::NI; ++ii) {
+      const int i = DEF ? ii : j;
+      for_columns<ND, RS, NV, NT, P::mfma, S>(i, [&](bool ok, int el2, int v, int r, int base, int sd) {
+        T* row = lt + el2 * L::PER_T + L::X + (ii * NV + v) * NQP + base;
+        const double* db = ld + el2 * L::PER_D;
+        double b0 = db[L::SL + ((2 * i) * NV + v) * NFQ + r], b1 = db[L::SL + ((2 * i + 1) * NV + v) * NFQ + r];
+        if constexpr (DEF) {
+          b0 *= db[L::SFN + ((2 * i) * ND + j) * NFQ + r];
+          b1 *= db[L::SFN + ((2 * i + 1) * ND + j) * NFQ + r];
+        }
+        T x[RS], y[RS];
+        load_row(row, sd, x);
+        con.faces(x, P::mfma ? 0. : b0, P::mfma ? b1 - b0 : b1, y);
+        if (ok)
 #pragma unroll
-            for (int k = 0; k < RS; ++k) row[k * sd] = y[k];
-        });
-      }
-      __syncthreads();
-      // (the next component's operands overwrite only this thread's own point)
-      for (int v = 0; v < NV; ++v) {
-        T g = 0;
-        for (int ii = 0; ii < L::NI; ++ii) g += my[L::X + (ii * NV + v) * NQP + qp];
-        grad[v][j] = g * T(inv_h);
-      }
+          for (int k = 0; k < RS; ++k) row[L::Y - L::X + k * sd] = y[k];
+      });
+      if constexpr (!P::mfma) __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();
+    // (the next component's operands overwrite only this thread's own point)
+    for (int v = 0; v < NV; ++v) {
+      T g = lds_get(my + L::Y + v * NQP + qp);
+      for (int ii = 1; ii < L::NI; ++ii) g += lds_get(my + L::Y + (ii * NV + v) * NQP + qp);
+      grad[v][j] = g * T(inv_h);
+      // (formed here: left to itself the compiler keeps the terms in registers until the flux needs the sum)
+      if constexpr (!P::mfma) asm volatile("" : "+v"(grad[v][j]));
     }
   }
   if constexpr (DEF) {
@@ -1379,7 +1351,7 @@ void k_local_ns(Dev_mesh m, Eops<RS, double> o,
         my[L::F + v * NQP + qp] = fv;
       }
     __syncthreads();
-    for_columns<ND, RS, NV, NT, P::mfma>(i, [&](bool ok, int el2, int v, int r, int base, int sd) {
+    for_columns<ND, RS, NV, NT, P::mfma, S>(i, [&](bool ok, int el2, int v, int r, int base, int sd) {
       T* b = lt + el2 * L::PER_T;
       T x[RS], y[RS], bx[2];
       load_row(b + L::F + v * NQP + base, sd, x);
@@ -1396,7 +1368,7 @@ void k_local_ns(Dev_mesh m, Eops<RS, double> o,
   // FP64 form: the viscous rate (filtered) moves to registers, its arrays take the convective rate
   T vrate[P::mfma ? 1 : NV];
   if constexpr (!P::mfma) {
-    if (use_filter) filter_columns<ND, RS, NV, NT>(o, lt + L::RV, L::PER_T);
+    if (use_filter) filter_columns<ND, RS, NV, NT, S>(o, lt + L::RV, L::PER_T);
     else __syncthreads();
     for (int v = 0; v < NV; ++v) vrate[v] = my[L::RV + v * NQP + qp];
   }
@@ -1413,7 +1385,7 @@ void k_local_ns(Dev_mesh m, Eops<RS, double> o,
       conv_point<ND, DEF, P>(u, p64, nrmd, ld + el * L::PER_D + L::SB + (2 * i) * NV * NFQ + Row<ND, RS>::fq(q, i), NFQ,
                              my + L::F + qp, ld + el * L::PER_D + L::PD + qp, NQP);
     __syncthreads();
-    for_columns<ND, RS, NV, NT, P::mfma>(i, [&](bool ok, int el2, int v, int r, int base, int sd) {
+    for_columns<ND, RS, NV, NT, P::mfma, S>(i, [&](bool ok, int el2, int v, int r, int base, int sd) {
       T* b = lt + el2 * L::PER_T;
       double* db = ld + el2 * L::PER_D;
       T y[RS];
@@ -1426,8 +1398,8 @@ void k_local_ns(Dev_mesh m, Eops<RS, double> o,
     });
   }
   if (use_filter) {
-    filter_columns<ND, RS, (P::mfma ? 2 : 1) * NV, NT>(o, lt + L::RT, L::PER_T);
-    if constexpr (P::mfma && DEF) filter_columns<ND, RS, ND, NT>(o, ld + L::RP, L::PER_D);
+    filter_columns<ND, RS, (P::mfma ? 2 : 1) * NV, NT, S>(o, lt + L::RT, L::PER_T);
+    if constexpr (P::mfma && DEF) filter_columns<ND, RS, ND, NT, S>(o, ld + L::RP, L::PER_D);
   } else {
     __syncthreads();
   }
