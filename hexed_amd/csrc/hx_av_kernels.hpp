@@ -143,8 +143,18 @@ struct Adv_lds
   static constexpr int PER = SB + 2 * RS * S::NFQ;
 };
 
+// the register target follows the waves per SIMD that the LDS allows (rounded up, at most 5): 3D row size 7, 16^3, 129 ->
+// 121 us per launch
+template <int ND, int RS>
+constexpr int adv_waves()
+{
+  constexpr int lds = Shape<ND, RS>::EPB * 8 * Adv_lds<ND, RS>::PER;
+  constexpr int w = ((163840 / lds) * ((Shape<ND, RS>::BLOCK + 63) / 64) + 3) / 4;
+  return w > 5 ? 5 : w;
+}
+
 template <int ND, int RS, bool DEF>
-__global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_adv_local(Dev_mesh m, Eops<RS, double> o, Av_consts<RS> ac,
+__global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) __attribute__((amdgpu_waves_per_eu(adv_waves<ND, RS>()))) void k_adv_local(Dev_mesh m, Eops<RS, double> o, Av_consts<RS> ac,
                                                                       double coef, int stage, int compute_residual,
                                                                       double advect_length, int project)
 {
@@ -152,8 +162,11 @@ __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_adv_local(Dev_mesh m
   using L = Adv_lds<ND, RS>;
   constexpr int NQ = S::NQ, NQP = S::NQP, NFQ = S::NFQ, EPB = S::EPB, NT = S::BLOCK;
   constexpr int cls = DEF ? HX_DEFORMED : HX_CARTESIAN;
+  // (the face slots go there where they cost no workgroup per compute unit: 3D row size 8 takes exactly half its LDS: 145 -> 114 us
+  // per launch at 14^3)
+  constexpr bool STAGE = 163840 / (EPB * (8 * L::PER + 8 * ND)) == 163840 / (EPB * 8 * L::PER);
   __shared__ double lds[EPB * L::PER];
-  __shared__ int fsl[EPB * 2 * ND];
+  __shared__ int fsl[STAGE ? EPB * 2 * ND : 1];
   const int t = threadIdx.x, el = t / NQ, q = t % NQ, qp = S::pad(q);
   const int n = m.n_elem[cls];
   const int e = blockIdx.x * EPB + el;
@@ -189,7 +202,7 @@ __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_adv_local(Dev_mesh m
     const I f(blockIdx.x, t, k);
     const double* s = slot_ptr(m, own[k]) + f.p;
     for (int v = 0; v < RS; ++v) sbr[k][v] = s[v * NFQ];
-    if (f.own && f.p == 0) fsl[f.el2 * 2 * ND + f.face] = own[k];
+    if (STAGE && f.own && f.p == 0) fsl[f.el2 * 2 * ND + f.face] = own[k];
   }
   // what the update at the end reads: requested ahead of the last direction's row phase
   double rcv[RS];
@@ -265,7 +278,9 @@ __global__ __launch_bounds__((Shape<ND, RS>::BLOCK)) void k_adv_local(Dev_mesh m
   for (int j = 0; j < ND; ++j) my[L::U + j * NQP + qp] = vel[j];
   for (int v = 0; v < RS; ++v) my[L::U + (ND + v) * NQP + qp] = a[v];
   __syncthreads();
-  write_faces_to<ND, RS, NT, ND + RS>(m, cls, blockIdx.x, o, lds + L::U, L::PER, [&](int el2) { return fsl + el2 * 2 * ND; });
+  write_faces_to<ND, RS, NT, ND + RS>(m, cls, blockIdx.x, o, lds + L::U, L::PER, [&](int el2) {
+    return STAGE ? fsl + el2 * 2 * ND : m.face_slot[cls] + size_t(blockIdx.x * EPB + el2) * 2 * ND;
+  });
 }
 
 // ---- Local<Smooth_art_visc / Fix_therm_admis> (Spatial.hpp:326-509, stage 0) -----------------------------------

@@ -28,10 +28,11 @@ struct Shape
   // LDS copies of per-point arrays. Pairs of doubles are read and written 16 lanes at a time over 16 banks of 8 bytes,
   // so rows (along the last dimension) of an even row size collide with each other and carry one pad slot; of an odd row
   // size they spread over the banks as they are, and padding would put them an even pitch apart (whole Navier-Stokes
-  // steps, padded -> not: 3D row size 7 1124 -> 961 us, 5 515 -> 504; 2D row size 7 137 -> 119, 5 108 -> 105, 3 198 -> 186).
-  // 3D row size 3 keeps the pad: 727 us with, 735 without. 3D row size 6 goes without where the rows are doubles: the pairs
-  // collide as often either way, and without it the in-place gradient of the Navier-Stokes Local fits the LDS four times.
-  static constexpr int PITCH = (RS % 2 && !(ND == 3 && RS == 3)) || (ND == 3 && RS == 6 && !F32) ? RS : RS + 1;
+  // steps, padded -> not: 3D row size 7 1124 -> 961 us, 5 515 -> 504, 3 716 -> 699; 2D row size 7 137 -> 119, 5 108 -> 105,
+  // 3 198 -> 186). Row size 2 goes without for the LDS it saves (two Navier-Stokes workgroups per compute unit, not one: 705 ->
+  // 559 us), as does 3D row size 6 where the rows are doubles (four workgroups with the in-place gradient; the pairs
+  // collide as often either way).
+  static constexpr int PITCH = RS % 2 || RS == 2 || (ND == 3 && RS == 6 && !F32) ? RS : RS + 1;
   static constexpr int NQP = NFQ * PITCH;
   static __device__ int pad(int q) { return PITCH == RS ? q : q + q / RS; }
   static __device__ int row_stride(int i_dim) { return i_dim == ND - 1 ? 1 : ipow(RS, ND - 2 - i_dim) * PITCH; }
@@ -842,7 +843,8 @@ constexpr int euler_block()
 }
 
 // Waves per SIMD that the workgroup's LDS allows (160 KB per CU, 4 SIMDs), at most 5: the register target given to
-// the compiler, so that registers do not lower the occupancy below what LDS permits. With face-flux folding, where a
+// the compiler, so that registers do not lower the occupancy below what LDS permits (rounded up: three workgroups of six
+// waves put five on two of the SIMDs; 3D row size 7, deformed, 210 -> 203 us per launch at 20^3). With face-flux folding, where a
 // thread computes more than one face point's flux, at most 4 (the registers of two face points' states and fluxes
 // would spill at 5), and so for the FP32-MFMA form at row sizes 7 and 8.
 template <int ND, int RS, bool DEF, class P, bool FOLD = false>
@@ -850,7 +852,7 @@ constexpr int euler_waves()
 {
   using L = Euler_lds<ND, RS, DEF, P>;
   constexpr int lds = Shape<ND, RS>::EPB * (int(sizeof(typename P::T)) * L::PER_T + 8 * L::PER_D);
-  constexpr int w = (163840 / lds) * (euler_block<ND, RS>() / 64) / 4;
+  constexpr int w = ((163840 / lds) * (euler_block<ND, RS>() / 64) + 3) / 4;
   constexpr bool two = FOLD && Shape<ND, RS>::EPB * 2 * ND * Shape<ND, RS>::NFQ > euler_block<ND, RS>();
   constexpr int cap = two || (P::mfma && RS >= 7) ? 4 : 5;
   return w < 1 ? 1 : (w > cap ? cap : w);
@@ -1135,14 +1137,17 @@ struct Ns_lds
   static constexpr int PER_D = SB_EARLY ? EARLY_D : LATE_D;
 };
 
-// waves per SIMD that the Navier-Stokes Local's LDS allows, at most 4 (3 for row sizes above 6, which spill at 4):
-// the register target follows it
+// waves per SIMD that the Navier-Stokes Local's LDS allows, at most 4 (3 for row sizes above 6, which spill at 4, and where a
+// thread of the 3D deformed FP32-MFMA form computes two face points' fluxes: row size 5, 30^3, 508 -> 352 us): the
+// register target follows it
 template <int ND, int RS, bool DEF, class P>
 constexpr int ns_waves()
 {
   using L = Ns_lds<ND, RS, DEF, P>;
   constexpr int lds = Shape<ND, RS>::EPB * (int(sizeof(typename P::T)) * L::PER_T + 8 * L::PER_D);
-  constexpr int w = (163840 / lds) * ((form_block<ND, RS, P>() + 63) / 64) / 4, cap = RS > 6 ? 3 : 4;
+  constexpr int w = (163840 / lds) * ((form_block<ND, RS, P>() + 63) / 64) / 4;
+  constexpr bool two = Shape<ND, RS>::EPB * 2 * ND * Shape<ND, RS>::NFQ > form_block<ND, RS, P>();
+  constexpr int cap = RS > 6 || (P::mfma && DEF && ND == 3 && two) ? 3 : 4;
   return w < 1 ? 1 : (w > cap ? cap : w);
 }
 
