@@ -17,19 +17,17 @@
 
 using namespace hx;
 
-// Scratch memory of hx_update_no_alloc, for callers that cannot allocate device memory: [0, 32) holds the reduction
-// words and the time step, [32, 32 + no_alloc_max_blocks) one fused Max_dt minimum per Euler Local workgroup (a mesh
-// of up to 262,144 workgroups: 262,144 elements at 3D row size 5 to 8). Each GPU holds its own copy (2 MiB) until the
-// process ends. Host code uses the address hipGetSymbolAddress returns for the current device (hx_ctx::scratch), never
-// the array's name.
+// Scratch memory of hx_update_no_alloc, for callers that cannot allocate device memory: one fused Max_dt minimum per
+// Euler Local workgroup (a mesh of up to 262,144 workgroups: 262,144 elements at 3D row size 5 to 8). Each GPU holds its
+// own copy (2 MiB) until the process ends. Host code uses the address hipGetSymbolAddress returns for the current device
+// (hx_ctx::scratch), never the array's name. Every context of a GPU shares it (Scratch_use); the reduction words and the
+// time step, which the stage kernels read after the call has returned, are the context's (hx_ctx::scalar).
 namespace {
 constexpr long long no_alloc_max_blocks = 1LL << 18;
-constexpr long long scratch_minima_offset = 32;
-constexpr int scratch_step_offset = 8 + dt_final_blocks;  // the step's Step_dev, after the reduction words
-static_assert(scratch_step_offset + sizeof(Step_dev) / sizeof(double) <= scratch_minima_offset, "the words fit");
-constexpr int ctx_words = 8 + dt_final_blocks;
+constexpr int ctx_step_offset = 8 + dt_final_blocks;  // the synchronous updates' Step_dev, after the reduction words
+constexpr int ctx_words = ctx_step_offset + int(sizeof(Step_dev) / sizeof(double));
 }  // namespace
-static __device__ __align__(256) double scratch[scratch_minima_offset + no_alloc_max_blocks];
+static __device__ __align__(256) double scratch[no_alloc_max_blocks];
 
 namespace {
 constexpr int max_devices = 64;
@@ -74,7 +72,9 @@ struct hx_ctx
   std::vector<char> host_ops[HX_MAX_ROW_SIZE + 1];  // host copies, for kernels taking constants by value
   std::vector<char> host_eops[HX_MAX_ROW_SIZE + 1];
   void* eops[HX_MAX_ROW_SIZE + 1] = {};             // device Eops<rs, double> tables
-  double* scalar = nullptr;             // device words for reductions (ctx_words of them, Dt_final::scalar)
+  // device words (ctx_words of them): the reductions' (Dt_final::scalar), then the step of the synchronous updates, whose
+  // stage kernels read it in stream order
+  double* scalar = nullptr;
   // pinned host memory: [0..4) readbacks, [4] the time step and [5] its sequence number (Dt_final::host), [6] the two flags
   // of the admissibility check
   double* host_scalar = nullptr;
@@ -151,12 +151,9 @@ struct hx_mesh
   // hx_update_async: the device status, the time step the stage kernels read while an update is enqueued with it
   // (null otherwise), and the captured steady-state update with the options and form it was captured for
   Step_dev* step = nullptr;
-  Step_dev* sync_step = nullptr;   // hx_update's own, of which it uses dt only
   const double* dt_dev = nullptr;
-  // the reduction scalar the mesh's calls use: the context's, or the file-scope scratch array during
-  // hx_update_no_alloc; and the scratch epoch of the last hx_update_no_alloc on this mesh (its fused minima sit in the
-  // scratch array and are current only while no other call has used the array since)
-  double* scalar = nullptr;
+  // the scratch epoch of the last hx_update_no_alloc on this mesh (its fused minima sit in the scratch array and are
+  // current only while no other call has used the array since)
   long long scratch_epoch = -1;
   int n_groups = 0;  // groups (hx_group) holding the mesh, which must be destroyed first
   // face-flux folding of the current stage of an update (Dev_mesh::partner): the buffer holding the face states the
@@ -251,7 +248,7 @@ void release_mesh_memory(hx_mesh* mesh)
   if (mesh->case_host) (void)hipHostFree(mesh->case_host);
   mesh->case_host = nullptr;
   mesh->dt_block_min = nullptr;
-  mesh->step = mesh->sync_step = nullptr;
+  mesh->step = nullptr;
   mesh->dtf = Dt_final{};
   mesh->dt_dev = nullptr;
   mesh->fuse = Dt_fuse{};
@@ -552,7 +549,7 @@ Launch make_launch(hx_mesh* mesh, bool writes = true)
   l.hops = mesh->ctx->host_ops[mesh->dm.rs].data();
   l.eops = mesh->ctx->eops[mesh->dm.rs];
   l.heops = mesh->ctx->host_eops[mesh->dm.rs].data();
-  l.scalar = mesh->scalar ? mesh->scalar : mesh->ctx->scalar;
+  l.scalar = mesh->ctx->scalar;
   l.precision = mesh->precision;
   l.fuse = mesh->fuse;
   l.dtf = mesh->dtf;
@@ -1530,7 +1527,6 @@ struct Update_setup
   double* block_min; // the fused per-workgroup minima: the mesh's buffer, or the scratch array
   long long n_blocks;
   bool in_scratch;
-  double* scalar;    // the reduction words (Dt_final::scalar)
   Step_dev* step;    // where the time step is formed on the device
 };
 
@@ -1541,8 +1537,8 @@ long long euler_local_blocks(const hx_mesh* mesh)
   return (mesh->dm.n_elem[0] + epb - 1) / epb + (mesh->dm.n_elem[1] + epb - 1) / epb;
 }
 
-// no_alloc: the minima, the reduction words and the time step go to the file-scope scratch array, and nothing is
-// allocated; `async`: the time step and the status it advances are those of hx_update_async
+// no_alloc: the minima go to the file-scope scratch array, and nothing is allocated; `async`: the time step and the status
+// it advances are those of hx_update_async, else the time step is the context's
 hx_status update_setup(hx_mesh* mesh, const hx_update_options* o, Update_setup* u, bool no_alloc = false,
                        bool async = false)
 {
@@ -1556,20 +1552,8 @@ hx_status update_setup(hx_mesh* mesh, const hx_update_options* o, Update_setup* 
     if (u->fusable && u->n_blocks > no_alloc_max_blocks)
       return fail(ctx, HX_ERR_INVALID, "mesh too large for hx_update_no_alloc: " + std::to_string(u->n_blocks) +
                                            " Euler Local workgroups, at most " + std::to_string(no_alloc_max_blocks));
-    u->block_min = ctx->scratch + scratch_minima_offset;
-    u->scalar = ctx->scratch;
-    u->step = reinterpret_cast<Step_dev*>(ctx->scratch + scratch_step_offset);
+    u->block_min = ctx->scratch;
   } else {
-    Step_dev*& step = async ? mesh->step : mesh->sync_step;
-    if (!step) {
-      void* p = nullptr;
-      HX_TRY(ctx, hipMalloc(&p, sizeof(Step_dev)), "hipMalloc(update status)");
-      mesh->allocs.push_back(p);
-      step = static_cast<Step_dev*>(p);
-      hipLaunchKernelGGL(k_set_status, dim3(1), dim3(1), 0, ctx->stream, step, 0., 0., 0LL);
-      HX_TRY(ctx, hipGetLastError(), "status");
-    }
-    u->step = step;
     if (u->fusable && !mesh->dt_block_min) {
       mesh->n_dt_blocks = u->n_blocks;
       void* p = nullptr;
@@ -1578,7 +1562,18 @@ hx_status update_setup(hx_mesh* mesh, const hx_update_options* o, Update_setup* 
       mesh->dt_block_min = static_cast<double*>(p);
     }
     u->block_min = mesh->dt_block_min;
-    u->scalar = ctx->scalar;
+  }
+  u->step = reinterpret_cast<Step_dev*>(ctx->scalar + ctx_step_offset);
+  if (async) {
+    if (!mesh->step) {
+      void* p = nullptr;
+      HX_TRY(ctx, hipMalloc(&p, sizeof(Step_dev)), "hipMalloc(update status)");
+      mesh->allocs.push_back(p);
+      mesh->step = static_cast<Step_dev*>(p);
+      hipLaunchKernelGGL(k_set_status, dim3(1), dim3(1), 0, ctx->stream, mesh->step, 0., 0., 0LL);
+      HX_TRY(ctx, hipGetLastError(), "status");
+    }
+    u->step = mesh->step;
   }
   u->n_cheby = o->n_cheby_flow;
   const double max_cheby = cheby_step(u->n_cheby, u->n_cheby - 1);
@@ -1628,7 +1623,7 @@ hx_status enqueue_max_dt(hx_mesh* mesh, const hx_update_options* o, const Update
   const double max_cfl_c = hx_basis_max_cfl(mesh->dm.rs) * u.msc;
   const double max_cfl_d = -2 / hx_basis_tables::eigenvalss[mesh->dm.rs - 2][1] * u.msd;
   if (!o->local_time) {
-    hipLaunchKernelGGL(k_fill, dim3(1), dim3(1), 0, ctx->stream, u.scalar, DBL_MAX);
+    hipLaunchKernelGGL(k_fill, dim3(1), dim3(1), 0, ctx->stream, ctx->scalar, DBL_MAX);
     HX_TRY(ctx, hipGetLastError(), "fill");
   }
   for (int cls = 0; cls < 2; ++cls) {
@@ -1738,10 +1733,10 @@ hx_status update_once(hx_mesh* mesh, const hx_update_options* o, const Update_se
         if ((s = enqueue_max_dt(mesh, o, u))) return s;
       Dt_final f{};
       if (device_dt) {
-        f.v = pending ? u.block_min : u.scalar;
+        f.v = pending ? u.block_min : ctx->scalar;
         f.n = o->local_time ? 0 : pending ? u.n_blocks : 1;
         f.blocks = dt_blocks_for(f.n);
-        f.scalar = u.scalar;
+        f.scalar = ctx->scalar;
         f.unit = o->local_time;
         f.max_time_step = o->max_time_step;
         f.cheby = cheby;
@@ -1906,22 +1901,14 @@ hx_status hx_update_no_alloc(hx_mesh* mesh, const hx_update_options* o, hx_updat
   bool pending = fused_pending(mesh, o, u);
   mesh->scratch_epoch = ++scratch_epochs[ctx->device];
   mesh->dt_cache.valid = false;
-  // the kernels' reduction scalar is the array's, and no event is created for timing
+  // no event is created for timing
   struct Scoped
   {
-    hx_mesh* mesh;
+    hx_ctx* ctx;
     bool events;
-    Scoped(hx_mesh* m) : mesh{m}, events{m->ctx->events_off}
-    {
-      mesh->scalar = mesh->ctx->scratch;
-      mesh->ctx->events_off = true;
-    }
-    ~Scoped()
-    {
-      mesh->scalar = nullptr;
-      mesh->ctx->events_off = events;
-    }
-  } scoped(mesh);
+    Scoped(hx_ctx* c) : ctx{c}, events{c->events_off} { ctx->events_off = true; }
+    ~Scoped() { ctx->events_off = events; }
+  } scoped(ctx);
   if (hx_status s = update_once(mesh, o, u, st, pending)) return s;
   if (u.fusable && pending) remember_fused(mesh, o, u);
   return HX_OK;

@@ -1,0 +1,54 @@
+"""The host code around the kernels on a HIP runtime without a device (tests/cpp/fake_hip.cpp): which calls an entry point
+makes, in which order, and on an error. Each script runs in a process of its own, since the runtime is chosen when the
+library is loaded; kernels do not run there, so no results are compared."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PRELUDE = """
+import ctypes, sys
+sys.path[:0] = [{root!r}, {here!r}]
+fake = ctypes.CDLL({lib!r}, ctypes.RTLD_GLOBAL)
+fake.fake_log.restype = ctypes.c_char_p
+import numpy as np
+from hexed_amd import abi, configs, mesh
+from hexed_amd.device import Context, Device_group, Device_mesh
+def calls():
+    out = fake.fake_log().decode().splitlines()
+    fake.fake_clear()
+    return out
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("fake") / "libamdhip64.so.7")
+    subprocess.run(["g++", "-O1", "-std=c++20", "-Wall", "-fPIC", "-shared", "-Wl,-soname,libamdhip64.so.7", "-o", lib,
+                    os.path.join(HERE, "cpp", "fake_hip.cpp")], check=True)
+
+    def script(text):
+        code = PRELUDE.format(root=os.path.dirname(HERE), here=HERE, lib=lib) + text
+        r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, f"status {r.returncode}\n{r.stdout}\n{r.stderr}"
+    return script
+
+
+def test_no_alloc_contexts_have_their_own_time_step(run):
+    """The stage kernels of hx_update_no_alloc read the time step after the call has returned, so a second context of the
+    GPU, on a stream of its own, must not form its time step in the same place."""
+    run("""
+seen = []
+for c in [Context(0), Context(0)]:
+    dev = Device_mesh(c, configs.euler_box(2, 4, seed=1))
+    st = abi.hx_update_status()
+    calls()
+    dev.lib.hx_update_no_alloc(dev.ptr, ctypes.byref(abi.update_options()), ctypes.byref(st))
+    at = {x for x in calls() if x.startswith("time step ")}
+    assert len(at) == 1 and at != {"time step (nil)"}, at
+    seen += at
+assert seen[0] != seen[1], seen
+""")

@@ -86,6 +86,30 @@ def test_no_alloc_two_meshes_share_the_array(ctx):
         d.close()
 
 
+def test_no_alloc_two_contexts_share_the_array(ctx):
+    """Two contexts of one GPU, each with a stream of its own, stepped alternately without a wait in between: the stages of
+    a call, the larger mesh's well over those of the smaller one, run beside the other context's next calls."""
+    say("[gpu] hx_update_no_alloc on two contexts stepped alternately")
+    opts = abi.update_options(max_safety=0.6)
+    other = Context(0)
+    m1, a1, b1 = twins(ctx, configs.euler_box(4, 5, mach=0.5, seed=5))
+    m2, a2, b2 = twins(other, configs.euler_box(24, 6, mach=0.8, seed=6))
+    s = [abi.hx_update_status() for _ in range(4)]
+    # the small mesh is stepped once, then several times, between two steps of the large one
+    order = [1, 2, 1, 1, 2, 1, 2, 2, 1, 1, 1, 2, 1]
+    for k in order:
+        no_alloc_update(b1 if k == 1 else b2, opts, s[1 if k == 1 else 3])
+    for k in order:
+        (a1 if k == 1 else a2).update(opts, s[0 if k == 1 else 2])
+    assert (s[0].time_step, s[0].flow_time) == (s[1].time_step, s[1].flow_time)
+    assert (s[2].time_step, s[2].flow_time) == (s[3].time_step, s[3].flow_time)
+    assert_same("two contexts, small", m1, a1, b1)
+    assert_same("two contexts, large", m2, a2, b2)
+    for d in (a1, b1, a2, b2):
+        d.close()
+    other.close()
+
+
 def test_no_alloc_rejects_the_fix(ctx):
     say("[gpu] hx_update_no_alloc rejects fix_admis")
     m = configs.euler_box(2, 4, seed=1)
