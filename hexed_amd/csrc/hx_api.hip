@@ -29,6 +29,8 @@ constexpr int ctx_words = ctx_step_offset + int(sizeof(Step_dev) / sizeof(double
 }  // namespace
 static __device__ __align__(256) double scratch[no_alloc_max_blocks];
 
+struct hx_ctx;
+
 namespace {
 constexpr int max_devices = 64;
 std::mutex scratch_mutex;
@@ -61,6 +63,14 @@ double* scratch_on(int device, hipError_t* err)
 }
 
 long long scratch_epoch(int device) { return scratch_epochs[device].load(); }
+
+// The context whose work may use the minima in each device's scratch array, and whether a call of it is under way
+struct
+{
+  const hx_ctx* owner = nullptr;
+  hipStream_t stream = nullptr;
+  bool in_call = false;
+} scratch_user[max_devices];
 }  // namespace
 
 struct hx_ctx
@@ -101,6 +111,37 @@ struct hx_ctx
   double* scratch = nullptr;     // this device's address of the file-scope scratch array (hx_update_no_alloc)
   hipError_t scratch_err = hipSuccess;
 };
+
+namespace {
+// A call's use of the minima in the scratch array, for its scope. Granted to the context that used them last, and to
+// another once that one's stream has run dry: the stages of a call run on after it returns, so that two contexts would
+// otherwise write the minima at the same time. A call without a grant runs Max_dt itself and leaves no minima.
+struct Scratch_use
+{
+  const hx_ctx* ctx;
+  bool granted;
+  Scratch_use(const hx_ctx* c) : ctx{c}
+  {
+    std::lock_guard<std::mutex> lock(scratch_mutex);
+    auto& u = scratch_user[ctx->device];
+    granted = !u.owner || u.owner == ctx || (!u.in_call && hipStreamQuery(u.stream) == hipSuccess);
+    if (granted) u = {ctx, ctx->stream, true};
+  }
+  ~Scratch_use()
+  {
+    if (!granted) return;
+    std::lock_guard<std::mutex> lock(scratch_mutex);
+    scratch_user[ctx->device].in_call = false;
+  }
+  Scratch_use(const Scratch_use&) = delete;
+  Scratch_use& operator=(const Scratch_use&) = delete;
+  static void release(const hx_ctx* ctx)  // the context's stream is about to go
+  {
+    std::lock_guard<std::mutex> lock(scratch_mutex);
+    if (scratch_user[ctx->device].owner == ctx) scratch_user[ctx->device] = {};
+  }
+};
+}  // namespace
 
 struct hx_mesh
 {
@@ -944,6 +985,7 @@ hx_status hx_ctx_destroy(hx_ctx* ctx)
   if (!ctx) return HX_OK;
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
+  Scratch_use::release(ctx);
   // meshes still alive are detached: their device memory is freed now, their handles stay valid for
   // hx_mesh_destroy, and every other call on them fails with HX_ERR_INVALID
   for (hx_group* g : ctx->groups) release_group(g);
@@ -1898,8 +1940,10 @@ hx_status hx_update_no_alloc(hx_mesh* mesh, const hx_update_options* o, hx_updat
     return fail(ctx, HX_ERR_UNSUPPORTED, "the admissibility fix allocates its flags; use hx_update");
   Update_setup u;
   if (hx_status s = update_setup(mesh, o, &u, true)) return s;
+  const Scratch_use use(ctx);
+  u.fusable = u.fusable && use.granted;
   bool pending = fused_pending(mesh, o, u);
-  mesh->scratch_epoch = ++scratch_epochs[ctx->device];
+  if (use.granted) mesh->scratch_epoch = ++scratch_epochs[ctx->device];
   mesh->dt_cache.valid = false;
   // no event is created for timing
   struct Scoped

@@ -380,9 +380,11 @@ hx_status hx_update_async(hx_mesh* mesh, const hx_update_options* opts, int n_up
  * minimum of every Euler Local workgroup in a file-scope device array of 262,144 doubles (2 MiB per GPU, held until the
  * process ends) instead of memory the library allocates.
  * Meshes with more than 262,144 Euler Local workgroups (elements / max(1, 256 / row_size^n_dim), both classes) are
- * rejected with HX_ERR_INVALID; fix_admis is rejected with HX_ERR_UNSUPPORTED (the fix allocates its flags). Every
- * call on one GPU shares the array: the fused Max_dt minima a call leaves are used by the mesh's next call only if no
- * other call used the array in between, and calls that overlap on one GPU race. No timing events are recorded. */
+ * rejected with HX_ERR_INVALID; fix_admis is rejected with HX_ERR_UNSUPPORTED (the fix may allocate artificial viscosity).
+ * Every call on one GPU shares the array: the fused Max_dt minima a call leaves are used by the mesh's next call only if no
+ * other call used the array in between, and a call that finds another context's work with the array unfinished runs
+ * Max_dt itself and leaves no minima. So contexts may call it in turn, or from a thread each, without waiting for each
+ * other; everything else a call uses is its context's or its mesh's. No timing events are recorded. */
 hx_status hx_update_no_alloc(hx_mesh* mesh, const hx_update_options* opts, hx_update_status* status);
 /* Waits for the mesh's stream and writes the device status of hx_update_async into `status` (time_step, flow_time,
  * iteration; fix_admis_iters is left as it is). */

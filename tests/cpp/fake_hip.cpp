@@ -15,6 +15,7 @@ std::map<const void*, std::string> kernels;
 std::map<void*, std::pair<void*, size_t>> blocks;  // address handed out -> mapping
 std::map<const void*, void*> symbols;
 int fail_after[2] = {-1, -1};  // calls of each kind (0 copy, 1 launch) that still succeed; -1 all
+int busy = 0;                  // stream queries that still find work
 int last_error = 0;
 
 void note(const std::string& s) { log_text += s + "\n"; }
@@ -63,6 +64,7 @@ extern "C" {
 const char* fake_log() { return log_text.c_str(); }
 void fake_clear() { log_text.clear(); }
 void fake_fail(int kind, int after) { fail_after[kind] = after; }
+void fake_busy(int queries) { busy = queries; }
 
 void* __hipRegisterFatBinary(const void*)
 {
@@ -124,15 +126,19 @@ int hipLaunchKernel(const void* f, Dim, Dim, void** args, size_t, void*)
 {
   if (fails(1)) return last_error = 1;
   note("launch " + kernels[f]);
-  // k_local_euler(mesh, operators by value, device operators, coefficient, device time step, ...)
-  if (kernels[f].find("k_local_euler") != std::string::npos) note("time step " + hex(*static_cast<void**>(args[4])));
+  // k_local_euler(mesh, operators by value, device operators, coefficient, device time step, stage, residual, filter,
+  // Dt_fuse {minima, ...}, ...)
+  if (kernels[f].find("k_local_euler") != std::string::npos) {
+    note("time step " + hex(*static_cast<void**>(args[4])));
+    note("minima " + hex(*static_cast<void**>(args[8])));
+  }
   return 0;
 }
 int hipStreamCreateWithFlags(void** s, unsigned) { return *s = new char, 0; }
 int hipStreamDestroy(void* s) { return delete static_cast<char*>(s), 0; }
 int hipStreamSynchronize(void*) { return note("wait"), 0; }
 int hipDeviceSynchronize() { return note("wait"), 0; }
-int hipStreamQuery(void*) { return note("query"), 0; }
+int hipStreamQuery(void*) { return busy > 0 ? (--busy, 600) : 0; }  // hipErrorNotReady
 int hipStreamBeginCapture(void*, int) { return 1; }
 int hipStreamEndCapture(void*, void**) { return 1; }
 int hipGraphInstantiate(void**, void*, void*, char*, size_t) { return 1; }

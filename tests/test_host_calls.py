@@ -52,3 +52,28 @@ for c in [Context(0), Context(0)]:
     seen += at
 assert seen[0] != seen[1], seen
 """)
+
+
+def test_no_alloc_minima_have_one_writer(run):
+    """The minima in the array that all contexts of a GPU share: a context leaves none there while another one's work with
+    the array is unfinished, and uses none that another has written since."""
+    run("""
+def minima(dev):
+    calls()
+    dev.lib.hx_update_no_alloc(dev.ptr, ctypes.byref(abi.update_options()), ctypes.byref(abi.hx_update_status()))
+    log = calls()
+    return [x for x in log if x.startswith("minima")], any("k_max_dt" in x for x in log)
+a, b = Context(0), Context(0)
+da, db = (Device_mesh(c, configs.euler_box(2, 4, seed=1)) for c in (a, b))
+kept = minima(da)[0]
+assert kept[0] == "minima (nil)" and kept[1] != "minima (nil)", kept
+fake.fake_busy(1)  # a's stages are running
+assert minima(db) == (["minima (nil)"] * 2, True)
+fake.fake_busy(1)  # its own unfinished work is no obstacle
+assert minima(da)[0] == kept
+assert minima(db) == (kept, True)
+fake.fake_busy(1)
+assert minima(da) == (["minima (nil)"] * 2, True)
+b.close()
+assert minima(da) == (kept, True)
+""")
