@@ -1378,10 +1378,11 @@ hx_status hx_reconcile_ldg_flux(hx_mesh* mesh, int cls, const hx_pde* pde, doubl
   return HX_OK;
 }
 
-hx_status hx_max_dt(hx_mesh* mesh, int cls, const hx_pde* pde, int is_local, int, double safety_conv, double safety_diff,
-                    double* dt_out)
+// Max_dt of one class. With local time stepping the result is 1 whatever the device holds, and this does not wait for the
+// time step scale.
+static hx_status max_dt_class(hx_mesh* mesh, int cls, const hx_pde* pde, int is_local, double safety_conv, double safety_diff,
+                              double* dt_out)
 {
-  if (!live(mesh) || !valid_cls(cls) || !dt_out) return HX_ERR_INVALID;
   Launch l = make_launch(mesh);
   bool visc;
   if (hx_status s = pde_check(mesh, pde, &visc, &l)) return s;
@@ -1401,13 +1402,38 @@ hx_status hx_max_dt(hx_mesh* mesh, int cls, const hx_pde* pde, int is_local, int
              "max_dt");
     else HX_TRY(mesh->ctx, mesh->ks->max_dt(l, cls, visc, is_local, max_cfl_c, max_cfl_d), "max_dt");
   }
-  // with local time stepping the result is 1 whatever the device holds: nothing to wait for
   if (is_local) return HX_OK;
   HX_TRY(mesh->ctx, hipMemcpyAsync(mesh->ctx->host_scalar, l.scalar, sizeof(double), hipMemcpyDeviceToHost, l.stream),
          "max_dt readback");
   HX_TRY(mesh->ctx, hipStreamSynchronize(l.stream), "max_dt sync");
   *dt_out = *mesh->ctx->host_scalar;
   return HX_OK;
+}
+
+// ... of both classes, the smaller
+static hx_status max_dt_classes(hx_mesh* mesh, const hx_pde* pde, int is_local, double safety_conv, double safety_diff,
+                                double* dt_out)
+{
+  double a, b;
+  if (hx_status s = max_dt_class(mesh, HX_CARTESIAN, pde, is_local, safety_conv, safety_diff, &a)) return s;
+  if (hx_status s = max_dt_class(mesh, HX_DEFORMED, pde, is_local, safety_conv, safety_diff, &b)) return s;
+  *dt_out = std::min(a, b);
+  return HX_OK;
+}
+
+// the entry points end with the stream run dry: a caller may read the time step scale from any stream
+static hx_status max_dt_wait(hx_mesh* mesh)
+{
+  HX_TRY(mesh->ctx, hipStreamSynchronize(mesh->ctx->stream), "max_dt sync");
+  return HX_OK;
+}
+
+hx_status hx_max_dt(hx_mesh* mesh, int cls, const hx_pde* pde, int is_local, int, double safety_conv, double safety_diff,
+                    double* dt_out)
+{
+  if (!live(mesh) || !valid_cls(cls) || !dt_out) return HX_ERR_INVALID;
+  if (hx_status s = max_dt_class(mesh, cls, pde, is_local, safety_conv, safety_diff, dt_out)) return s;
+  return max_dt_wait(mesh);
 }
 
 hx_status hx_prolong_refined(hx_mesh* mesh, const hx_pde* pde, int scale, int offset)
@@ -1497,21 +1523,16 @@ hx_status hx_compute_navier_stokes(hx_mesh* mesh, const hx_kernel_options* o, hx
   return hx_prolong_refined(mesh, &p, 0, 0);
 }
 
-hx_status hx_max_dt_euler(hx_mesh* mesh, const hx_kernel_options* o, double msc, double msd, int local_time, double* dt_out)
+hx_status hx_max_dt_euler(hx_mesh* mesh, const hx_kernel_options*, double msc, double msd, int local_time, double* dt_out)
 {
   if (!live(mesh) || !dt_out) return HX_ERR_INVALID;
   hx_pde p{};
   p.kind = HX_PDE_EULER;
-  double a, b;
-  hx_status s;
-  const int uf = o ? o->use_filter : 0;
-  if ((s = hx_max_dt(mesh, HX_CARTESIAN, &p, local_time, uf, msc, msd, &a))) return s;
-  if ((s = hx_max_dt(mesh, HX_DEFORMED, &p, local_time, uf, msc, msd, &b))) return s;
-  *dt_out = std::min(a, b);
-  return HX_OK;
+  if (hx_status s = max_dt_classes(mesh, &p, local_time, msc, msd, dt_out)) return s;
+  return max_dt_wait(mesh);
 }
 
-hx_status hx_max_dt_navier_stokes(hx_mesh* mesh, const hx_kernel_options* o, double msc, double msd, int local_time,
+hx_status hx_max_dt_navier_stokes(hx_mesh* mesh, const hx_kernel_options*, double msc, double msd, int local_time,
                                   hx_transport visc, hx_transport cond, double* dt_out)
 {
   if (!live(mesh) || !dt_out) return HX_ERR_INVALID;
@@ -1519,13 +1540,8 @@ hx_status hx_max_dt_navier_stokes(hx_mesh* mesh, const hx_kernel_options* o, dou
   p.kind = HX_PDE_NAVIER_STOKES;
   p.visc = visc;
   p.cond = cond;
-  double a, b;
-  hx_status s;
-  const int uf = o ? o->use_filter : 0;
-  if ((s = hx_max_dt(mesh, HX_CARTESIAN, &p, local_time, uf, msc, msd, &a))) return s;
-  if ((s = hx_max_dt(mesh, HX_DEFORMED, &p, local_time, uf, msc, msd, &b))) return s;
-  *dt_out = std::min(a, b);
-  return HX_OK;
+  if (hx_status s = max_dt_classes(mesh, &p, local_time, msc, msd, dt_out)) return s;
+  return max_dt_wait(mesh);
 }
 
 hx_status hx_compute_write_face(hx_mesh* mesh)
@@ -2281,6 +2297,7 @@ hx_status hx_update_cases(hx_mesh* mesh, const hx_update_options* o, hx_update_s
       st[k].flow_time += one.flow_time;
       st[k].iteration += one.iteration;
     }
+    HX_TRY(ctx, hipStreamSynchronize(ctx->stream), "update sync");
     return HX_OK;
   }
   Cases_step c;
@@ -2312,6 +2329,7 @@ hx_status hx_update_cases(hx_mesh* mesh, const hx_update_options* o, hx_update_s
     }
   }
   cases_end(mesh, o, c, pending, st);
+  HX_TRY(ctx, hipStreamSynchronize(ctx->stream), "update sync");
   return HX_OK;
 }
 
@@ -2574,6 +2592,7 @@ hx_status hx_group_update(hx_group* g, const hx_update_options* o, hx_update_sta
     }
   }
   for (int k = 0, off = 0; k < n; off += g->meshes[k]->n_cases, ++k) cases_end(g->meshes[k], o, c[k], pending[k], st + off);
+  HX_TRY(ctx, hipStreamSynchronize(ctx->stream), "update sync");
   return HX_OK;
 }
 
@@ -2724,36 +2743,26 @@ hx_status hx_compute_prolong_advection(hx_mesh* mesh, double advect_length)
   return hx_prolong_refined(mesh, &p, 0, 0);
 }
 
-hx_status hx_max_dt_advection(hx_mesh* mesh, const hx_kernel_options* o, double msc, double msd, int local_time,
+hx_status hx_max_dt_advection(hx_mesh* mesh, const hx_kernel_options*, double msc, double msd, int local_time,
                               double advect_length, double* dt_out)
 {
   if (!live(mesh) || !dt_out) return HX_ERR_INVALID;
   hx_pde p{};
   p.kind = HX_PDE_ADVECTION;
   p.advect_length = advect_length;
-  double a, b;
-  hx_status s;
-  const int uf = o ? o->use_filter : 0;
-  if ((s = hx_max_dt(mesh, HX_CARTESIAN, &p, local_time, uf, msc, msd, &a))) return s;
-  if ((s = hx_max_dt(mesh, HX_DEFORMED, &p, local_time, uf, msc, msd, &b))) return s;
-  *dt_out = std::min(a, b);
-  return HX_OK;
+  if (hx_status s = max_dt_classes(mesh, &p, local_time, msc, msd, dt_out)) return s;
+  return max_dt_wait(mesh);
 }
 
-hx_status hx_max_dt_smooth_av(hx_mesh* mesh, const hx_kernel_options* o, double msc, double msd, int local_time,
+hx_status hx_max_dt_smooth_av(hx_mesh* mesh, const hx_kernel_options*, double msc, double msd, int local_time,
                               double* dt_out)
 {
   if (!live(mesh) || !dt_out) return HX_ERR_INVALID;
   hx_pde p{};
   p.kind = HX_PDE_SMOOTH_AV;
   p.diff_time = p.cheby_step = 1.;  // Max_dt<Smooth_art_visc>(..., 1., 1.) (kernels_max_dt.cpp:15)
-  double a, b;
-  hx_status s;
-  const int uf = o ? o->use_filter : 0;
-  if ((s = hx_max_dt(mesh, HX_CARTESIAN, &p, local_time, uf, msc, msd, &a))) return s;
-  if ((s = hx_max_dt(mesh, HX_DEFORMED, &p, local_time, uf, msc, msd, &b))) return s;
-  *dt_out = std::min(a, b);
-  return HX_OK;
+  if (hx_status s = max_dt_classes(mesh, &p, local_time, msc, msd, dt_out)) return s;
+  return max_dt_wait(mesh);
 }
 
 // The fix's boundary faces: mode 1 ghost state = inside (Solver.cpp:1066-1071), mode 2 ghost LDG = -inside
@@ -3038,19 +3047,14 @@ hx_status hx_compute_fix_therm_admis(hx_mesh* mesh, const hx_kernel_options* o)
   return hx_prolong_refined(mesh, &p, 0, 0);
 }
 
-hx_status hx_max_dt_fix_therm_admis(hx_mesh* mesh, const hx_kernel_options* o, double msc, double msd, int local_time,
+hx_status hx_max_dt_fix_therm_admis(hx_mesh* mesh, const hx_kernel_options*, double msc, double msd, int local_time,
                                     double* dt_out)
 {
   if (!live(mesh) || !dt_out) return HX_ERR_INVALID;
   hx_pde p{};
   p.kind = HX_PDE_FIX_ADMIS;
-  double a, b;
-  hx_status s;
-  const int uf = o ? o->use_filter : 0;
-  if ((s = hx_max_dt(mesh, HX_CARTESIAN, &p, local_time, uf, msc, msd, &a))) return s;
-  if ((s = hx_max_dt(mesh, HX_DEFORMED, &p, local_time, uf, msc, msd, &b))) return s;
-  *dt_out = std::min(a, b);
-  return HX_OK;
+  if (hx_status s = max_dt_classes(mesh, &p, local_time, msc, msd, dt_out)) return s;
+  return max_dt_wait(mesh);
 }
 
 // Solver::is_admissible (Solver.cpp:921-959)
@@ -3109,7 +3113,9 @@ hx_status hx_fix_admissibility(hx_mesh* mesh, const hx_update_options* o, double
     HX_TRY(ctx, mesh->ks->fix_av(l, 0), "fix_av");
     hx_kernel_options ko{0., 0, 0, 0};
     double dummy;
-    if ((s = hx_max_dt_fix_therm_admis(mesh, &ko, stability_ratio, stability_ratio, 1, &dummy))) return s;
+    hx_pde fix{};
+    fix.kind = HX_PDE_FIX_ADMIS;
+    if ((s = max_dt_classes(mesh, &fix, 1, stability_ratio, stability_ratio, &dummy))) return s;
     // dt = 1: the two steps of a second-order stabilized update (Solver.cpp:1059-1064)
     const double linear = 1., quadratic = 1. / 8 / 0.9;
     double step[2];
@@ -3123,17 +3129,17 @@ hx_status hx_fix_admissibility(hx_mesh* mesh, const hx_update_options* o, double
     // the flow's Max_dt (Solver.cpp:1076-1079); only its time step scale remains
     auto cheby = [](double n, double i) { return 1 / (1 - std::cos((n - i - 0.5) * M_PI / n)); };
     const double max_cheby = cheby(o->n_cheby_flow, o->n_cheby_flow - 1);
-    ko.use_filter = o->use_filter;
-    s = o->use_ldg ? hx_max_dt_navier_stokes(mesh, &ko, o->max_safety / max_cheby, o->max_safety, o->local_time, o->visc,
-                                             o->cond, &dummy)
-                   : hx_max_dt_euler(mesh, &ko, o->max_safety / max_cheby, o->max_safety, o->local_time, &dummy);
-    if (s) return s;
+    hx_pde flow{};
+    flow.kind = o->use_ldg ? HX_PDE_NAVIER_STOKES : HX_PDE_EULER;
+    flow.visc = o->visc;
+    flow.cond = o->cond;
+    if ((s = max_dt_classes(mesh, &flow, o->local_time, o->max_safety / max_cheby, o->max_safety, &dummy))) return s;
     l = make_launch(mesh);
     HX_TRY(ctx, mesh->ks->fix_av(l, 1), "fix_av");
   }
   --iter;
   *n_iters_out = iter;
-  return HX_OK;
+  return iter ? max_dt_wait(mesh) : HX_OK;
 }
 
 // Solver::update_art_visc_smoothness (Solver.cpp:457-582) with diffuse_art_visc (Solver.cpp:428-455)
@@ -3169,7 +3175,10 @@ hx_status hx_update_art_visc_smoothness(hx_mesh* mesh, const hx_av_options* o, d
   }
   // enforce CFL condition
   if ((s = hx_compute_prolong(mesh, 0, 0))) return s;
-  if ((s = hx_max_dt_advection(mesh, &ko, o->advect_max_safety, 1., 1, L, &dummy))) return s;
+  hx_pde adv{};
+  adv.kind = HX_PDE_ADVECTION;
+  adv.advect_length = L;
+  if ((s = max_dt_classes(mesh, &adv, 1, o->advect_max_safety, 1., &dummy))) return s;
   for (int iter = 0; iter < o->advect_iters; ++iter) {
     if ((s = hx_compute_write_face_advection(mesh, L))) return s;
     if ((s = hx_compute_prolong_advection(mesh, L))) return s;
@@ -3187,7 +3196,10 @@ hx_status hx_update_art_visc_smoothness(hx_mesh* mesh, const hx_av_options* o, d
   // root-smear-square
   const double diff_time = o->diff_ratio * L * L / n_real;
   ko = hx_kernel_options{0., 0, 0, 0};
-  if ((s = hx_max_dt_smooth_av(mesh, &ko, 1., o->diff_max_safety, 1, &dummy))) return s;
+  hx_pde smooth{};
+  smooth.kind = HX_PDE_SMOOTH_AV;
+  smooth.diff_time = smooth.cheby_step = 1.;
+  if ((s = max_dt_classes(mesh, &smooth, 1, 1., o->diff_max_safety, &dummy))) return s;
   if ((s = hx_compute_write_face_smooth_av(mesh))) return s;
   if ((s = hx_compute_prolong(mesh, 0, 0))) return s;
   for (int iter = 0; iter < o->diff_iters; ++iter)

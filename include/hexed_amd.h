@@ -11,6 +11,12 @@
  * per-element layouts) and copied to device memory by `hx_mesh_create`; afterwards all kernels run on the
  * device copy, stream-ordered on the context's stream, and fields move with hx_mesh_upload/hx_mesh_download.
  *
+ * Return points. hx_max_dt*, hx_is_admissible, hx_fix_admissibility, hx_calc_jacobian, hx_stab_art_visc,
+ * hx_set_art_visc_admis, hx_update_cases and hx_group_update return after the device has finished what they enqueued.
+ * Every other call may return while the device still works on it, hx_update and hx_update_no_alloc with their stages under
+ * way (hx_update with fix_admis once the last stage's check is done): a caller that reads or writes a field through
+ * hx_mesh_device_ptr on another stream first waits for hx_ctx_stream, or calls hx_ctx_synchronize.
+ *
  * Errors. Every call returns an `hx_status`; on failure `hx_last_error` returns the message. Argument
  * errors that the reference raises as std::runtime_error (kernel_factory.hpp:114-116, HEXED_ASSERT in
  * Spatial.hpp:322-323,539-540) return HX_ERR_INVALID with the reference's message text.

@@ -2,11 +2,13 @@
 case alone: the same time step per case and bit-identical states, in both arithmetic forms, for Euler and
 Navier-Stokes (single cases are themselves compared with the oracle in test_gpu_parity.py); plus the errors of
 the registration."""
+import ctypes
+
 import numpy as np
 import pytest
 
 from hexed_amd import abi, configs, mesh
-from hexed_amd.device import Context, Device_mesh, HxError
+from hexed_amd.device import Context, Device_group, Device_mesh, HxError
 
 from helpers import init_faces, per_var_rel_l2, say
 
@@ -110,4 +112,59 @@ def test_batch_errors(ctx):
         dev.set_cases(2, [ids, None])
     with pytest.raises(HxError, match="out of range"):
         dev.set_cases(1, [ids, None])
+    dev.close()
+
+
+@pytest.fixture(scope="module")
+def stream_idle(ctx):
+    """Whether every kernel enqueued on the context's stream has finished (hipStreamQuery)."""
+    query = ctypes.CDLL("libamdhip64.so.7").hipStreamQuery
+    query.argtypes = [ctypes.c_void_p]
+    stream = ctypes.c_void_p(ctx.stream)
+
+    def idle():
+        rc = query(stream)
+        assert rc in (0, 600), rc  # 600: hipErrorNotReady
+        return rc == 0
+    return idle
+
+
+@pytest.mark.parametrize("group", [False, True], ids=["cases", "group"])
+def test_batch_updates_return_finished(ctx, stream_idle, group):
+    """Every batch and group update, not the first of a sequence alone, returns after its stages have finished, so that a
+    caller may read a device view of a field on any stream."""
+    say(f"[gpu] stream idle after a batch update, group {group}")
+    devs = []
+    for n, rs in ((20, 6), (2, 5), (2, 4)):
+        host = configs.euler_box(n, rs, mach=0.5, seed=3)
+        init_faces(host)
+        devs.append(Device_mesh(ctx, host))
+        devs[-1].set_cases(1, [np.zeros(host.n_elem[0], np.int32), None])
+    opts = abi.update_options(max_safety=0.5)
+    g = Device_group(ctx, devs)
+    for _ in range(4):
+        g.update(opts) if group else devs[0].update_cases(opts)
+        assert stream_idle()
+    g.close()
+    for d in devs:
+        d.close()
+
+
+@pytest.mark.parametrize("entry", ["class", "mesh", "aux"])
+def test_local_max_dt_returns_finished(ctx, stream_idle, entry):
+    """The Max_dt entry points return after the time step scale is written, with local time stepping too, whose result
+    needs no readback."""
+    say(f"[gpu] stream idle after a local Max_dt, entry {entry}")
+    host = configs.euler_box(48, 4, mach=0.5, seed=3)
+    init_faces(host)
+    dev = Device_mesh(ctx, host)
+    out, ko = ctypes.c_double(), abi.hx_kernel_options(0., 0, 0, 0)
+    for _ in range(3):
+        if entry == "class":
+            out.value = dev.max_dt(abi.HX_CARTESIAN, is_local=True)
+        elif entry == "mesh":
+            ctx.check(dev.lib.hx_max_dt_euler(dev.ptr, ctypes.byref(ko), 0.5, 0.5, 1, ctypes.byref(out)))
+        else:
+            out.value = dev.max_dt_fix_therm_admis(0.7, 0.6, True)
+        assert stream_idle() and out.value == 1.
     dev.close()
