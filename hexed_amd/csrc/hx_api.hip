@@ -2952,6 +2952,12 @@ hx_status hx_calc_jacobian(hx_mesh* mesh, const hx_vertex_data* v)
   const long long n_def = dm.n_elem[HX_DEFORMED];
   const size_t n_pos = size_t(n_def * nvert * nd), n_adj = size_t(n_def * 2 * nd * nfq);
   double* const vt = vc.vert;
+  // the uploads read the caller's arrays until the stream has passed them, so that an early return waits for it as well
+  struct Drain
+  {
+    hx_ctx* ctx;
+    ~Drain() { (void)hipStreamSynchronize(ctx->stream); }
+  } drain{ctx};
   HX_TRY(ctx, vc_buffer(&vc.pos, n_pos, false), "hipMalloc(vertex positions)");
   if (n_pos)
     HX_TRY(ctx, hipMemcpyAsync(vc.pos, v->position, n_pos * sizeof(double), hipMemcpyHostToDevice, ctx->stream),

@@ -77,3 +77,30 @@ assert minima(da) == (["minima (nil)"] * 2, True)
 b.close()
 assert minima(da) == (kept, True)
 """)
+
+
+def test_calc_jacobian_errors_wait_for_the_uploads(run):
+    """The uploads of hx_calc_jacobian read the caller's arrays: whichever later call fails, it returns only after the
+    stream has passed them."""
+    run("""
+m = mesh.box(3, 3, 2, deformed=True, jitter=0.1, seed=1, bc=(abi.HX_BC_COPY, [0.] * 5))
+m.node_adj = np.zeros((m.n_elem[1], 6, m.nfq))
+dev = Device_mesh(Context(0), m)
+vd = m.vertex_data()
+jacobian = lambda: dev.lib.hx_calc_jacobian(dev.ptr, ctypes.byref(vd))
+assert jacobian() == abi.HX_OK
+failed = 0
+for kind in (0, 1):
+    for after in range(100):
+        calls()
+        fake.fake_fail(kind, after)
+        status = jacobian()
+        fake.fake_fail(kind, -1)
+        log = calls()
+        copies = [k for k, x in enumerate(log) if x.startswith("copy")]
+        assert not copies or "wait" in log[copies[-1]:], (kind, after, log)
+        if status == abi.HX_OK:
+            break
+        failed += 1
+assert failed >= 8, failed
+""")
