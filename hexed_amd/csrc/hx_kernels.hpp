@@ -810,9 +810,11 @@ __device__ inline double max_dt_scale_u(const Dev_mesh& m, const Ops<RS>* __rest
 __device__ inline double step_coef(double coef, const double* dtp) { return dtp ? coef * *dtp : coef; }
 
 // ---- Local, Euler (Spatial.hpp:326-509 with Navier_stokes<false>) -----------------------------------------
+// (the FP32-MFMA form's deformed elements run the FP64 kernel (euler_form): there is no layout for its pressure rows here)
 template <int ND, int RS, bool DEF, class P>
 struct Euler_lds
 {
+  static_assert(!(P::mfma && DEF), "deformed elements take euler_form");
   using S = Shape<ND, RS, P::mfma>;
   // arrays of T (padded)
   static constexpr int F = 0;                               // [NV][NQP] flux along the current direction
@@ -820,9 +822,7 @@ struct Euler_lds
   static constexpr int PER_T = RT + S::NV * S::NQP;
   // arrays of double
   static constexpr int SB = 0;                              // [2ND][NV][NFQ] numerical face fluxes, the last face first
-  static constexpr int PD = SB + 2 * ND * S::NV * S::NFQ;   // [ND][NQP] FP32-MFMA, deformed: pressure part p n_iv
-  static constexpr int RP = PD + ND * S::NQP;               // [ND][NQP] FP32-MFMA, deformed: its derivative, summed
-  static constexpr int LOOP_D = PD + (P::mfma && DEF ? 2 * ND * S::NQP : 0);
+  static constexpr int SB_END = SB + 2 * ND * S::NV * S::NFQ;
   static constexpr int U = 0;                                // [NV][NQP] updated state, for Write_face (after the loop)
   // what the end of the tile reads of the element's tables: vertex time step scale [2^ND], face slots [2ND] (int), node
   // coordinates [RS] (element 0). Written during the last direction's row phase, when every other direction's fluxes
@@ -830,7 +830,8 @@ struct Euler_lds
   // points of U). It starts past U, which is written while slower waves still read it.
   static constexpr int TB = S::NV * S::NQP;
   static constexpr int TB_SLOT = TB + S::NVERT, TB_NODE = TB_SLOT + ND, TB_END = TB_NODE + RS;
-  static constexpr int PER_D = LOOP_D > TB_END ? LOOP_D : TB_END;
+  static_assert(TB >= SB + 2 * S::NV * S::NFQ, "the last direction's fluxes lie below the tables");
+  static constexpr int PER_D = SB_END > TB_END ? SB_END : TB_END;
   static constexpr __device__ int sb(int face) { return SB + (2 * ND - 1 - face) * S::NV * S::NFQ; }
 };
 
@@ -884,7 +885,6 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
   constexpr int NQ = S::NQ, NQP = S::NQP, NFQ = S::NFQ, NV = S::NV, EPB = S::EPB, NT = euler_block<ND, RS>();
   constexpr int NVERT = S::NVERT;
   constexpr int cls = DEF ? HX_DEFORMED : HX_CARTESIAN;
-  constexpr bool EARLY_RC = true;
   const int t = threadIdx.x;
   const bool pt = t < EPB * NQ;
   const int el = pt ? t / NQ : 0, q = pt ? t % NQ : 0, qp = S::pad(q);
@@ -940,7 +940,6 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
     if (f.own)
       for (int v = 0; v < NV; ++v) ld[el2 * L::PER_D + L::sb(face) + v * NFQ + p] = fl[v];
   }
-  const double p64 = P::mfma ? pressure_of<ND>(u) : 0.;
   const bool fused_dt = (fuse.block_min || fuse.elem_scale[cls]) && !compute_residual;
   // what the end of the tile reads from memory: the residual cache (stage 1), the nominal size, the time step scale, the
   // Jacobian determinant, and for the fused time step the viscosity coefficients; and the element's tables (L::TB),
@@ -949,27 +948,23 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
   // (bulk and lap start as some loaded value: with a constant, the compiler moves their first use up to the load)
   double tss_q = 0., nom = 1., det_q = 1., bulk = u[0], lap = u[0], vert = 0., node = 0.;
   int slot = 0;
-  const auto load_update_operands = [&] {
-    if (stage) {
-      const double* rc = m.rcache[cls] + size_t(ec) * S::NRC * NQ;
-      for (int v = 0; v < NV; ++v) rcv[v] = rc[v * NQ + q];
-    } else {
-      for (int v = 0; v < NV; ++v) rcv[v] = 0.;
-    }
-  };
   for (int i = 0; i < ND; ++i) {
     // volume flux along reference direction i (Spatial.hpp:404-419), in FP64
     if constexpr (!DEF)
       for (int j = 0; j < ND; ++j) nrm[j] = double(i == j);
     if (i || P::mfma) __syncthreads();
     if (pt)
-      conv_point<ND, DEF, P>(u, p64, nrm, myd + L::sb(2 * i) + Row<ND, RS>::fq(q, i), NFQ, my + L::F + qp, myd + L::PD + qp,
-                             NQP);
+      conv_point<ND, DEF, P>(u, 0., nrm, myd + L::sb(2 * i) + Row<ND, RS>::fq(q, i), NFQ, my + L::F + qp, nullptr, NQP);
     if constexpr (DEF)
       if (i + 1 < ND)
         for (int j = 0; j < ND; ++j) nrm[j] = mt[((i + 1) * ND + j) * NQ];
     if (i == ND - 1) {
-      if constexpr (EARLY_RC) load_update_operands();
+      if (stage) {
+        const double* rc = m.rcache[cls] + size_t(ec) * S::NRC * NQ;
+        for (int v = 0; v < NV; ++v) rcv[v] = rc[v * NQ + q];
+      } else {
+        for (int v = 0; v < NV; ++v) rcv[v] = 0.;
+      }
       tss_q = m.tss[cls][size_t(ec) * NQ + q];
       if constexpr (DEF) det_q = mt[ND * ND * NQ];
       nom = m.nom_size[cls][ec];
@@ -988,25 +983,17 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
       T* b = lt + el2 * L::PER_T;
       double* db = ld + el2 * L::PER_D;
       T y[RS];
-      conv_row<ND, RS, DEF, P>(con, [&]() -> const Eops<RS, double>& { return o; }, v, b + L::F + v * NQP + base, db + L::PD + (v % ND) * NQP + base, sd,
+      conv_row<ND, RS, DEF, P>(con, [&]() -> const Eops<RS, double>& { return o; }, v, b + L::F + v * NQP + base, nullptr, sd,
                                db[L::sb(2 * i) + v * NFQ + r], db[L::sb(2 * i + 1) + v * NFQ + r], y);
-      if (ok) {
-        sub_row(b + L::RT + v * NQP + base, sd, y, i == 0);
-        pressure_row<ND, RS, DEF, P>([&]() -> const Eops<RS, double>& { return o; }, i, v, db + L::PD + (v % ND) * NQP + base, db + L::RP + (v % ND) * NQP + base, sd);
-      }
+      if (ok) sub_row(b + L::RT + v * NQP + base, sd, y, i == 0);
     });
   }
   if (t < EPB * NVERT) ld[(t / NVERT) * L::PER_D + L::TB + t % NVERT] = vert;
   if (t < EPB * 2 * ND) reinterpret_cast<int*>(ld + (t / (2 * ND)) * L::PER_D + L::TB_SLOT)[t % (2 * ND)] = slot;
   if (t < RS) ld[L::TB_NODE + t] = node;
-  if (use_filter) {
-    filter_columns<ND, RS, NV, NT, S>(o, lt + L::RT, L::PER_T);
-    if constexpr (P::mfma && DEF) filter_columns<ND, RS, ND, NT, S>(o, ld + L::RP, L::PER_D);
-  } else {
-    __syncthreads();
-  }
+  if (use_filter) filter_columns<ND, RS, NV, NT, S>(o, lt + L::RT, L::PER_T);
+  else __syncthreads();
   // stage update (Spatial.hpp:483-503)
-  if constexpr (!EARLY_RC) load_update_operands();
   if (valid) {
     double mult = step_coef(coef, dtp) * tss_q / nom;
     if constexpr (DEF) mult /= det_q;
@@ -1014,7 +1001,6 @@ __device__ __forceinline__ void local_euler_tile(const Dev_mesh& m, int blk, typ
     double* sw = m.state[cls] + size_t(e) * NV * NQ;
     for (int v = 0; v < NV; ++v) {
       double r = double(my[L::RT + v * NQP + qp]);
-      if (has_pressure<ND, DEF>(v) && P::mfma) r -= myd[L::RP + v * NQP + qp];
       if (stage) r -= rcv[v];
       else rcw[v * NQ + q] = r;
       r *= mult;
