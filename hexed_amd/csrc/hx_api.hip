@@ -2477,8 +2477,7 @@ hx_status hx_group_create(hx_ctx* ctx, hx_mesh* const* meshes, int n_meshes, hx_
   for (hx_mesh* m : g->meshes) {
     g->n_cases += m->n_cases;
     g->with_def = g->with_def || m->dm.n_elem[HX_DEFORMED] > 0;
-    fusable = fusable && hx::fused_set_nd3()->supports(m->dm.rs) && !ensure_ops(ctx, m->dm.rs);
-    g->hops[m->dm.rs] = ctx->host_ops[m->dm.rs].data();
+    fusable = fusable && hx::fused_set_nd3()->supports(m->dm.rs);
   }
   auto bail = [&](hx_status s) {
     release_group(g);
@@ -2491,6 +2490,12 @@ hx_status hx_group_create(hx_ctx* ctx, hx_mesh* const* meshes, int n_meshes, hx_
   std::memset(g->dts, 0, (g->n_cases + 1) * sizeof(double));
   if (fusable) {
     g->fs = hx::fused_set_nd3();
+    // the fused Local takes the operators of every row size it is built for, also of those the group has none of
+    for (int rs = 2; rs <= HX_MAX_ROW_SIZE; ++rs)
+      if (g->fs->supports(rs)) {
+        if (hx_status s = ensure_ops(ctx, rs)) return bail(s);
+        g->hops[rs] = ctx->host_ops[rs].data();
+      }
     if (hipMalloc(reinterpret_cast<void**>(&g->mem), 2 * n_meshes * sizeof(hx::Fused_member)) != hipSuccess ||
         hipMalloc(reinterpret_cast<void**>(&g->plans), 3 * sizeof(hx::Fused_plan)) != hipSuccess)
       return bail(fail(ctx, HX_ERR_HIP, "hipMalloc(group tables)"));

@@ -104,3 +104,19 @@ for kind in (0, 1):
         failed += 1
 assert failed >= 8, failed
 """)
+
+
+@pytest.mark.parametrize("row_sizes", [[4], [5], [6], [4, 6]], ids=str)
+def test_group_of_some_row_sizes(run, row_sizes):
+    """A fused group that has no mesh of some of the row sizes its kernels are built for."""
+    run(f"""
+ctx, devs = Context(0), []
+for rs in {row_sizes}:
+    m = configs.euler_box(2, rs, seed=1)
+    devs.append(Device_mesh(ctx, m))
+    devs[-1].set_cases(1, [np.zeros(m.n_elem[0], np.int32), None])
+g = Device_group(ctx, devs)
+assert g.fused
+g.update(abi.update_options())
+assert sum("k_fused_local_euler" in x for x in calls()) == 2
+""")
