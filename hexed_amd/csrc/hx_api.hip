@@ -240,7 +240,8 @@ struct hx_group
   hx::Fused_plan* plans = nullptr;      // device [3]: state BCs, Neighbor, Local
   hx::Fused_plan hplan[3]{};
   std::vector<hx::Fused_member> hmem;   // host copy of `mem`
-  double* dts = nullptr;                // pinned host: every case's time step, then the sequence number
+  double* dts = nullptr;                // pinned host [cap_dts]: every case's time step, then the sequence number
+  int cap_dts = 0;
   int order = 2, per_cu = 0;            // launch shape of the fused Local (hx_group_set_shape)
   int n_cu = 0;
   const void* hops[HX_MAX_ROW_SIZE + 1] = {};  // the context's host Ops<rs> tables, by row size
@@ -2339,6 +2340,25 @@ hx_status hx_update_cases(hx_mesh* mesh, const hx_update_options* o, hx_update_s
 
 namespace {
 
+// the members' cases counted (hx_mesh_set_cases may have registered others since the last call), with room for their time
+// steps
+hx_status group_time_steps(hx_group* g)
+{
+  hx_ctx* ctx = g->ctx;
+  g->n_cases = 0;
+  for (hx_mesh* m : g->meshes) g->n_cases += m->n_cases;
+  if (g->n_cases < g->cap_dts) return HX_OK;
+  if (g->dts) (void)hipHostFree(g->dts);
+  g->dts = nullptr;
+  g->cap_dts = 0;
+  const size_t bytes = size_t(g->n_cases + 1) * sizeof(double);
+  HX_TRY(ctx, hipHostMalloc(reinterpret_cast<void**>(&g->dts), bytes, hipHostMallocMapped | hipHostMallocCoherent),
+         "hipHostMalloc(group time steps)");
+  std::memset(g->dts, 0, bytes);
+  g->cap_dts = g->n_cases + 1;
+  return HX_OK;
+}
+
 // the plan of one fused kernel: a segment per (mesh, class) with work, tiles from the fused set
 void build_plan(hx_group* g, int kind, hx::Fused_plan& p)
 {
@@ -2475,7 +2495,6 @@ hx_status hx_group_create(hx_ctx* ctx, hx_mesh* const* meshes, int n_meshes, hx_
   g->meshes.assign(meshes, meshes + n_meshes);
   bool fusable = meshes[0]->dm.nd == 3;
   for (hx_mesh* m : g->meshes) {
-    g->n_cases += m->n_cases;
     g->with_def = g->with_def || m->dm.n_elem[HX_DEFORMED] > 0;
     fusable = fusable && hx::fused_set_nd3()->supports(m->dm.rs);
   }
@@ -2484,10 +2503,7 @@ hx_status hx_group_create(hx_ctx* ctx, hx_mesh* const* meshes, int n_meshes, hx_
     delete g;
     return s;
   };
-  if (hipHostMalloc(reinterpret_cast<void**>(&g->dts), (g->n_cases + 1) * sizeof(double),
-                    hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
-    return bail(fail(ctx, HX_ERR_HIP, "hipHostMalloc(group time steps)"));
-  std::memset(g->dts, 0, (g->n_cases + 1) * sizeof(double));
+  if (hx_status s = group_time_steps(g)) return bail(s);
   if (fusable) {
     g->fs = hx::fused_set_nd3();
     // the fused Local takes the operators of every row size it is built for, also of those the group has none of
@@ -2563,6 +2579,7 @@ hx_status hx_group_update(hx_group* g, const hx_update_options* o, hx_update_sta
     pending[k] = c[k].pending;
   }
   if (hx_status s = upload_members(g, fuse)) return s;
+  if (hx_status s = group_time_steps(g)) return s;
   for (int i_flow = 0; i_flow < o->flow_iters; ++i_flow) {
     for (int i_cheby = 0; i_cheby < c[0].n_cheby; ++i_cheby) {
       bool fused = true;

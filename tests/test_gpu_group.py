@@ -7,7 +7,7 @@ Navier-Stokes; the lifetime and registration errors."""
 import numpy as np
 import pytest
 
-from hexed_amd import abi, configs
+from hexed_amd import abi, configs, mesh
 from hexed_amd.device import Context, Device_group, Device_mesh, HxError
 
 from helpers import init_faces, say
@@ -138,6 +138,29 @@ def test_group_navier_stokes_steps_meshes_alone(ctx):
             d.update_cases(opts, s)
         g.update(opts, st_g)
     compare("navier-stokes", hosts, singles, members)
+    g.close()
+    for d in singles + members:
+        d.close()
+
+
+def test_group_cases_registered_anew(ctx):
+    """Cases registered anew on a member of a live group, fewer than it was created with and more."""
+    say("[gpu] group, cases registered anew")
+    two = mesh.concat([configs.euler_box(2, 5, mach=0.4, seed=1), configs.euler_box(3, 5, mach=0.6, seed=2)])
+    hosts = [two, configs.euler_box(3, 4, mach=0.5, seed=3)]
+    singles, members = devices(ctx, hosts, abi.HX_FP64), devices(ctx, hosts, abi.HX_FP64)
+    g = Device_group(ctx, members)
+    opts = abi.update_options(max_safety=0.5)
+    for n in (2, 1, 2):
+        for d in (singles[0], members[0]):
+            d.set_cases(n, [(two.case_id[0] * (n - 1)).astype(np.int32), None])
+        st_s, st_g = [(abi.hx_update_status * n)(), (abi.hx_update_status * 1)()], (abi.hx_update_status * (n + 1))()
+        for step in range(STEPS):
+            for d, s in zip(singles, st_s):
+                d.update_cases(opts, s)
+            g.update(opts, st_g)
+            assert [s.time_step for s in st_g] == [x.time_step for s in st_s for x in s], (n, step)
+            compare(f"{n} cases, step {step}", hosts, singles, members)
     g.close()
     for d in singles + members:
         d.close()

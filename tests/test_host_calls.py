@@ -120,3 +120,20 @@ assert g.fused
 g.update(abi.update_options())
 assert sum("k_fused_local_euler" in x for x in calls()) == 2
 """)
+
+
+def test_group_cases_registered_anew(run):
+    """More cases on a member of a live group than the group was created with: their time steps have room."""
+    run("""
+ctx = Context(0)
+m = mesh.concat([configs.euler_box(1, 4, seed=k) for k in range(20)])
+dev = Device_mesh(ctx, m)
+dev.set_cases(1, [np.zeros(20, np.int32), None])
+g = Device_group(ctx, [dev])
+opts = abi.update_options()
+g.update(opts)
+for n in (20, 1, 10):
+    dev.set_cases(n, [(np.arange(20) * n // 20).astype(np.int32), None])
+    dev.lib.hx_mesh_mark_changed(dev.ptr)
+    g.update(opts, (abi.hx_update_status * n)())
+""")
