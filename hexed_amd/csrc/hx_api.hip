@@ -2498,6 +2498,7 @@ hx_status hx_group_create(hx_ctx* ctx, hx_mesh* const* meshes, int n_meshes, hx_
     g->with_def = g->with_def || m->dm.n_elem[HX_DEFORMED] > 0;
     fusable = fusable && hx::fused_set_nd3()->supports(m->dm.rs);
   }
+  for (hx_mesh* m : g->meshes) ++m->n_groups;
   auto bail = [&](hx_status s) {
     release_group(g);
     delete g;
@@ -2525,7 +2526,6 @@ hx_status hx_group_create(hx_ctx* ctx, hx_mesh* const* meshes, int n_meshes, hx_
       return bail(fail(ctx, HX_ERR_HIP, "hipGetDeviceProperties"));
     g->n_cu = prop.multiProcessorCount;
   }
-  for (hx_mesh* m : g->meshes) ++m->n_groups;
   ctx->groups.push_back(g);
   *out = g;
   return HX_OK;

@@ -137,3 +137,21 @@ for n in (20, 1, 10):
     dev.lib.hx_mesh_mark_changed(dev.ptr)
     g.update(opts, (abi.hx_update_status * n)())
 """)
+
+
+def test_failed_group_leaves_its_meshes_free(run):
+    """A group whose creation fails does not count among its meshes' groups."""
+    run("""
+ctx = Context(0)
+m = configs.euler_box(2, 4, seed=1)
+dev = Device_mesh(ctx, m)
+dev.set_cases(1, [np.zeros(m.n_elem[0], np.int32), None])
+fake.fake_fail(0, 0)  # the upload of the member tables
+try:
+    Device_group(ctx, [dev])
+    raise SystemExit("the group was created")
+except RuntimeError:
+    pass
+fake.fake_fail(0, -1)
+dev.close()
+""")
