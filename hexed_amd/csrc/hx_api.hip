@@ -1557,6 +1557,9 @@ hx_status hx_compute_restrict(hx_mesh* mesh, int scale, int offset) { return hx_
 
 }  // extern "C"
 
+static hx_status fix_admissibility(hx_mesh* mesh, const hx_update_options* o, double stability_ratio, bool failed,
+                                   int* n_iters_out);
+
 namespace {
 
 // member-wise equality (structure padding is not compared)
@@ -1845,7 +1848,7 @@ hx_status update_once(hx_mesh* mesh, const hx_update_options* o, const Update_se
               fold = fold && i;
               Stage_fold off(mesh, false, false, 0);
               int iters = 0;
-              if ((s = hx_fix_admissibility(mesh, o, o->fix_admis_max_safety, &iters))) return s;
+              if ((s = fix_admissibility(mesh, o, o->fix_admis_max_safety, true, &iters))) return s;
               st->fix_admis_iters += iters;
               fixed = iters || fixed;
             }
@@ -3104,9 +3107,10 @@ hx_status hx_is_admissible(hx_mesh* mesh, int* admissible)
 // admissible state (an inadmissible one restarts the count), so its coefficient is zero everywhere. Here every
 // iteration therefore swaps with a zero coefficient, which leaves the same state, time step scale and artificial
 // viscosity (Laplacian coefficient zero) as the reference.
-hx_status hx_fix_admissibility(hx_mesh* mesh, const hx_update_options* o, double stability_ratio, int* n_iters_out)
+// `failed`: the caller has just found the state inadmissible.
+static hx_status fix_admissibility(hx_mesh* mesh, const hx_update_options* o, double stability_ratio, bool failed,
+                                   int* n_iters_out)
 {
-  if (!live(mesh) || !o || !n_iters_out) return HX_ERR_INVALID;
   hx_ctx* ctx = mesh->ctx;
   Dev_mesh& dm = mesh->dm;
   hx_status s;
@@ -3116,8 +3120,8 @@ hx_status hx_fix_admissibility(hx_mesh* mesh, const hx_update_options* o, double
     if (iter >= 100000)
       return fail(ctx, HX_ERR_INVALID,
                   "failed to fix thermodynamic admissability in " + std::to_string(iter) + " iterations");
-    int admissible = 0;
-    if ((s = hx_is_admissible(mesh, &admissible))) return s;
+    bool admissible = false;
+    if ((iter || !failed) && (s = check_admissible(mesh, 0, &admissible))) return s;
     if (admissible) {
       if (iter) n_iters = std::min(n_iters, 2 * iter);
       else {
@@ -3168,6 +3172,12 @@ hx_status hx_fix_admissibility(hx_mesh* mesh, const hx_update_options* o, double
   --iter;
   *n_iters_out = iter;
   return iter ? max_dt_wait(mesh) : HX_OK;
+}
+
+hx_status hx_fix_admissibility(hx_mesh* mesh, const hx_update_options* o, double stability_ratio, int* n_iters_out)
+{
+  if (!live(mesh) || !o || !n_iters_out) return HX_ERR_INVALID;
+  return fix_admissibility(mesh, o, stability_ratio, false, n_iters_out);
 }
 
 // Solver::update_art_visc_smoothness (Solver.cpp:457-582) with diffuse_art_visc (Solver.cpp:428-455)

@@ -16,6 +16,7 @@ std::map<void*, std::pair<void*, size_t>> blocks;  // address handed out -> mapp
 std::map<const void*, void*> symbols;
 int fail_after[2] = {-1, -1};  // calls of each kind (0 copy, 1 launch) that still succeed; -1 all
 int busy = 0;                  // stream queries that still find work
+int verdict = -1, verdicts = 0;  // the next `verdicts` launches of k_admissible raise flag `verdict`
 int last_error = 0;
 
 void note(const std::string& s) { log_text += s + "\n"; }
@@ -65,6 +66,7 @@ const char* fake_log() { return log_text.c_str(); }
 void fake_clear() { log_text.clear(); }
 void fake_fail(int kind, int after) { fail_after[kind] = after; }
 void fake_busy(int queries) { busy = queries; }
+void fake_verdict(int flag, int launches) { verdict = flag, verdicts = launches; }
 
 void* __hipRegisterFatBinary(const void*)
 {
@@ -131,6 +133,11 @@ int hipLaunchKernel(const void* f, Dim, Dim, void** args, size_t, void*)
   if (kernels[f].find("k_local_euler") != std::string::npos) {
     note("time step " + hex(*static_cast<void**>(args[4])));
     note("minima " + hex(*static_cast<void**>(args[8])));
+  }
+  // k_admissible(mesh, class, flags)
+  if (kernels[f].find("k_admissibleI") != std::string::npos && verdicts > 0) {
+    (*static_cast<int**>(args[2]))[verdict] = 1;
+    --verdicts;
   }
   return 0;
 }

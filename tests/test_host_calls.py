@@ -155,3 +155,22 @@ except RuntimeError:
 fake.fake_fail(0, -1)
 dev.close()
 """)
+
+
+UPDATE_WITH_FIX = """
+m = configs.euler_box(2, 4, seed=1)
+dev = Device_mesh(Context(0), m)
+opts, st = abi.update_options(local_time=True, fix_admis=True), abi.hx_update_status()
+calls()
+"""
+
+
+def test_update_checks_admissibility_once_before_a_fix(run):
+    """The verdict that makes an update call the fix is the fix's first: one check per iteration and one per stage."""
+    run(UPDATE_WITH_FIX + """
+fake.fake_verdict(0, 1)
+dev.update(opts, st)
+assert st.fix_admis_iters == 1
+log = calls()
+assert sum("k_admissibleI" in x for x in log) == 3, log
+""")
