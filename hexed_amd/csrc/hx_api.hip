@@ -1833,18 +1833,21 @@ hx_status update_once(hx_mesh* mesh, const hx_update_options* o, const Update_se
           }
           if (s) return s;
           if (o->fix_admis) {
-            // the check reads the faces where the stage left them; a fix works on the primary buffer, so after a folded
-            // stage 0 that needs one the faces move there and stage 1 goes without folding
+            // the check reads the faces where the stage left them. A fix works on the primary buffer, so after a folded
+            // stage 0 that needs one the faces move there and stage 1 goes without folding; they move as well where the
+            // check ends the update with an error (a state that is not finite), for whoever looks at what it left
             bool admissible = false;
-            if ((s = check_admissible(mesh, mesh->alt_wr, &admissible))) return s;
+            s = check_admissible(mesh, mesh->alt_wr, &admissible);
+            if (mesh->alt_wr && (s || !admissible)) {
+              const long long n = (long long)mesh->dm.n_slot * mesh->dm.nv * mesh->dm.nfq;
+              if (n)
+                hipLaunchKernelGGL(k_faces_to_primary, dim3(unsigned((n + 255) / 256)), dim3(256), 0, ctx->stream,
+                                   mesh->dm, n);
+              const hipError_t e = hipGetLastError();
+              if (!s) HX_TRY(ctx, e, "faces to the primary buffer");
+            }
+            if (s) return s;
             if (!admissible) {
-              if (mesh->alt_wr) {
-                const long long n = (long long)mesh->dm.n_slot * mesh->dm.nv * mesh->dm.nfq;
-                if (n)
-                  hipLaunchKernelGGL(k_faces_to_primary, dim3(unsigned((n + 255) / 256)), dim3(256), 0, ctx->stream,
-                                     mesh->dm, n);
-                HX_TRY(ctx, hipGetLastError(), "faces to the primary buffer");
-              }
               fold = fold && i;
               Stage_fold off(mesh, false, false, 0);
               int iters = 0;

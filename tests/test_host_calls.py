@@ -174,3 +174,15 @@ assert st.fix_admis_iters == 1
 log = calls()
 assert sum("k_admissibleI" in x for x in log) == 3, log
 """)
+
+
+def test_update_that_ends_not_finite_leaves_its_faces(run):
+    """A folded stage 0 extrapolates into the second face buffer; an update that its check ends leaves the faces in the
+    first, where a download reads them."""
+    run(UPDATE_WITH_FIX + """
+fake.fake_verdict(1, 1)
+assert dev.lib.hx_update(dev.ptr, ctypes.byref(opts), ctypes.byref(st)) == abi.HX_ERR_NOT_FINITE
+log = calls()
+check = [k for k, x in enumerate(log) if "k_admissibleI" in x][-1]
+assert any("k_faces_to_primary" in x for x in log[check:]), log
+""")
