@@ -521,7 +521,8 @@ std::string validate(const hx_host_mesh* d, const Sizes& z)
 // The face-flux folding tables (Dev_mesh::partner, mortar_con) of a validated mesh. Every element face in a connection
 // that touches no hanging-face mortar gets its neighbour slot, the packed direction with its side, the connection class
 // and a boundary bit, and (deformed connections) the connection's normal slot; every other face (mortar neighbours,
-// coarse hanging faces) is marked precomputed. Every entry ends with the face's own slot. Connections touching a mortar are listed per class.
+// coarse hanging faces) is marked precomputed. Every entry ends with the face's own slot. Connections touching a mortar
+// are listed per class.
 // ref_con[4 * i + f]: the connection (class << 30 | index) of mortar f of refined face i, -1 where the face has none.
 // Returns whether the mortars of every refined face are exactly the fine faces its stretch leaves (Restrict_refined's)
 // and each is in a connection, which k_mortar_restrict requires.
@@ -1960,7 +1961,7 @@ hx_status hx_update_no_alloc(hx_mesh* mesh, const hx_update_options* o, hx_updat
   if (!ctx->scratch)
     return fail(ctx, HX_ERR_HIP, std::string("the scratch array has no device address: ") + hipGetErrorString(ctx->scratch_err));
   if (o->fix_admis)
-    return fail(ctx, HX_ERR_UNSUPPORTED, "the admissibility fix allocates its flags; use hx_update");
+    return fail(ctx, HX_ERR_UNSUPPORTED, "the admissibility fix allocates artificial viscosity where a mesh has none; use hx_update");
   Update_setup u;
   if (hx_status s = update_setup(mesh, o, &u, true)) return s;
   const Scratch_use use(ctx);
@@ -1986,7 +1987,7 @@ hx_status hx_update_status_sync(hx_mesh* mesh, hx_update_status* st)
   if (!live(mesh) || !st) return HX_ERR_INVALID;
   hx_ctx* ctx = mesh->ctx;
   if (!mesh->step) return fail(ctx, HX_ERR_INVALID, "no asynchronous update has run on this mesh");
-  static_assert(sizeof(Step_dev) <= 8 * sizeof(double), "the status fits the pinned readback buffer");
+  static_assert(sizeof(Step_dev) <= 4 * sizeof(double), "the status fits the words for readbacks");
   HX_TRY(ctx, hipMemcpyAsync(ctx->host_scalar, mesh->step, sizeof(Step_dev), hipMemcpyDeviceToHost, ctx->stream),
          "status readback");
   HX_TRY(ctx, hipStreamSynchronize(ctx->stream), "status sync");

@@ -25,13 +25,14 @@ struct Shape
   static constexpr int BLOCK = EPB * NQ;
   static constexpr int NFACE_DOF = 2 * ND * NV * NFQ;  // face values per element
   static constexpr int NRC = NV > RS ? NV : RS;         // residual-cache variables per point
-  // LDS copies of per-point arrays. Pairs of doubles are read and written 16 lanes at a time over 16 banks of 8 bytes,
-  // so rows (along the last dimension) of an even row size collide with each other and carry one pad slot; of an odd row
-  // size they spread over the banks as they are, and padding would put them an even pitch apart (whole Navier-Stokes
-  // steps, padded -> not: 3D row size 7 1124 -> 961 us, 5 515 -> 504, 3 716 -> 699; 2D row size 7 137 -> 119, 5 108 -> 105,
-  // 3 198 -> 186). Row size 2 goes without for the LDS it saves (two Navier-Stokes workgroups per compute unit, not one: 705 ->
-  // 559 us), as does 3D row size 6 where the rows are doubles (four workgroups with the in-place gradient; the pairs
-  // collide as often either way).
+  // LDS copies of per-point arrays. Along the last dimension the lanes of a row phase stand one row apart. Doubles are read
+  // 32 lanes at a time over 32 banks of 8 bytes and written 16 over 16 (floats 32 over 32 of 4 bytes): an even pitch puts
+  // such lanes on the same banks, so rows of an even row size carry one pad slot; an odd row size spreads as it is, and a
+  // pad would make its pitch even (whole Navier-Stokes steps, padded -> not: 3D row size 7 1124 -> 961 us, 5 515 -> 504,
+  // 3 716 -> 699; 2D row size 7 137 -> 119, 5 108 -> 105, 3 198 -> 186). Two even ones go without, for the LDS that the
+  // Navier-Stokes Local saves, by which the pitch of every kernel of the row size is chosen: row size 2 (two of its
+  // workgroups per compute unit, not one: 705 -> 559 us) and 3D row size 6 in doubles (four with the in-place gradient, not
+  // three; a pitch of 6 puts two of the 32 lanes on a bank).
   static constexpr int PITCH = RS % 2 || RS == 2 || (ND == 3 && RS == 6 && !F32) ? RS : RS + 1;
   static constexpr int NQP = NFQ * PITCH;
   static __device__ int pad(int q) { return PITCH == RS ? q : q + q / RS; }

@@ -405,7 +405,7 @@ hx_status hx_compute_residual(hx_mesh* mesh, const hx_update_options* opts);
  * (Spatial.hpp:293-510, 601-705) -- is launched once for all meshes, both element classes and every row size: a
  * workgroup runs one tile (one per-class workgroup's worth of work) of the (mesh, class) segment it falls in, with the
  * row size as a template argument, so results are bit-identical to stepping each mesh with hx_update_cases. Hanging
- * faces (Prolong/Restrict_refined) and the per-case time steps stay per mesh. Navier-Stokes options, local time stepping
+ * faces (Prolong/Restrict_refined) stay per mesh, as do the time steps of a sequence's first step. Navier-Stokes options, local time stepping
  * and fix_admis step the meshes one at a time. Meshes must outlive the group (hx_mesh_destroy refuses a mesh in a
  * group); hx_ctx_destroy detaches live groups. */
 typedef struct hx_group hx_group;
@@ -422,7 +422,8 @@ hx_status hx_group_destroy(hx_group* group);
 /* 1 when the group's Euler stages run as fused launches, 0 when its meshes step one at a time. */
 int hx_group_fused(const hx_group* group);
 hx_status hx_group_set_shape(hx_group* group, int order, int workgroups_per_cu);
-/* One Solver::update of every case of every mesh; `status` holds one entry per case, meshes in order. */
+/* One Solver::update of every case of every mesh; `status` holds one entry per case (as registered now), meshes in order.
+ * Returns when the stages have finished. */
 hx_status hx_group_update(hx_group* group, const hx_update_options* opts, hx_update_status* status);
 /* Times the fused Local under each candidate launch shape (one tile per workgroup; persistent grids of 2, 4, 8 and 16
  * workgroups per compute unit, strided and chunked), `reps` launches each after a warm-up, the best of them counted, and
@@ -474,7 +475,7 @@ hx_status hx_mesh_set_cases(hx_mesh* mesh, int n_cases, const int* case_cartesia
  * (its own Max_dt minimum, computed and applied on the device); status[n_cases] is advanced in place. Each case's
  * result equals hx_update on a mesh holding that case alone. Afterwards the time step scale field holds each case's
  * last time step (hx_update leaves 1 there). With local time stepping every case takes the same step, as in
- * hx_update. */
+ * hx_update. Returns when the stages have finished. */
 hx_status hx_update_cases(hx_mesh* mesh, const hx_update_options* opts, hx_update_status* status);
 
 /* ---- artificial-viscosity generator (the per-kernel entry points above also take HX_PDE_ADVECTION and
