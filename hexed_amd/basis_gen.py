@@ -144,43 +144,41 @@ def _round_tree(t):
     return _to_double(t)
 
 
-def stability_operators(rs, n_elem=N_ELEM_STABILITY):
-    """Discrete -d/dx and d^2/dx^2 on a periodic 1D mesh of `n_elem` unit elements (Basis.py:158-196).
+def stability_blocks(rs):
+    """The discrete -d/dx of advection and d/dx of diffusion on a periodic 1D mesh of unit elements (Basis.py:158-196), as
+    their blocks {-1, 0, 1: matrix} from an element's left neighbour, itself and its right neighbour."""
+    nodes, weights = gauss_legendre_nodes(rs)
+    bound = [[_lagrange(nodes, j, mpmath.mpf(s)) for j in range(rs)] for s in (0, 1)]
+    advection, gradient = ({d: mpmath.matrix(rs, rs) for d in (-1, 0, 1)} for _ in range(2))
+    for i in range(rs):
+        for j in range(rs):
+            deriv = _lagrange_deriv(nodes, i, j)
+            advection[0][i, j] -= deriv
+            gradient[0][i, j] += deriv
+            # both sides of a face: side si's equation takes half the sum (gradient) or difference (upwinding) of the
+            # values extrapolated from side sj
+            for si in (0, 1):
+                for sj in (0, 1):
+                    lift = bound[1 - sj][j] * bound[1 - si][i] / weights[i] / 2
+                    average = (2 * sj - 1) * lift
+                    gradient[sj - si][i, j] += average
+                    advection[sj - si][i, j] += (lift if si != sj else -lift) - average
+    return advection, gradient
 
-    Entries are formed the way the reference forms them: the 20-digit table values (derivative,
-    boundary interpolant) combined with full-precision weights, accumulated in float64.
-    """
+
+def eigenvals(rs, n_elem=N_ELEM_STABILITY):
+    """The smallest real parts over the eigenvalues of advection and of diffusion, the gradient applied twice. The operators
+    are block-circulant, so their eigenvalues are those of n_elem matrices of one element, one per wave number, which
+    mpmath finds to the last bit of a double on every machine (a float64 solver of the full operator leaves a few)."""
     with mpmath.workdps(CALC_DPS):
-        nodes, weights = gauss_legendre_nodes(rs)
-        nodes = [+x for x in nodes]
-        weights = [+w for w in weights]
-        d20 = [[_to_double(_lagrange_deriv(nodes, i, j)) for j in range(rs)] for i in range(rs)]
-        # interpolate() returns 20-digit values; dividing by the 50-digit weight happens at high precision
-        b20 = [[mpmath.mpf(str(sympy.Float(mpmath.nstr(_lagrange(nodes, j, mpmath.mpf(s)), CALC_DPS + 5), REPR_DIGITS)))
-                for j in range(rs)] for s in (0, 1)]
-        n = n_elem * rs
-        local_grad = np.zeros((n, n))
-        avrg = np.zeros((n, n))
-        jump = np.zeros((n, n))
-        for e in range(n_elem):
-            for i in range(rs):
-                for j in range(rs):
-                    local_grad[e * rs + i, e * rs + j] = d20[i][j]
-                    for si in (0, 1):
-                        for sj in (0, 1):
-                            row = ((e + si) % n_elem) * rs + i
-                            col = ((e + sj) % n_elem) * rs + j
-                            # the reference adds a high-precision term to a float64 entry and rounds the sum once
-                            bnd = b20[1 - sj][j] * b20[1 - si][i] / weights[i]
-                            avrg[row, col] = float(mpmath.mpf(avrg[row, col]) + mpmath.mpf(0.5 * (2 * sj - 1)) * bnd)
-                            jump[row, col] = float(mpmath.mpf(jump[row, col]) + mpmath.mpf(0.5 * (1 - 2 * (sj == si))) * bnd)
-    advection = -local_grad + -avrg + jump
-    diffusion = (local_grad + avrg) @ (local_grad + avrg)
-    return advection, diffusion
-
-
-def eigenvals(rs):
-    return [float(np.linalg.eigvals(m).real.min()) for m in stability_operators(rs)]
+        advection, gradient = stability_blocks(rs)
+        smallest = [mpmath.inf, mpmath.inf]
+        for k in range(n_elem):
+            z = mpmath.expjpi(mpmath.mpf(2 * k) / n_elem)
+            for which, (m, power) in enumerate(((advection, 1), (gradient, 2))):
+                values = mpmath.eig(m[0] + m[1] * z + m[-1] / z, left=False, right=False)
+                smallest[which] = min(smallest[which], *(mpmath.re(x ** power) for x in values))
+        return [_to_double(x) for x in smallest]
 
 
 def generate():
