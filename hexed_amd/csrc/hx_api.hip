@@ -2059,6 +2059,8 @@ hx_status hx_mesh_set_cases(hx_mesh* mesh, int n_cases, const int* case_cartesia
     mesh->allocs.push_back(*p);
     return true;
   };
+  // from here on the mesh holds no cases until all of their tables are there
+  mesh->n_cases = 0;
   int* dev_ids[2] = {};
   void *cmin = nullptr, *cdt = nullptr;
   for (int c = 0; c < 2; ++c) {
@@ -2568,6 +2570,8 @@ hx_status hx_group_update(hx_group* g, const hx_update_options* o, hx_update_sta
   if (!g || !g->ctx || !o || !st) return HX_ERR_INVALID;
   hx_ctx* ctx = g->ctx;
   const int n = int(g->meshes.size());
+  for (hx_mesh* m : g->meshes)
+    if (m->n_cases < 1) return fail(ctx, HX_ERR_INVALID, "no cases registered (hx_mesh_set_cases)");
   for (hx_mesh* m : g->meshes)
     if (m->precision != g->meshes[0]->precision)
       return fail(ctx, HX_ERR_INVALID, "group meshes must share the arithmetic form");

@@ -1,6 +1,6 @@
 // A HIP runtime without a device, for tests of the host code around the kernels: memory is host memory (each allocation
 // ends at an inaccessible page, so that an overrun faults), copies happen at once, kernels do not run, and every call is
-// appended to a log. hipMemcpyAsync and launches can be made to fail.
+// appended to a log. Asynchronous copies, launches and allocations can be made to fail.
 #include <sys/mman.h>
 
 #include <cstdio>
@@ -14,7 +14,7 @@ std::string log_text;
 std::map<const void*, std::string> kernels;
 std::map<void*, std::pair<void*, size_t>> blocks;  // address handed out -> mapping
 std::map<const void*, void*> symbols;
-int fail_after[2] = {-1, -1};  // calls of each kind (0 copy, 1 launch) that still succeed; -1 all
+int fail_after[3] = {-1, -1, -1};  // calls of each kind (0 copy, 1 launch, 2 allocation) that still succeed; -1 all
 int busy = 0;                  // stream queries that still find work
 int verdict = -1, verdicts = 0;  // the next `verdicts` launches of k_admissible raise flag `verdict`
 int last_error = 0;
@@ -110,9 +110,9 @@ int hipGetLastError()
   return e;
 }
 int hipGetSymbolAddress(void** p, const void* var) { return *p = symbols[var], 0; }
-int hipMalloc(void** p, size_t n) { return take(p, n); }
+int hipMalloc(void** p, size_t n) { return fails(2) ? 2 : take(p, n); }
 int hipFree(void* p) { return give(p); }
-int hipHostMalloc(void** p, size_t n, unsigned) { return take(p, n); }
+int hipHostMalloc(void** p, size_t n, unsigned) { return fails(2) ? 2 : take(p, n); }
 int hipHostFree(void* p) { return give(p); }
 int hipMemcpy(void* d, const void* s, size_t n, int) { return std::memcpy(d, s, n), 0; }
 int hipMemcpyAsync(void* d, const void* s, size_t n, int, void*)

@@ -186,3 +186,34 @@ log = calls()
 check = [k for k, x in enumerate(log) if "k_admissibleI" in x][-1]
 assert any("k_faces_to_primary" in x for x in log[check:]), log
 """)
+
+
+def test_cases_that_could_not_be_registered_are_refused(run):
+    """A registration that runs out of memory leaves no cases: neither the old ones, some of whose tables are gone, nor a part
+    of the new ones."""
+    run("""
+ctx = Context(0)
+m = mesh.concat([configs.euler_box(1, 4, seed=k) for k in range(8)])
+dev = Device_mesh(ctx, m)
+one, eight = np.zeros(8, np.int32), np.arange(8, dtype=np.int32)
+dev.set_cases(1, [one, None])
+g = Device_group(ctx, [dev])
+opts, st = abi.update_options(), (abi.hx_update_status * 8)()
+failed = 0
+for after in range(100):
+    dev.set_cases(1, [one, None])
+    dev.lib.hx_mesh_mark_changed(dev.ptr)
+    fake.fake_fail(2, after)
+    status = dev.lib.hx_mesh_set_cases(dev.ptr, 8, abi.iptr(eight), None)
+    fake.fake_fail(2, -1)
+    if status == abi.HX_OK:
+        break
+    calls()
+    assert dev.lib.hx_update_cases(dev.ptr, ctypes.byref(opts), st) == abi.HX_ERR_INVALID, after
+    assert dev.lib.hx_group_update(g.ptr, ctypes.byref(opts), st) == abi.HX_ERR_INVALID, after
+    assert not any(x.startswith("launch") for x in calls())
+    failed += 1
+assert failed >= 4, failed
+dev.set_cases(8, [eight, None])
+g.update(opts, st)
+""")
