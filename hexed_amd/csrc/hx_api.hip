@@ -137,6 +137,7 @@ struct Scratch_use
   Scratch_use& operator=(const Scratch_use&) = delete;
   static void release(const hx_ctx* ctx)  // the context's stream is about to go
   {
+    if (!ctx->scratch) return;
     std::lock_guard<std::mutex> lock(scratch_mutex);
     if (scratch_user[ctx->device].owner == ctx) scratch_user[ctx->device] = {};
   }
